@@ -7,27 +7,733 @@
 // faces with a 6x signed volume above 1e-7 (FP32) visible, visible faces
 // removed in place, one new face per horizon edge appended in the order the
 // visible faces and their edges are listed.  The reference runs that loop on
-// one CPU thread per cloud; here one wave owns a cloud and each step is
-// data-parallel over the wave: visibility over faces, the horizon test over
-// the visible faces' edges, the order-preserving compaction by ballots and
-// prefix counts.  Moments are summed in face order by one lane, as the
-// reference sums them (:433-481), so they are bit-identical too.
+// one CPU thread per cloud; here half a wave, a wave or a block owns a cloud
+// (by its size) and each step is data-parallel over it: visibility over faces,
+// the horizon test over the visible faces' edges, order-preserving
+// compaction and appends by ballots and prefix counts.  Moments are summed in
+// face order, as the reference sums them (:433-481), so they are
+// bit-identical too.
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "ogjk_internal.hpp"
+#include "ogjk_math.hpp"
 #include "opengjk/ogjk.h"
 
 ogjk_status ogjk_fail(ogjk_status code, const char* fmt, ...);
 
 namespace {
 
+using ogjk::xpair;
+
 constexpr int kWave = 64;
-// A cloud whose face capacity is at most this works in LDS (faces, visible
-// list and horizon: 24 B per face, 6 KiB per wave) and copies its faces out
-// once; larger clouds work in the output buffer and the workspace.
-constexpr int kLdsFaces = 256;
+
+// Results of d_nfaces that pass a cloud on to the next kernel of the call
+// (no result that a caller sees: the last kernel leaves none of them).
+constexpr int kToBlock = -100, kToBig = -101, kToGeneral = -102, kNowhere = -103;
+
+// A point of the working set and a face with its plane: the normal of
+// (v0, v1, v2) as vol6 forms it, and the packed vertex ids.
+struct Tri {
+  float nx, ny, nz;
+  uint32_t ids;
+};
+
+__device__ __forceinline__ Tri make_tri(float4 a, float4 b, float4 c, uint32_t ids) {
+  const float bx = b.x - a.x, by = b.y - a.y, bz = b.z - a.z;
+  const float cx = c.x - a.x, cy = c.y - a.y, cz = c.z - a.z;
+  return Tri{by * cz - bz * cy, bz * cx - bx * cz, bx * cy - by * cx, ids};
+}
+
+// 6x signed volume of the face and q: the operations of the reference's
+// signed volume in its order, with the face's normal kept from its creation
+// (same operands, so the same bits).
+__device__ __forceinline__ float vol6(const Tri& f, float4 a, float4 q) {
+  const float dx = q.x - a.x, dy = q.y - a.y, dz = q.z - a.z;
+  return f.nx * dx + f.ny * dy + f.nz * dz;
+}
+
+__device__ __forceinline__ float vol6(float4 a, float4 b, float4 c, float4 q) {
+  return vol6(make_tri(a, b, c, 0u), a, q);
+}
+
+__device__ __forceinline__ uint64_t ballot(bool v) { return __ballot(v); }
+
+__device__ __forceinline__ int rank_below(uint64_t mask, int lane) {
+  return ogjk::lanes_below<kWave>(mask, lane);
+}
+
+// Orders the LDS accesses of the lanes of one wave.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <int L, int M = 1>
+__device__ __forceinline__ int group_min_i(int v) {
+  if constexpr (M < L) {
+    int a, b;
+    xpair<M>(v, a, b);
+    return group_min_i<L, 2 * M>(a < b ? a : b);
+  } else {
+    return v;
+  }
+}
+
+// Of the lanes' (value, index) candidates (index < 0: none), the largest
+// value's lowest index, or -1.  No value is NaN or -inf.
+template <int L>
+__device__ __forceinline__ int group_argmax(float v, int i) {
+  const float m = ogjk::group_max_f<L>(i >= 0 ? v : -INFINITY);
+  const int r = group_min_i<L>(i >= 0 && v == m ? i : 0x7fffffff);
+  return r == 0x7fffffff ? -1 : r;
+}
+
+// The first four points of the hull of pt[0..n) (lane: of a group of L), in
+// the reference's choice and orientation.  Returns false when there is no
+// tetrahedron.  lo, hi, lo_i, hi_i: this lane's axis extremes over its points
+// i = lane, lane + L, ... (first index on ties, -1 without a point).
+template <int L, class Pts>
+__device__ __forceinline__ bool first_tetrahedron(const Pts& pt, int n, int lane,
+                                                  const float (&lo)[3], const int (&lo_i)[3],
+                                                  const float (&hi)[3], const int (&hi_i)[3],
+                                                  int (&id)[4]) {
+  int c[6];
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    c[2 * k] = group_argmax<L>(-lo[k], lo_i[k]);
+    c[2 * k + 1] = group_argmax<L>(hi[k], hi_i[k]);
+  }
+  // most separated pair among the six, the first in (a, b) order on ties:
+  // pair p = lane of 15, in chunks where the group is narrower
+  int i0 = 0, i1 = 1;
+  {
+    float bv = 0.0f;
+    int bp = -1;
+    for (int p = lane; p < 15; p += L) {
+      const int a = p < 5 ? 0 : p < 9 ? 1 : p < 12 ? 2 : p < 14 ? 3 : 4;
+      const int b = p < 5 ? p + 1 : p < 9 ? p - 3 : p < 12 ? p - 6 : p < 14 ? p - 8 : 5;
+      int ca = c[0], cb = c[1];
+#pragma unroll
+      for (int k = 1; k < 6; k++) {
+        ca = a == k ? c[k] : ca;
+        cb = b == k ? c[k] : cb;
+      }
+      const float4 A = pt(ca), B = pt(cb);
+      const float dx = B.x - A.x, dy = B.y - A.y, dz = B.z - A.z;
+      const float d = dx * dx + dy * dy + dz * dz;
+      if (d > bv) {
+        bv = d;
+        bp = p;
+      }
+    }
+    const int p = group_argmax<L>(bv, bp);
+    if (p >= 0) {
+      const int a = p < 5 ? 0 : p < 9 ? 1 : p < 12 ? 2 : p < 14 ? 3 : 4;
+      const int b = p < 5 ? p + 1 : p < 9 ? p - 3 : p < 12 ? p - 6 : p < 14 ? p - 8 : 5;
+      i0 = c[0];
+      i1 = c[1];
+#pragma unroll
+      for (int k = 1; k < 6; k++) {
+        i0 = a == k ? c[k] : i0;
+        i1 = b == k ? c[k] : i1;
+      }
+    }
+  }
+  const float4 p0 = pt(i0), p1 = pt(i1);
+  // farthest from the line i0-i1
+  int i2;
+  {
+    const float e0 = p1.x - p0.x, e1 = p1.y - p0.y, e2 = p1.z - p0.z;
+    float bv = 0.0f;
+    int bi = -1;
+    for (int i = lane; i < n; i += L) {
+      if (i == i0 || i == i1) continue;
+      const float4 p = pt(i);
+      const float vx = p.x - p0.x, vy = p.y - p0.y, vz = p.z - p0.z;
+      const float cx = vy * e2 - vz * e1, cy = vz * e0 - vx * e2, cz = vx * e1 - vy * e0;
+      const float d = cx * cx + cy * cy + cz * cz;
+      if (d > bv) {
+        bv = d;
+        bi = i;
+      }
+    }
+    i2 = group_argmax<L>(bv, bi);
+  }
+  if (i2 < 0) return false;
+  const float4 p2 = pt(i2);
+  // farthest from the plane i0-i1-i2
+  int i3;
+  {
+    const Tri t = make_tri(p0, p1, p2, 0u);
+    float bv = 0.0f;
+    int bi = -1;
+    for (int i = lane; i < n; i += L) {
+      if (i == i0 || i == i1 || i == i2) continue;
+      float d = vol6(t, p0, pt(i));
+      if (d < 0) d = -d;
+      if (d > bv) {
+        bv = d;
+        bi = i;
+      }
+    }
+    i3 = group_argmax<L>(bv, bi);
+  }
+  if (i3 < 0) return false;
+  const bool swap = vol6(p0, p1, p2, pt(i3)) > 0;
+  id[0] = i0;
+  id[1] = swap ? i2 : i1;
+  id[2] = swap ? i1 : i2;
+  id[3] = i3;
+  return true;
+}
+
+// Corner j of initial face f: (0,1,2) (0,2,3) (0,3,1) (1,3,2).
+__device__ __forceinline__ int init_corner(const int (&id)[4], int f, int j) {
+  const uint32_t map[4] = {0x210u, 0x320u, 0x130u, 0x231u};
+  const uint32_t m = f == 0 ? map[0] : f == 1 ? map[1] : f == 2 ? map[2] : map[3];
+  const int k = (m >> (4 * j)) & 3;
+  return k == 0 ? id[0] : k == 1 ? id[1] : k == 2 ? id[2] : id[3];
+}
+
+// ------------------------------------------------- clouds of few points
+//
+// Clouds of NMIN..NMAX points, L lanes each, the whole working set in LDS.
+// Bound by vector instructions (a step has ~20 faces and ~12 edges to look
+// at), hence: as many lanes as a small hull fills (16 for up to 32 points:
+// four clouds share a wave's instructions), the plane of each face kept from
+// its creation (an insertion reads it and one corner instead of three
+// gathered corners and a cross product), and the horizon test by one bit per
+// directed edge of the visible faces (row = start, bit = end) instead of a
+// search of their list.  100,000 clouds of 8-32 points: 0.29 ms at 16 lanes,
+// 0.33 at 32, 0.90 with one wave per cloud and no kept planes.
+template <int NMAX, int FMAX>
+struct GroupHull {
+  static constexpr int W = (NMAX + 31) / 32;  // words of a row of edge bits
+  float4 pt[NMAX];
+  Tri face[FMAX];
+  uint32_t vis[FMAX];
+  uint32_t adj[NMAX * W];
+};
+
+template <int L, int NMAX, int FMAX>
+__device__ __forceinline__ int hull_group(const float* __restrict__ P, int n, int cap,
+                                          GroupHull<NMAX, FMAX>& s, int lane) {
+  constexpr int W = GroupHull<NMAX, FMAX>::W;
+  static_assert(NMAX <= 256, "vertex ids are packed in 8 bits");
+  const auto pt = [&](int i) { return s.pt[i]; };
+  float lo[3], hi[3];
+  int lo_i[3], hi_i[3];
+  bool bad = false;
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    lo[k] = INFINITY;
+    hi[k] = -INFINITY;
+    lo_i[k] = hi_i[k] = -1;
+  }
+  wave_sync();
+  for (int i = lane; i < n; i += L) {
+    const float p[3] = {P[3 * i], P[3 * i + 1], P[3 * i + 2]};
+    s.pt[i] = make_float4(p[0], p[1], p[2], 0.0f);
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      bad |= !isfinite(p[k]);
+      if (lo_i[k] < 0 || p[k] < lo[k]) { lo[k] = p[k]; lo_i[k] = i; }
+      if (hi_i[k] < 0 || p[k] > hi[k]) { hi[k] = p[k]; hi_i[k] = i; }
+    }
+  }
+  for (int i = lane; i < NMAX * W; i += L) s.adj[i] = 0u;
+  if (ogjk::group_any<L>(bad)) return -2;
+  wave_sync();
+  int id[4];
+  if (!first_tetrahedron<L>(pt, n, lane, lo, lo_i, hi, hi_i, id)) return 0;
+  if (cap < 4) return -1;
+  if (lane < 4) {
+    const int a = init_corner(id, lane, 0), b = init_corner(id, lane, 1),
+              c = init_corner(id, lane, 2);
+    s.face[lane] = make_tri(s.pt[a], s.pt[b], s.pt[c], (uint32_t)(a | b << 8 | c << 16));
+  }
+  wave_sync();
+  int nf = 4;
+  const int k0 = lane / 3, e0 = lane - 3 * k0;  // the edge of this lane's first horizon test
+  for (int q = 0; q < n; q++) {
+    if (q == id[0] || q == id[1] || q == id[2] || q == id[3]) continue;
+    const float4 Q = s.pt[q];
+    // Visible faces leave the list (in place: a chunk is read before it is
+    // written, and only to lower positions) and mark their edges.
+    int nv = 0, w = 0;
+    for (int base = 0; base < nf; base += L) {
+      const int f = base + lane;
+      const bool in = f < nf;
+      const Tri F = s.face[in ? f : 0];
+      const bool v = in && vol6(F, s.pt[F.ids & 255u], Q) > 1e-7f;
+      const auto bv = ogjk::lanes_where<L>(v);
+      const int left = nf - base < L ? nf - base : L;
+      if (bv == 0 && nv == 0) {
+        w += left;
+        continue;
+      }
+      const int r = ogjk::lanes_below<L>(bv, lane);
+      if (v) {
+        s.vis[nv + r] = F.ids;
+        const uint32_t a = F.ids & 255u, b = (F.ids >> 8) & 255u, c = F.ids >> 16;
+        atomicOr(&s.adj[a * W + (b >> 5)], 1u << (b & 31u));
+        atomicOr(&s.adj[b * W + (c >> 5)], 1u << (c & 31u));
+        atomicOr(&s.adj[c * W + (a >> 5)], 1u << (a & 31u));
+      } else if (in) {
+        s.face[w + lane - r] = F;  // lanes below that are not visible
+      }
+      const int c = ogjk::count_lanes<L>(bv);
+      nv += c;
+      w += left - c;
+    }
+    if (nv == 0) continue;
+    wave_sync();
+    // horizon: directed edges of visible faces whose reverse no visible face
+    // has, in (visible face, edge) order; each is the base of a new face
+    int nh = 0;
+    const int ne = 3 * nv;
+    for (int base = 0; base < ne; base += L) {
+      const int h = base + lane;
+      uint32_t a = 0u, b = 0u;
+      bool hz = false;
+      if (h < ne) {
+        const int k = base == 0 ? k0 : h / 3, e = base == 0 ? e0 : h - 3 * k;
+        const uint32_t ids = s.vis[k];
+        a = (ids >> (8 * e)) & 255u;
+        b = (e == 2 ? ids : ids >> (8 * e + 8)) & 255u;
+        hz = !((s.adj[b * W + (a >> 5)] >> (a & 31u)) & 1u);
+      }
+      const auto bl = ogjk::lanes_where<L>(hz);
+      const int r = w + nh + ogjk::lanes_below<L>(bl, lane);
+      if (hz && r < FMAX) s.face[r] = make_tri(s.pt[a], s.pt[b], Q, a | b << 8 | (uint32_t)q << 16);
+      nh += ogjk::count_lanes<L>(bl);
+    }
+    wave_sync();
+    if constexpr (NMAX * W <= 2 * L) {
+      for (int i = lane; i < NMAX * W; i += L) s.adj[i] = 0u;
+    } else {
+      for (int h = lane; h < ne; h += L) {
+        const int k = h / 3, e = h - 3 * k;
+        const uint32_t ids = s.vis[k];
+        const uint32_t a = (ids >> (8 * e)) & 255u;
+        const uint32_t b = (e == 2 ? ids : ids >> (8 * e + 8)) & 255u;
+        s.adj[a * W + (b >> 5)] = 0u;
+      }
+    }
+    nf = w + nh;
+    if (nf > cap) return -1;
+    if (nf > FMAX) return kToBlock;
+    wave_sync();
+  }
+  return nf;
+}
+
+// Clouds of NMIN..NMAX points, kWave / L to a one-wave block; gridDim.x *
+// kWave / L groups take the clouds in turn.
+template <int L, int NMIN, int NMAX, int FMAX>
+__global__ __launch_bounds__(kWave) void k_hull_group(const float* __restrict__ pts,
+                                                      const int64_t* __restrict__ off,
+                                                      const int32_t* __restrict__ cnt, int nm,
+                                                      const int64_t* __restrict__ face_off,
+                                                      int64_t total_faces,
+                                                      int32_t* __restrict__ faces,
+                                                      int32_t* __restrict__ nfaces) {
+  constexpr int G = kWave / L;
+  __shared__ GroupHull<NMAX, FMAX> lds[G];
+  GroupHull<NMAX, FMAX>& s = lds[threadIdx.x / L];
+  const int lane = threadIdx.x & (L - 1);
+  const int groups = gridDim.x * G;
+  const int g = blockIdx.x * G + threadIdx.x / L;
+  // L clouds of this group at a time, the ones of its class by ballot
+  for (int64_t first = g; first < nm; first += (int64_t)groups * L) {
+    const int64_t mine = first + (int64_t)groups * lane;
+    int n_mine = -1;
+    if (mine < nm) n_mine = cnt[mine] < 0 ? 0 : cnt[mine];
+    uint64_t todo = ogjk::group_ballot<L>(n_mine >= NMIN && n_mine <= NMAX);
+    while (todo != 0) {
+      const int src = (int)__builtin_ctzll(todo);
+      todo &= todo - 1;
+      const int64_t m = first + (int64_t)groups * src;
+      const int n = __shfl(n_mine, src, L);
+      const int64_t f0 = face_off[m], cap64 = face_off[m + 1] - f0;
+      int nf;
+      if (f0 < 0 || cap64 < 0 || face_off[m + 1] > total_faces) {
+        nf = -3;
+      } else if (n < 4) {
+        nf = 0;
+      } else {
+        nf = hull_group<L>(pts + 3 * off[m], n, cap64 < 0x7fffffff ? (int)cap64 : 0x7fffffff, s,
+                           lane);
+      }
+      wave_sync();
+      int32_t* out = faces + 3 * f0;
+      for (int f = lane; f < nf; f += L) {
+        const uint32_t ids = s.face[f].ids;
+        out[3 * f] = (int32_t)(ids & 255u);
+        out[3 * f + 1] = (int32_t)((ids >> 8) & 255u);
+        out[3 * f + 2] = (int32_t)(ids >> 16);
+      }
+      if (lane == 0) nfaces[m] = nf;
+    }
+  }
+}
+
+// ------------------------------------------------ clouds of more points
+//
+// A block of T threads per cloud.  Insertions are serial and a cloud of 500
+// points has a thousand faces to test at each, so one wave per cloud leaves
+// the largest cloud of a call to run alone for milliseconds (4.4 ms for 2,000
+// ellipsoid clouds of 8-512 points, now 1.5 in all; an insertion into 512
+// points took 8 us, now 1.7).  The
+// whole block tests the faces (planes kept in LDS, as above) and notes the
+// visible ones; then the first wave alone does the short ordered part
+// (horizon, new faces): two block barriers per insertion, and what counts is
+// the chain of LDS round trips between them, so lists that would be written
+// and read again are avoided.  A face that leaves stays behind as a dead
+// slot, so nothing moves: slots are in creation order, which is the order the
+// reference's compaction keeps, and the first wave closes the gaps now and
+// then.  Each wave tests one contiguous run of slots, so the waves' lists of
+// visible faces joined together are in slot order.
+//
+// Directed edges of the visible faces: a bit per (start, end) for at most
+// 512 points, else a hash set.
+template <int NP>
+struct EdgeBits {
+  static constexpr int W = (NP + 31) / 32;
+  uint32_t bits[NP * W];
+  __device__ __forceinline__ void clear_all(int t, int threads) {
+    for (int i = t; i < NP * W; i += threads) bits[i] = 0u;
+  }
+  __device__ __forceinline__ bool insert(uint32_t a, uint32_t b) {
+    atomicOr(&bits[a * W + (b >> 5)], 1u << (b & 31u));
+    return true;
+  }
+  __device__ __forceinline__ bool found(uint32_t a, uint32_t b) const {
+    return (bits[a * W + (b >> 5)] >> (b & 31u)) & 1u;
+  }
+  __device__ __forceinline__ void erase(uint32_t a, uint32_t b) { bits[a * W + (b >> 5)] = 0u; }
+  __device__ __forceinline__ void end_step(int) {}
+};
+
+struct EdgeHash {
+  static constexpr uint32_t kSize = 4096, kNone = 0xffffffffu;
+  static constexpr int kProbes = 32;  // an edge lies within this many places of its own, or nowhere
+  uint32_t key[kSize];
+  __device__ __forceinline__ static uint32_t place(uint32_t k) {
+    return (k * 0x9e3779b1u) >> 20;
+  }
+  __device__ __forceinline__ void clear_all(int t, int threads) {
+    for (int i = t; i < (int)kSize; i += threads) key[i] = kNone;
+  }
+  __device__ __forceinline__ bool insert(uint32_t a, uint32_t b) {
+    const uint32_t k = a << 10 | b, h = place(k);
+    for (int p = 0; p < kProbes; p++) {
+      const uint32_t was = atomicCAS(&key[(h + p) & (kSize - 1u)], kNone, k);
+      if (was == kNone || was == k) return true;
+    }
+    return false;
+  }
+  __device__ __forceinline__ bool found(uint32_t a, uint32_t b) const {
+    const uint32_t k = a << 10 | b, h = place(k);
+    for (int p = 0; p < kProbes; p++) {
+      const uint32_t x = key[(h + p) & (kSize - 1u)];
+      if (x == k) return true;
+      if (x == kNone) return false;
+    }
+    return false;
+  }
+  __device__ __forceinline__ void erase(uint32_t, uint32_t) {}
+  __device__ __forceinline__ void end_step(int lane) {
+    for (int i = lane; i < (int)kSize; i += kWave) key[i] = kNone;
+  }
+};
+
+template <int T, int S, int NP>
+struct BlockHull {
+  static constexpr int kWaves = T / kWave;
+  static constexpr int kSeg = 128;        // visible faces a wave can note at one insertion
+  static constexpr int kRow = kWave / kWaves;  // of which the first wave takes these in one go
+  Tri face[S];                      // ids: 3 x 10 bits, kDead
+  float4 pt[NP];
+  std::conditional_t<NP <= 512, EdgeBits<NP>, EdgeHash> edges;
+  uint32_t seg[kWaves][kSeg];  // vertex ids of the visible faces each wave found
+  int cnt[2][kWaves];          // how many, by the parity of the step
+  int tail, status;            // read by every thread after an insertion
+  int full;                    // an edge found no place
+  int id[4];
+};
+constexpr uint32_t kDead = 0x80000000u;
+
+// Live slots of [0, tail) moved down in order, by one wave.  Returns their count.
+__device__ __forceinline__ int close_gaps(Tri* face, int tail, int lane) {
+  int w = 0;
+  for (int base = 0; base < tail; base += kWave) {
+    const int f = base + lane;
+    Tri F{};
+    if (f < tail) F = face[f];
+    const bool live = f < tail && !(F.ids & kDead);
+    const uint64_t b = ballot(live);
+    wave_sync();
+    if (live) face[w + rank_below(b, lane)] = F;
+    wave_sync();
+    w += __popcll(b);
+  }
+  return w;
+}
+
+// Whole block.  Returns the face count (faces in s.face[0..)), a status of
+// d_nfaces, or kToBig when the working set is too small.
+template <int T, int S, int NP>
+__device__ int hull_block(const float* __restrict__ P, int n, int cap, BlockHull<T, S, NP>& s) {
+  using B = BlockHull<T, S, NP>;
+  static_assert(NP <= 1024, "vertex ids are packed in 10 bits");
+  const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
+  const auto pt = [&](int i) { return s.pt[i]; };
+  __syncthreads();  // the block's previous cloud has been written out
+  s.edges.clear_all(t, T);
+  for (int i = t; i < n; i += T) s.pt[i] = make_float4(P[3 * i], P[3 * i + 1], P[3 * i + 2], 0.0f);
+  __syncthreads();
+  if (wave == 0) {
+    float lo[3], hi[3];
+    int lo_i[3], hi_i[3];
+    bool bad = false;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      lo[k] = INFINITY;
+      hi[k] = -INFINITY;
+      lo_i[k] = hi_i[k] = -1;
+    }
+    for (int i = lane; i < n; i += kWave) {
+      const float4 p4 = s.pt[i];
+      const float p[3] = {p4.x, p4.y, p4.z};
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        bad |= !isfinite(p[k]);
+        if (lo_i[k] < 0 || p[k] < lo[k]) { lo[k] = p[k]; lo_i[k] = i; }
+        if (hi_i[k] < 0 || p[k] > hi[k]) { hi[k] = p[k]; hi_i[k] = i; }
+      }
+    }
+    int id[4] = {0, 0, 0, 0};
+    int st = 4;
+    if (ballot(bad)) st = -2;
+    else if (!first_tetrahedron<kWave>(pt, n, lane, lo, lo_i, hi, hi_i, id)) st = 0;
+    else if (cap < 4) st = -1;
+    if (st == 4 && lane < 4) {
+      const int a = init_corner(id, lane, 0), b = init_corner(id, lane, 1),
+                c = init_corner(id, lane, 2);
+      s.face[lane] = make_tri(s.pt[a], s.pt[b], s.pt[c], (uint32_t)(a | b << 10 | c << 20));
+    }
+    if (lane == 0) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) s.id[k] = id[k];
+      s.tail = 4;
+      s.full = 0;
+      s.status = st;
+    }
+  }
+  __syncthreads();
+  if (s.status != 4) return s.status;
+  const int f0 = s.id[0], f1 = s.id[1], f2 = s.id[2], f3 = s.id[3];
+  int tail = 4, alive = 4;  // alive: the first wave's
+  float4 next = s.pt[0];
+  for (int q = 0, step = 0; q < n; q++) {
+    const float4 Q = next;
+    next = s.pt[q + 1 < n ? q + 1 : q];
+    if (q == f0 || q == f1 || q == f2 || q == f3) continue;
+    const int run = (tail + T - 1) / T * kWave;
+    const int end = min(tail, (wave + 1) * run);
+    int found = 0;
+    constexpr int U = 2;  // chunks in flight
+    for (int base = wave * run; base < end; base += U * kWave) {
+      Tri F[U];
+      float4 a[U];
+      bool v[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int f = base + u * kWave + lane;
+        F[u] = Tri{0.0f, 0.0f, 0.0f, kDead};
+        if (f < end) F[u] = s.face[f];
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++) a[u] = s.pt[F[u].ids & 1023u];
+#pragma unroll
+      for (int u = 0; u < U; u++) v[u] = !(F[u].ids & kDead) && vol6(F[u], a[u], Q) > 1e-7f;
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const uint64_t bv = ballot(v[u]);
+        if (v[u]) {
+          const int f = base + u * kWave + lane;
+          const uint32_t ids = F[u].ids;
+          const uint32_t x = ids & 1023u, y = (ids >> 10) & 1023u, z = ids >> 20;
+          s.face[f].ids = ids | kDead;
+          const int r = found + rank_below(bv, lane);
+          if (r < B::kSeg) s.seg[wave][r] = ids;
+          const bool i0 = s.edges.insert(x, y), i1 = s.edges.insert(y, z), i2 = s.edges.insert(z, x);
+          if (!i0 || !i1 || !i2) s.full = 1;
+        }
+        found += __popcll(bv);
+      }
+    }
+    int* cnt = s.cnt[step & 1];
+    if (lane == 0) cnt[wave] = found;
+    step++;
+    __syncthreads();
+    const int here = cnt[lane / B::kRow];  // found by the wave whose row this lane stands for
+    if (ballot(here != 0) == 0) continue;
+    if (wave == 0) {
+      int status = 4, nh = 0, nv = 0, at = tail;
+      if (ballot(here > B::kSeg) != 0 || s.full) {
+        status = kToBig;
+      } else {
+        // Each lane takes a visible face (valid: ids), in slot order: its
+        // edges whose reverse no visible face has are bases of new faces, in
+        // (face, edge) order.
+        const auto fan = [&](bool valid, uint32_t ids) {
+          const uint32_t x[3] = {ids & 1023u, (ids >> 10) & 1023u, ids >> 20};
+          float4 p[3];
+          bool hz[3];
+#pragma unroll
+          for (int e = 0; e < 3; e++) p[e] = s.pt[x[e]];
+#pragma unroll
+          for (int e = 0; e < 3; e++) hz[e] = valid && !s.edges.found(x[(e + 1) % 3], x[e]);
+          int r = at + nh;
+#pragma unroll
+          for (int e = 0; e < 3; e++) {
+            const uint64_t b = ballot(hz[e]);
+            r += rank_below(b, lane);
+            nh += __popcll(b);
+          }
+#pragma unroll
+          for (int e = 0; e < 3; e++) {
+            if (hz[e]) {
+              if (r < S)
+                s.face[r] = make_tri(p[e], p[(e + 1) % 3], Q,
+                                     x[e] | x[(e + 1) % 3] << 10 | (uint32_t)q << 20);
+              r++;
+            }
+          }
+        };
+        const auto unmark = [&](uint32_t ids) {
+          const uint32_t x0 = ids & 1023u, x1 = (ids >> 10) & 1023u, x2 = ids >> 20;
+          s.edges.erase(x0, x1);
+          s.edges.erase(x1, x2);
+          s.edges.erase(x2, x0);
+        };
+        if (ballot(here > B::kRow) == 0) {
+          // a few per wave, as always but on dense clouds: lane (wave, rank)
+          const int w = lane / B::kRow, k = lane - w * B::kRow;
+          const bool valid = k < here;
+          const uint32_t ids = valid ? s.seg[w][k] : 0u;
+          nv = __popcll(ballot(valid));
+          fan(valid, ids);
+          if (valid) unmark(ids);
+        } else {
+          int pre[B::kWaves + 1];  // visible faces of the waves before
+          pre[0] = 0;
+#pragma unroll
+          for (int w = 0; w < B::kWaves; w++) pre[w + 1] = pre[w] + cnt[w];
+          nv = pre[B::kWaves];
+          const auto visible = [&](int j) {
+            int w = 0, st = 0;
+#pragma unroll
+            for (int k = 1; k < B::kWaves; k++) {
+              w = j >= pre[k] ? k : w;
+              st = j >= pre[k] ? pre[k] : st;
+            }
+            return s.seg[w][j - st];
+          };
+          for (int base = 0; base < nv; base += kWave) {
+            const bool valid = base + lane < nv;
+            fan(valid, valid ? visible(base + lane) : 0u);
+          }
+          for (int j = lane; j < nv; j += kWave) unmark(visible(j));
+        }
+        s.edges.end_step(lane);
+        alive += nh - nv;
+        at += nh;
+        if (alive > cap) {
+          status = -1;
+        } else if (at > S) {
+          status = kToBig;
+        } else if (at > S - 384 || at > 2 * alive + T) {
+          wave_sync();
+          at = close_gaps(s.face, at, lane);
+        }
+      }
+      if (lane == 0) {
+        s.tail = at;
+        s.status = status;
+      }
+    }
+    __syncthreads();
+    if (s.status != 4) return s.status;
+    tail = s.tail;
+  }
+  __syncthreads();
+  if (wave == 0) {
+    const int nf = close_gaps(s.face, tail, lane);
+    if (lane == 0) s.tail = nf;
+  }
+  __syncthreads();
+  return s.tail;
+}
+
+// Clouds of NMIN..NP points and those an earlier kernel passed on as FROM; the
+// blocks of the grid take the clouds in turn.  PASS: how this kernel passes on.
+template <int T, int S, int NMIN, int NP, int FROM, int PASS>
+__global__ __launch_bounds__(T) void k_hull_block(const float* __restrict__ pts,
+                                                  const int64_t* __restrict__ off,
+                                                  const int32_t* __restrict__ cnt, int nm,
+                                                  const int64_t* __restrict__ face_off,
+                                                  int64_t total_faces,
+                                                  int32_t* __restrict__ faces,
+                                                  int32_t* __restrict__ nfaces) {
+  __shared__ BlockHull<T, S, NP> s;
+  const int lane = threadIdx.x & (kWave - 1);
+  for (int64_t first = blockIdx.x; first < nm; first += (int64_t)gridDim.x * kWave) {
+    const int64_t mine = first + (int64_t)gridDim.x * lane;
+    int n_mine = -1;
+    bool take = false;
+    if (mine < nm) {
+      n_mine = cnt[mine];
+      take = n_mine >= NMIN ? n_mine <= NP : nfaces[mine] == FROM;
+    }
+    uint64_t todo = ballot(take);  // the same in every wave of the block
+    while (todo != 0) {
+      const int src = (int)__builtin_ctzll(todo);
+      todo &= todo - 1;
+      const int64_t m = first + (int64_t)gridDim.x * src;
+      const int n = __shfl(n_mine, src, kWave);
+      const int64_t f0 = face_off[m], cap64 = face_off[m + 1] - f0;
+      int nf;
+      if (f0 < 0 || cap64 < 0 || face_off[m + 1] > total_faces) {
+        nf = -3;
+      } else {
+        nf = hull_block(pts + 3 * off[m], n, cap64 < 0x7fffffff ? (int)cap64 : 0x7fffffff, s);
+        if (nf == kToBig) nf = PASS;
+      }
+      int32_t* out = faces + 3 * f0;
+      for (int f = threadIdx.x; f < nf; f += T) {
+        const uint32_t ids = s.face[f].ids;
+        out[3 * f] = (int32_t)(ids & 1023u);
+        out[3 * f + 1] = (int32_t)((ids >> 10) & 1023u);
+        out[3 * f + 2] = (int32_t)(ids >> 20);
+      }
+      // every wave has read its clouds' nfaces before this write only for the
+      // chunk at hand; a result is never FROM, so a later read cannot take it
+      if (threadIdx.x == 0) nfaces[m] = nf;
+    }
+  }
+}
+
+// ------------------------------------------------------ any other cloud
+//
+// More than 1,024 points, or a working set past the block's LDS: one wave per
+// cloud over the output buffer and the workspace.
 
 __device__ __forceinline__ float vol6(const float* __restrict__ p, int a, int b, int c,
                                       float qx, float qy, float qz) {
@@ -37,12 +743,6 @@ __device__ __forceinline__ float vol6(const float* __restrict__ p, int a, int b,
   const float dx = qx - ax, dy = qy - ay, dz = qz - az;
   const float nx = by * cz - bz * cy, ny = bz * cx - bx * cz, nz = bx * cy - by * cx;
   return nx * dx + ny * dy + nz * dz;
-}
-
-__device__ __forceinline__ uint64_t ballot(bool v) { return __ballot(v); }
-
-__device__ __forceinline__ int rank_below(uint64_t mask, int lane) {
-  return __popcll(mask & ((uint64_t(1) << lane) - 1));
 }
 
 // Wave argmax over (value, index): larger value, then lower index.  Lanes
@@ -69,39 +769,9 @@ __device__ __forceinline__ void wave_argmin(float& v, int& i) {
   }
 }
 
-// One wave per cloud.  faces/scratch of cloud m start at 3 * face_off[m] and
-// hold face_off[m + 1] - face_off[m] faces; nfaces[m] = face count, 0 for no
-// hull (fewer than 4 points, collinear or coplanar), -1 when the capacity is
-// exceeded, -2 for a non-finite coordinate, -3 when the cloud's face range is
-// not inside [0, total_faces] (nothing is written for it).
-__global__ __launch_bounds__(kWave) void k_hull(const float* __restrict__ pts,
-                                                const int64_t* __restrict__ off,
-                                                const int32_t* __restrict__ cnt,
-                                                const int64_t* __restrict__ face_off,
-                                                int64_t total_faces,
-                                                int32_t* __restrict__ faces,
-                                                int32_t* __restrict__ nfaces,
-                                                int32_t* __restrict__ scratch) {
-  const int m = blockIdx.x;
-  const int lane = threadIdx.x;
-  const int n = cnt[m];
-  const float* P = pts + 3 * off[m];
-  const int64_t f0 = face_off[m];
-  const int64_t cap64 = face_off[m + 1] - f0;
-  if (f0 < 0 || cap64 < 0 || face_off[m + 1] > total_faces) {
-    if (lane == 0) nfaces[m] = -3;
-    return;
-  }
-  const int cap = cap64 < 0x7fffffff ? (int)cap64 : 0x7fffffff;
-  __shared__ int32_t lds[6 * kLdsFaces];
-  const bool in_lds = cap64 <= kLdsFaces;
-  int32_t* F = in_lds ? lds : faces + 3 * f0;                          // 3 * cap entries
-  int32_t* vis = in_lds ? lds + 3 * kLdsFaces : scratch + 3 * f0;     // cap entries
-  int32_t* hor = in_lds ? lds + 4 * kLdsFaces : scratch + 3 * f0 + cap64;  // 2 * cap
-  if (n < 4) {
-    if (lane == 0) nfaces[m] = 0;
-    return;
-  }
+// F: 3 * cap entries, vis: cap, hor: 2 * cap.
+__device__ int hull_global(const float* __restrict__ P, int n, int cap, int32_t* F, int32_t* vis,
+                           int32_t* hor, int lane) {
   // axis extremes (first index on ties), rejecting non-finite input
   float mnv[3], mxv[3];
   int mni[3], mxi[3];
@@ -122,8 +792,7 @@ __global__ __launch_bounds__(kWave) void k_hull(const float* __restrict__ pts,
     }
   }
   if (ballot(bad)) {
-    if (lane == 0) nfaces[m] = -2;
-    return;
+    return -2;
   }
 #pragma unroll
   for (int k = 0; k < 3; k++) {
@@ -166,8 +835,7 @@ __global__ __launch_bounds__(kWave) void k_hull(const float* __restrict__ pts,
     i2 = bi;
   }
   if (i2 < 0) {
-    if (lane == 0) nfaces[m] = 0;
-    return;
+    return 0;
   }
   // farthest from the plane i0-i1-i2
   int i3;
@@ -184,8 +852,7 @@ __global__ __launch_bounds__(kWave) void k_hull(const float* __restrict__ pts,
     i3 = bi;
   }
   if (i3 < 0) {
-    if (lane == 0) nfaces[m] = 0;
-    return;
+    return 0;
   }
   if (vol6(P, i0, i1, i2, P[3 * i3], P[3 * i3 + 1], P[3 * i3 + 2]) > 0) {
     const int t = i1;
@@ -193,8 +860,7 @@ __global__ __launch_bounds__(kWave) void k_hull(const float* __restrict__ pts,
     i2 = t;
   }
   if (cap < 4) {
-    if (lane == 0) nfaces[m] = -1;
-    return;
+    return -1;
   }
   if (lane < 12) {
     const int init[12] = {i0, i1, i2, i0, i2, i3, i0, i3, i1, i1, i3, i2};
@@ -270,8 +936,7 @@ __global__ __launch_bounds__(kWave) void k_hull(const float* __restrict__ pts,
       __syncthreads();
     }
     if (nh > cap || w + nh > cap) {
-      if (lane == 0) nfaces[m] = -1;
-      return;
+      return -1;
     }
     for (int r = lane; r < nh; r += kWave) {
       F[3 * (w + r)] = hor[2 * r];
@@ -281,55 +946,130 @@ __global__ __launch_bounds__(kWave) void k_hull(const float* __restrict__ pts,
     nf = w + nh;
     __syncthreads();
   }
-  if (in_lds) {
-    int32_t* out = faces + 3 * f0;
-    for (int i = lane; i < 3 * nf; i += kWave) out[i] = F[i];
-  }
-  if (lane == 0) nfaces[m] = nf;
+  return nf;
 }
 
-// One thread per cloud: moments summed in face order (mesh_builder.cpp:433-462),
-// centre of mass as center_hull_verts shifts by it (0 below volume 1e-10) and
-// the inertia factors of compute_hull_inertia_k (:464-481).
-__global__ __launch_bounds__(64) void k_hull_moments(const float* __restrict__ pts,
-                                                     const int64_t* __restrict__ off,
-                                                     const int32_t* __restrict__ faces,
-                                                     const int64_t* __restrict__ face_off,
-                                                     const int32_t* __restrict__ nfaces, int nm,
-                                                     double* __restrict__ moments,
-                                                     float* __restrict__ com,
-                                                     float* __restrict__ inertia_k) {
-  const int m = blockIdx.x * 64 + threadIdx.x;
-  if (m >= nm) return;
-  const float* P = pts + 3 * off[m];
-  const int32_t* F = faces + 3 * face_off[m];
-  const int nf = nfaces[m] > 0 ? nfaces[m] : 0;
-  double vol = 0, cx = 0, cy = 0, cz = 0, ix2 = 0, iy2 = 0, iz2 = 0;
-  for (int f = 0; f < nf; f++) {
-    const float* a = P + 3 * F[3 * f];
-    const float* b = P + 3 * F[3 * f + 1];
-    const float* c = P + 3 * F[3 * f + 2];
-    const double dv =
-        ((double)a[0] * ((double)b[1] * (double)c[2] - (double)b[2] * (double)c[1]) -
-         (double)a[1] * ((double)b[0] * (double)c[2] - (double)b[2] * (double)c[0]) +
-         (double)a[2] * ((double)b[0] * (double)c[1] - (double)b[1] * (double)c[0])) /
-        6.0;
-    vol += dv;
-    cx += dv * (a[0] + b[0] + c[0]);
-    cy += dv * (a[1] + b[1] + c[1]);
-    cz += dv * (a[2] + b[2] + c[2]);
-    ix2 += dv / 10.0 *
-           ((double)a[0] * a[0] + (double)a[0] * b[0] + (double)b[0] * b[0] +
-            (double)a[0] * c[0] + (double)b[0] * c[0] + (double)c[0] * c[0]);
-    iy2 += dv / 10.0 *
-           ((double)a[1] * a[1] + (double)a[1] * b[1] + (double)b[1] * b[1] +
-            (double)a[1] * c[1] + (double)b[1] * c[1] + (double)c[1] * c[1]);
-    iz2 += dv / 10.0 *
-           ((double)a[2] * a[2] + (double)a[2] * b[2] + (double)b[2] * b[2] +
-            (double)a[2] * c[2] + (double)b[2] * c[2] + (double)c[2] * c[2]);
+// Clouds of more than NMAX points and those passed on as kToGeneral, one
+// wave each; the waves take the clouds in turn.
+template <int NMAX>
+__global__ __launch_bounds__(kWave) void k_hull_global(const float* __restrict__ pts,
+                                                       const int64_t* __restrict__ off,
+                                                       const int32_t* __restrict__ cnt, int nm,
+                                                       const int64_t* __restrict__ face_off,
+                                                       int64_t total_faces,
+                                                       int32_t* __restrict__ faces,
+                                                       int32_t* __restrict__ nfaces,
+                                                       int32_t* __restrict__ scratch) {
+  const int lane = threadIdx.x;
+  for (int64_t first = blockIdx.x; first < nm; first += (int64_t)gridDim.x * kWave) {
+    const int64_t mine = first + (int64_t)gridDim.x * lane;
+    bool take = false;
+    if (mine < nm) take = cnt[mine] > NMAX || nfaces[mine] == kToGeneral;
+    uint64_t todo = ballot(take);
+    while (todo != 0) {
+      const int64_t m = first + (int64_t)gridDim.x * (int)__builtin_ctzll(todo);
+      todo &= todo - 1;
+      const int64_t f0 = face_off[m], cap64 = face_off[m + 1] - f0;
+      int nf = -3;
+      if (!(f0 < 0 || cap64 < 0 || face_off[m + 1] > total_faces))
+        nf = hull_global(pts + 3 * off[m], cnt[m], cap64 < 0x7fffffff ? (int)cap64 : 0x7fffffff,
+                         faces + 3 * f0, scratch + 3 * f0, scratch + 3 * f0 + cap64, lane);
+      if (lane == 0) nfaces[m] = nf;
+    }
   }
-  double* mo = moments + 7 * (int64_t)m;
-  mo[0] = vol; mo[1] = cx; mo[2] = cy; mo[3] = cz; mo[4] = ix2; mo[5] = iy2; mo[6] = iz2;
+}
+
+// Moments summed in face order (mesh_builder.cpp:433-462), centre of mass as
+// center_hull_verts shifts by it (0 below volume 1e-10) and the inertia factors
+// of compute_hull_inertia_k (:464-481).  L lanes per cloud work out the terms of
+// L faces at a time; then lane k < 7 adds the k-th moment's terms one by one
+// in face order (the sums' bits depend on it).  A wave holds 64 / 16 clouds
+// of at most 64 faces, a larger cloud gets the wave to itself.  Bound by the
+// gathers and the chain of additions; with one thread per cloud 100,000
+// clouds of 8-32 points took 95 us (now 43), 2,000 of 8-512 points 570 (51).
+constexpr int kMom = 7;
+
+template <int L>
+__device__ __forceinline__ double hull_moment(const float* __restrict__ P,
+                                              const int32_t* __restrict__ F, int nf,
+                                              double (*term)[kWave], int base_lane, int lane) {
+  double acc = 0.0;
+  for (int base = 0; base < nf; base += L) {
+    const int f = base + lane;
+    if (f < nf) {
+      const float* a = P + 3 * (int64_t)F[3 * (int64_t)f];
+      const float* b = P + 3 * (int64_t)F[3 * (int64_t)f + 1];
+      const float* c = P + 3 * (int64_t)F[3 * (int64_t)f + 2];
+      const double dv =
+          ((double)a[0] * ((double)b[1] * (double)c[2] - (double)b[2] * (double)c[1]) -
+           (double)a[1] * ((double)b[0] * (double)c[2] - (double)b[2] * (double)c[0]) +
+           (double)a[2] * ((double)b[0] * (double)c[1] - (double)b[1] * (double)c[0])) /
+          6.0;
+      const int at = base_lane + lane;
+      term[0][at] = dv;
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        term[1 + k][at] = dv * (a[k] + b[k] + c[k]);
+        term[4 + k][at] = dv / 10.0 *
+                          ((double)a[k] * a[k] + (double)a[k] * b[k] + (double)b[k] * b[k] +
+                           (double)a[k] * c[k] + (double)b[k] * c[k] + (double)c[k] * c[k]);
+      }
+    }
+    wave_sync();
+    if (lane < kMom) {
+      const int m = nf - base < L ? nf - base : L;
+      const double* t = term[lane] + base_lane;
+      int j = 0;
+      for (; j + 8 <= m; j += 8) {
+        double x[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) x[u] = t[j + u];
+#pragma unroll
+        for (int u = 0; u < 8; u++) acc += x[u];
+      }
+      for (; j < m; j++) acc += t[j];
+    }
+    wave_sync();
+  }
+  return acc;
+}
+
+__global__ __launch_bounds__(kWave) void k_hull_moments(const float* __restrict__ pts,
+                                                        const int64_t* __restrict__ off,
+                                                        const int32_t* __restrict__ faces,
+                                                        const int64_t* __restrict__ face_off,
+                                                        const int32_t* __restrict__ nfaces, int nm,
+                                                        double* __restrict__ moments,
+                                                        float* __restrict__ com,
+                                                        float* __restrict__ inertia_k) {
+  constexpr int L = 16, G = kWave / L;
+  __shared__ double term[kMom][kWave];
+  const int lane = threadIdx.x, sub = lane & (L - 1), g0 = lane & ~(L - 1);
+  const int m = blockIdx.x * G + lane / L;
+  int nf = 0;
+  const float* P = pts;
+  const int32_t* F = faces;
+  if (m < nm) {
+    nf = nfaces[m] > 0 ? nfaces[m] : 0;
+    P = pts + 3 * off[m];
+    F = faces + 3 * face_off[m];
+  }
+  double acc = hull_moment<L>(P, F, nf <= kWave ? nf : 0, term, g0, sub);
+  for (uint64_t big = ballot(sub == 0 && nf > kWave); big != 0; big &= big - 1) {
+    const int src = (int)__builtin_ctzll(big);
+    const int mb = blockIdx.x * G + src / L;
+    const double a = hull_moment<kWave>(pts + 3 * off[mb], faces + 3 * face_off[mb], nfaces[mb],
+                                        term, 0, lane);
+    const double mine = __shfl(a, sub, kWave);  // lanes 0..6 hold the moments
+    if (g0 == src) acc = mine;
+  }
+  double mo[kMom];
+#pragma unroll
+  for (int k = 0; k < kMom; k++) mo[k] = __shfl(acc, k, L);
+  if (m >= nm) return;
+  if (sub < kMom) moments[kMom * (int64_t)m + sub] = acc;
+  if (sub != 0) return;
+  const double vol = mo[0];
   float* co = com + 3 * (int64_t)m;
   float* ko = inertia_k + 3 * (int64_t)m;
   if (vol < 1e-10) {
@@ -337,13 +1077,12 @@ __global__ __launch_bounds__(64) void k_hull_moments(const float* __restrict__ p
     ko[0] = ko[1] = ko[2] = 1.0f / 10.0f;
     return;
   }
-  const double c0 = cx / (4.0 * vol), c1 = cy / (4.0 * vol), c2 = cz / (4.0 * vol);
-  co[0] = (float)c0;
-  co[1] = (float)c1;
-  co[2] = (float)c2;
-  ko[0] = (float)((ix2 - vol * c0 * c0) / vol);
-  ko[1] = (float)((iy2 - vol * c1 * c1) / vol);
-  ko[2] = (float)((iz2 - vol * c2 * c2) / vol);
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    const double c = mo[1 + k] / (4.0 * vol);
+    co[k] = (float)c;
+    ko[k] = (float)((mo[4 + k] - vol * c * c) / vol);
+  }
 }
 
 // points of cloud m minus com[m], one thread per point
@@ -382,8 +1121,38 @@ ogjk_status ogjk_build_hulls(const float* d_points, const int64_t* d_point_off,
   const size_t need = (size_t)total_faces * 3 * sizeof(int32_t);
   if (!d_workspace || workspace_bytes < need)
     return ogjk_fail(OGJK_ERR_INVALID, "workspace of %zu bytes needed", need);
-  hipLaunchKernelGGL(k_hull, dim3((unsigned)n_clouds), dim3(kWave), 0, (hipStream_t)stream,
-                     d_points, d_point_off, d_point_cnt, d_face_off, total_faces, d_faces,
+  const hipStream_t st = (hipStream_t)stream;
+  // Sizes are on the device, so every class's kernel goes over the counts (an
+  // idle one takes about 4 us) and takes its own clouds; one whose working set
+  // outgrows its LDS leaves a mark in d_nfaces and a later kernel starts it
+  // again.  Classes, measured alone on equal clouds: up to 32 points 16 lanes
+  // a cloud, then a wave (1.2 us an insertion at 128 points, 1.7 as a block),
+  // then a block as large as 2 n faces fill (at 512 points 1.7 us an
+  // insertion, one wave over global memory 8), and past 1,024 points, where
+  // ids and planes no longer fit, one wave over global memory as before.
+  // Blocks are launched per cloud up to 2,048, so that the dispatcher balances
+  // them; larger batches take the clouds in turn.
+  const auto grid = [&](int clouds_per_block, int64_t most) {
+    const int64_t b = ((int64_t)n_clouds + clouds_per_block - 1) / clouds_per_block;
+    return dim3((unsigned)(b < most ? b : most));
+  };
+  hipLaunchKernelGGL((k_hull_group<16, 0, 32, 96>), grid(4, 1 << 20), dim3(kWave), 0, st, d_points,
+                     d_point_off, d_point_cnt, n_clouds, d_face_off, total_faces, d_faces,
+                     d_nfaces);
+  hipLaunchKernelGGL((k_hull_group<64, 33, 128, 528>), grid(1, 2560), dim3(kWave), 0, st, d_points,
+                     d_point_off, d_point_cnt, n_clouds, d_face_off, total_faces, d_faces,
+                     d_nfaces);
+  hipLaunchKernelGGL((k_hull_block<256, 1024, 129, 256, kNowhere, kToBlock>), grid(1, 2048),
+                     dim3(256), 0, st, d_points, d_point_off, d_point_cnt, n_clouds, d_face_off,
+                     total_faces, d_faces, d_nfaces);
+  hipLaunchKernelGGL((k_hull_block<512, 2048, 257, 512, kToBlock, kToBig>), grid(1, 2048),
+                     dim3(512), 0, st, d_points, d_point_off, d_point_cnt, n_clouds, d_face_off,
+                     total_faces, d_faces, d_nfaces);
+  hipLaunchKernelGGL((k_hull_block<1024, 7168, 513, 1024, kToBig, kToGeneral>), grid(1, 512),
+                     dim3(1024), 0, st, d_points, d_point_off, d_point_cnt, n_clouds, d_face_off,
+                     total_faces, d_faces, d_nfaces);
+  hipLaunchKernelGGL((k_hull_global<1024>), grid(1, 4096), dim3(kWave), 0, st, d_points,
+                     d_point_off, d_point_cnt, n_clouds, d_face_off, total_faces, d_faces,
                      d_nfaces, (int32_t*)d_workspace);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? OGJK_OK : hip_err(e, "hull launch");
@@ -398,7 +1167,7 @@ ogjk_status ogjk_hull_moments(const float* d_points, const int64_t* d_point_off,
   if (!d_points || !d_point_off || !d_faces || !d_face_off || !d_nfaces || !d_moments ||
       !d_com || !d_inertia_k)
     return ogjk_fail(OGJK_ERR_INVALID, "NULL argument");
-  hipLaunchKernelGGL(k_hull_moments, dim3((unsigned)((n_clouds + 63) / 64)), dim3(64), 0,
+  hipLaunchKernelGGL(k_hull_moments, dim3((unsigned)((n_clouds + 3) / 4)), dim3(kWave), 0,
                      (hipStream_t)stream, d_points, d_point_off, d_faces, d_face_off, d_nfaces,
                      n_clouds, d_moments, d_com, d_inertia_k);
   const hipError_t e = hipGetLastError();

@@ -8,6 +8,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #pragma clang fp contract(off)
 
 
@@ -49,6 +51,37 @@ OGJK_DEV uint64_t group_ballot(bool p) {
     const int base = lane_id() & ~(LPP - 1);
     return (b >> base) & ((1ull << LPP) - 1);
   }
+}
+
+// A group's ballot in the narrowest form: bit l = lane l of the group, in 32
+// bits for groups of up to half a wave.
+template <int LPP>
+using lane_mask = std::conditional_t<LPP == 64, uint64_t, uint32_t>;
+
+template <int LPP>
+OGJK_DEV lane_mask<LPP> lanes_where(bool p) {
+  const uint64_t b = __ballot(p);
+  if constexpr (LPP == 64) {
+    return b;
+  } else {
+    const uint32_t half = (lane_id() & 32) ? (uint32_t)(b >> 32) : (uint32_t)b;
+    if constexpr (LPP == 32) return half;
+    else return (half >> (lane_id() & 31 & ~(LPP - 1))) & ((1u << LPP) - 1u);
+  }
+}
+template <int LPP>
+OGJK_DEV int count_lanes(lane_mask<LPP> m) {
+  if constexpr (LPP == 64) return __popcll(m);
+  else return __popc(m);
+}
+// Set bits of m below lane l of the group (l = this lane's index in it).
+template <int LPP>
+OGJK_DEV int lanes_below(lane_mask<LPP> m, int l) {
+  if constexpr (LPP == 64)
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                          __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+  else
+    return __popc(m & ((1u << l) - 1u));
 }
 
 template <int LPP>
