@@ -399,6 +399,11 @@ __global__ __launch_bounds__(kWave) void k_hull_group(const float* __restrict__ 
 // then.  Each wave tests one contiguous run of slots, so the waves' lists of
 // visible faces joined together are in slot order.
 //
+// The largest class keeps vertex ids alone (4 bytes a face, the normal formed
+// anew from the three corners), for the room: on dense, nearly coplanar
+// surfaces the face list grows tenfold within the last insertions, and such a
+// cloud of 8-512 points took 10 ms and more in the general kernel.
+//
 // Directed edges of the visible faces: a bit per (start, end) for at most
 // 512 points, else a hash set.
 template <int NP>
@@ -420,11 +425,11 @@ struct EdgeBits {
 };
 
 struct EdgeHash {
-  static constexpr uint32_t kSize = 4096, kNone = 0xffffffffu;
+  static constexpr uint32_t kSize = 8192, kNone = 0xffffffffu;
   static constexpr int kProbes = 32;  // an edge lies within this many places of its own, or nowhere
-  uint32_t key[kSize];
+  alignas(16) uint32_t key[kSize];
   __device__ __forceinline__ static uint32_t place(uint32_t k) {
-    return (k * 0x9e3779b1u) >> 20;
+    return (k * 0x9e3779b1u) >> 19;
   }
   __device__ __forceinline__ void clear_all(int t, int threads) {
     for (int i = t; i < (int)kSize; i += threads) key[i] = kNone;
@@ -448,16 +453,20 @@ struct EdgeHash {
   }
   __device__ __forceinline__ void erase(uint32_t, uint32_t) {}
   __device__ __forceinline__ void end_step(int lane) {
-    for (int i = lane; i < (int)kSize; i += kWave) key[i] = kNone;
+    for (int i = lane; i < (int)kSize / 4; i += kWave)
+      ((uint4*)key)[i] = uint4{kNone, kNone, kNone, kNone};
   }
 };
 
 template <int T, int S, int NP>
 struct BlockHull {
   static constexpr int kWaves = T / kWave;
-  static constexpr int kSeg = 128;        // visible faces a wave can note at one insertion
+  static constexpr bool kPlanes = NP <= 512;
+  using Face = std::conditional_t<kPlanes, Tri, uint32_t>;
+  static constexpr int kSeg = kPlanes ? 128 : 256;  // visible faces a wave notes at an insertion
+  static constexpr int kRoom = kPlanes ? 384 : 2048;  // slots an insertion finds free
   static constexpr int kRow = kWave / kWaves;  // of which the first wave takes these in one go
-  Tri face[S];                      // ids: 3 x 10 bits, kDead
+  Face face[S];                     // ids: 3 x 10 bits, kDead
   float4 pt[NP];
   std::conditional_t<NP <= 512, EdgeBits<NP>, EdgeHash> edges;
   uint32_t seg[kWaves][kSeg];  // vertex ids of the visible faces each wave found
@@ -468,14 +477,18 @@ struct BlockHull {
 };
 constexpr uint32_t kDead = 0x80000000u;
 
+__device__ __forceinline__ uint32_t& ids_of(Tri& f) { return f.ids; }
+__device__ __forceinline__ uint32_t& ids_of(uint32_t& f) { return f; }
+
 // Live slots of [0, tail) moved down in order, by one wave.  Returns their count.
-__device__ __forceinline__ int close_gaps(Tri* face, int tail, int lane) {
+template <class Face>
+__device__ __forceinline__ int close_gaps(Face* face, int tail, int lane) {
   int w = 0;
   for (int base = 0; base < tail; base += kWave) {
     const int f = base + lane;
-    Tri F{};
+    Face F{};
     if (f < tail) F = face[f];
-    const bool live = f < tail && !(F.ids & kDead);
+    const bool live = f < tail && !(ids_of(F) & kDead);
     const uint64_t b = ballot(live);
     wave_sync();
     if (live) face[w + rank_below(b, lane)] = F;
@@ -493,6 +506,10 @@ __device__ int hull_block(const float* __restrict__ P, int n, int cap, BlockHull
   static_assert(NP <= 1024, "vertex ids are packed in 10 bits");
   const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
   const auto pt = [&](int i) { return s.pt[i]; };
+  const auto put = [&](int f, float4 a, float4 b, float4 c, uint32_t ids) {
+    if constexpr (B::kPlanes) s.face[f] = make_tri(a, b, c, ids);
+    else s.face[f] = ids;
+  };
   __syncthreads();  // the block's previous cloud has been written out
   s.edges.clear_all(t, T);
   for (int i = t; i < n; i += T) s.pt[i] = make_float4(P[3 * i], P[3 * i + 1], P[3 * i + 2], 0.0f);
@@ -525,7 +542,7 @@ __device__ int hull_block(const float* __restrict__ P, int n, int cap, BlockHull
     if (st == 4 && lane < 4) {
       const int a = init_corner(id, lane, 0), b = init_corner(id, lane, 1),
                 c = init_corner(id, lane, 2);
-      s.face[lane] = make_tri(s.pt[a], s.pt[b], s.pt[c], (uint32_t)(a | b << 10 | c << 20));
+      put(lane, s.pt[a], s.pt[b], s.pt[c], (uint32_t)(a | b << 10 | c << 20));
     }
     if (lane == 0) {
 #pragma unroll
@@ -549,27 +566,32 @@ __device__ int hull_block(const float* __restrict__ P, int n, int cap, BlockHull
     int found = 0;
     constexpr int U = 2;  // chunks in flight
     for (int base = wave * run; base < end; base += U * kWave) {
-      Tri F[U];
-      float4 a[U];
+      typename B::Face F[U];
       bool v[U];
 #pragma unroll
       for (int u = 0; u < U; u++) {
         const int f = base + u * kWave + lane;
-        F[u] = Tri{0.0f, 0.0f, 0.0f, kDead};
+        F[u] = typename B::Face{};
+        ids_of(F[u]) = kDead;
         if (f < end) F[u] = s.face[f];
       }
 #pragma unroll
-      for (int u = 0; u < U; u++) a[u] = s.pt[F[u].ids & 1023u];
-#pragma unroll
-      for (int u = 0; u < U; u++) v[u] = !(F[u].ids & kDead) && vol6(F[u], a[u], Q) > 1e-7f;
+      for (int u = 0; u < U; u++) {
+        const uint32_t ids = ids_of(F[u]);
+        const float4 a = s.pt[ids & 1023u];
+        float d;
+        if constexpr (B::kPlanes) d = vol6(F[u], a, Q);
+        else d = vol6(a, s.pt[(ids >> 10) & 1023u], s.pt[(ids >> 20) & 1023u], Q);
+        v[u] = !(ids & kDead) && d > 1e-7f;
+      }
 #pragma unroll
       for (int u = 0; u < U; u++) {
         const uint64_t bv = ballot(v[u]);
         if (v[u]) {
           const int f = base + u * kWave + lane;
-          const uint32_t ids = F[u].ids;
+          const uint32_t ids = ids_of(F[u]);
           const uint32_t x = ids & 1023u, y = (ids >> 10) & 1023u, z = ids >> 20;
-          s.face[f].ids = ids | kDead;
+          ids_of(s.face[f]) = ids | kDead;
           const int r = found + rank_below(bv, lane);
           if (r < B::kSeg) s.seg[wave][r] = ids;
           const bool i0 = s.edges.insert(x, y), i1 = s.edges.insert(y, z), i2 = s.edges.insert(z, x);
@@ -611,8 +633,7 @@ __device__ int hull_block(const float* __restrict__ P, int n, int cap, BlockHull
           for (int e = 0; e < 3; e++) {
             if (hz[e]) {
               if (r < S)
-                s.face[r] = make_tri(p[e], p[(e + 1) % 3], Q,
-                                     x[e] | x[(e + 1) % 3] << 10 | (uint32_t)q << 20);
+                put(r, p[e], p[(e + 1) % 3], Q, x[e] | x[(e + 1) % 3] << 10 | (uint32_t)q << 20);
               r++;
             }
           }
@@ -659,7 +680,7 @@ __device__ int hull_block(const float* __restrict__ P, int n, int cap, BlockHull
           status = -1;
         } else if (at > S) {
           status = kToBig;
-        } else if (at > S - 384 || at > 2 * alive + T) {
+        } else if (at > S - B::kRoom || at > 2 * alive + T) {
           wave_sync();
           at = close_gaps(s.face, at, lane);
         }
@@ -718,7 +739,7 @@ __global__ __launch_bounds__(T) void k_hull_block(const float* __restrict__ pts,
       }
       int32_t* out = faces + 3 * f0;
       for (int f = threadIdx.x; f < nf; f += T) {
-        const uint32_t ids = s.face[f].ids;
+        const uint32_t ids = ids_of(s.face[f]);
         out[3 * f] = (int32_t)(ids & 1023u);
         out[3 * f + 1] = (int32_t)((ids >> 10) & 1023u);
         out[3 * f + 2] = (int32_t)(ids >> 20);
@@ -1148,7 +1169,7 @@ ogjk_status ogjk_build_hulls(const float* d_points, const int64_t* d_point_off,
   hipLaunchKernelGGL((k_hull_block<512, 2048, 257, 512, kToBlock, kToBig>), grid(1, 2048),
                      dim3(512), 0, st, d_points, d_point_off, d_point_cnt, n_clouds, d_face_off,
                      total_faces, d_faces, d_nfaces);
-  hipLaunchKernelGGL((k_hull_block<1024, 7168, 513, 1024, kToBig, kToGeneral>), grid(1, 512),
+  hipLaunchKernelGGL((k_hull_block<1024, 16384, 513, 1024, kToBig, kToGeneral>), grid(1, 512),
                      dim3(1024), 0, st, d_points, d_point_off, d_point_cnt, n_clouds, d_face_off,
                      total_faces, d_faces, d_nfaces);
   hipLaunchKernelGGL((k_hull_global<1024>), grid(1, 4096), dim3(kWave), 0, st, d_points,
