@@ -110,17 +110,46 @@ OGJK_DEV Sweep32 sweep32_begin(D3 dir) {
   return s;
 }
 
-template <int STRIDE>
-OGJK_DEV void sweep32_step(const Body<float, STRIDE>& b, int i, Sweep32& s) {
-  const float px = b.rx(i), py = b.ry(i), pz = b.rz(i);
-  const float d = fmaf(px, s.dx, fmaf(py, s.dy, pz * s.dz));
+// The sweep's update for one vertex (d = -inf leaves the state as it is).
+// Selects, not a branch: the update costs less than the jump round it.
+OGJK_DEV void sweep32_take(Sweep32& s, float px, float py, float pz, float d, int i) {
   s.second = fmaxf(s.second, fminf(s.best, d));
-  if (d > s.best) {
-    s.best = d;
-    s.bi = i;
-    s.bx = px;
-    s.by = py;
-    s.bz = pz;
+  const bool better = d > s.best;
+  s.best = better ? d : s.best;
+  s.bi = better ? i : s.bi;
+  s.bx = better ? px : s.bx;
+  s.by = better ? py : s.by;
+  s.bz = better ? pz : s.bz;
+}
+
+// One lane's share of the FP32 sweep: vertices lane, lane + LPP, ...  Four of
+// them are loaded at a time: with one per trip the loop waits out a memory
+// round trip for every LPP vertices, and a sweep is little else.
+template <int LPP, int STRIDE>
+OGJK_DEV void sweep32(const Body<float, STRIDE>& b, int lane, Sweep32& s) {
+  constexpr int U = 4;
+  int base = 0;
+#pragma clang loop unroll(disable)
+  for (; base + LPP < b.n; base += U * LPP) {
+    float px[U], py[U], pz[U];
+#pragma unroll
+    for (int k = 0; k < U; k++) {
+      const int i = min(base + k * LPP + lane, b.n - 1);
+      px[k] = b.rx(i);
+      py[k] = b.ry(i);
+      pz[k] = b.rz(i);
+    }
+#pragma unroll
+    for (int k = 0; k < U; k++) {
+      const int i = base + k * LPP + lane;
+      const float d = fmaf(px[k], s.dx, fmaf(py[k], s.dy, pz[k] * s.dz));
+      sweep32_take(s, px[k], py[k], pz[k], i < b.n ? d : -INFINITY, i);
+    }
+  }
+  if (base + lane < b.n) {
+    const int i = base + lane;
+    const float px = b.rx(i), py = b.ry(i), pz = b.rz(i);
+    sweep32_take(s, px, py, pz, fmaf(px, s.dx, fmaf(py, s.dy, pz * s.dz)), i);
   }
 }
 
@@ -183,16 +212,43 @@ OGJK_DEV Sup finish1(Cand c, const Query& q) {
   return Sup{c.i, D3{shfl_d<LPP>(c.p.x, src), shfl_d<LPP>(c.p.y, src), shfl_d<LPP>(c.p.z, src)}};
 }
 
-// Support point of one body (FP32 sweep, FP64 re-rank of the window).
+// The support point of a float body with its coordinates as stored (they are
+// exact in FP32, so a group exchanges half the words).
+struct SupF {
+  int i;
+  float x, y, z;
+};
+OGJK_DEV Sup widen(const SupF& s) { return Sup{s.i, D3{(double)s.x, (double)s.y, (double)s.z}}; }
+
+// Support point of one body (FP32 sweep, FP64 re-rank of the window).  Nearly
+// always a single vertex lies in the window: its lane is known from one
+// ballot, its index and FP32 point are fetched, and every lane evaluates the
+// acceptance rule's FP64 product itself.
 template <int LPP, int STRIDE>
-OGJK_DEV Sup support(const Body<float, STRIDE>& A, const Query& q, int lane) {
+OGJK_DEV SupF support_f(const Body<float, STRIDE>& A, const Query& q, int lane) {
   Sweep32 sw = sweep32_begin(q.dir);
-  for (int i = lane; i < A.n; i += LPP) sweep32_step(A, i, sw);
+  sweep32<LPP>(A, lane, sw);
   const float m = group_max_f<LPP>(sw.best);
   // |D32 - scale*D64| <= 16u * r1 (u = 2^-24): candidates lie within 2x that.
   const float t = m - 0x1.0p-19f * A.r1;
   const bool multi = group_any<LPP>(sw.second >= t);
-  return finish1<LPP>(candidates32<LPP>(A, sw, t, multi, q.dir, lane), q);
+  const auto holders = lanes_where<LPP>(sw.bi >= 0 && sw.best >= t);
+  if (!multi && count_lanes<LPP>(holders) == 1) {
+    const int src = first_lane<LPP>(holders);
+    const SupF r{shfl_i<LPP>(sw.bi, src), shfl_f<LPP>(sw.bx, src), shfl_f<LPP>(sw.by, src),
+                 shfl_f<LPP>(sw.bz, src)};
+    const double v = dot(D3{(double)r.x, (double)r.y, (double)r.z}, q.dir);
+    if (q.has_inc && !(v > dot(q.inc_pt, q.dir)))
+      return SupF{q.inc_idx, (float)q.inc_pt.x, (float)q.inc_pt.y, (float)q.inc_pt.z};
+    if (!q.has_inc && !(v > -1e10)) return SupF{-1, 0.0f, 0.0f, 0.0f};
+    return r;
+  }
+  const Sup r = finish1<LPP>(candidates32<LPP>(A, sw, t, multi, q.dir, lane), q);
+  return SupF{r.i, (float)r.p.x, (float)r.p.y, (float)r.p.z};
+}
+template <int LPP, int STRIDE>
+OGJK_DEV Sup support(const Body<float, STRIDE>& A, const Query& q, int lane) {
+  return widen(support_f<LPP>(A, q, lane));
 }
 
 // ------------------------------------------------ clustered support sweep
@@ -423,50 +479,107 @@ OGJK_DEV Sup support_clustered(const CBody& A, const Query& q, int lane) {
   return finish1<LPP, false>(c, q);
 }
 
-// Calls f(k) for every slot of the clusters base + b for the set bits b of
-// m (a group ballot), each slot on exactly one lane.
-template <int LPP, class F>
-OGJK_DEV void visit_mask(const CBody& A, int base, uint64_t m, int lane, F&& f) {
-  while (m != 0) {
-    if constexpr (LPP >= kCluster) {
-      constexpr int PER = LPP / kCluster;
-      int cid = -1;
+// Whole-wave form.  A query is a chain of dependent memory round trips, and a
+// wave has little else to do meanwhile, so what can be in flight together is:
+// bounds stay in registers from the pass that finds the best cluster, the two
+// best clusters are swept at once (one per half of the wave: the threshold is
+// then the larger maximum of two, and there are fewer others to visit), and the
+// clusters that reach the threshold are swept kBatch pairs at a time.
+
+constexpr int kBatch = 4;
+
+// Calls f(k, x, y, z, in range) for the slots k of the clusters that the lanes
+// with `live` name, kCluster lanes to a cluster and kBatch pairs of clusters in
+// flight.  One permute packs the names into the lowest lanes; taking them from
+// the ballot bit by bit made the scalar unit the slowest part of a query.
+template <class F>
+OGJK_DEV void visit_live(bool live, int c, int n, const float* sx, const float* sy,
+                         const float* sz, int lane, F&& f) {
+  const uint64_t m = __ballot(live);
+  const int cnt = (int)__popcll(m);
+  if (cnt == 0) return;
+  const int below = lanes_below<64>(m, lane);
+  const int list = __builtin_amdgcn_ds_permute((live ? below : cnt + lane - below) << 2, c);
+  const int half = lane >> 5, in = lane & (kCluster - 1);
+  for (int at = 0; at < cnt; at += 2 * kBatch) {
+    int k[kBatch];
+    float px[kBatch], py[kBatch], pz[kBatch];
 #pragma unroll
-      for (int j = 0; j < PER; j++) {
-        if (m != 0) {
-          if (j == lane / kCluster) cid = (int)__builtin_ctzll(m);
-          m &= m - 1;
-        }
-      }
-      if (cid >= 0) {
-        const int k = (base + cid) * kCluster + (lane & (kCluster - 1));
-        if (k < A.n) f(k);
-      }
-    } else {
-      const int cid = (int)__builtin_ctzll(m);
-      m &= m - 1;
+    for (int u = 0; u < kBatch; u++) {
+      const int e = at + 2 * u + half;
+      const int slot = __builtin_amdgcn_ds_bpermute(e << 2, list) * kCluster + in;
+      k[u] = e < cnt && slot < n ? slot : -1;
+    }
 #pragma unroll
-      for (int t = lane; t < kCluster; t += LPP) {
-        const int k = (base + cid) * kCluster + t;
-        if (k < A.n) f(k);
+    for (int u = 0; u < kBatch; u++) {
+      if (at + 2 * u < cnt) {
+        const int slot = max(k[u], 0);
+        px[u] = sx[slot];
+        py[u] = sy[slot];
+        pz[u] = sz[slot];
       }
     }
+#pragma unroll
+    for (int u = 0; u < kBatch; u++)
+      if (at + 2 * u < cnt) f(k[u], px[u], py[u], pz[u], k[u] >= 0);
   }
 }
 
-// One-level clustered query, for scenes without superclusters (the cluster
-// build gives superclusters to every body of more than kSuperMinClusters
-// clusters, so here a body has at most that many: K per lane).  Same
-// selection as support_clustered<LPP, false>, with fewer dependent memory
-// round trips: each lane keeps the bounds of its clusters in registers from
-// the first pass (the survivor test reads no bounds again), the best
-// cluster's sweep is the first step of the window sweep (it is not swept
-// twice), and each lane's input index is fetched before the final
-// reductions instead of after them.
-template <int LPP>
-OGJK_DEV Sup support_clustered1(const CBody& A, const Query& q, int lane) {
-  if (A.slot < 0) return support<LPP>(static_cast<const Body<float, 1>&>(A), q, lane);
-  constexpr int K = (kSuperMinClusters + LPP - 1) / LPP;
+// The entry with the largest of the lanes' values (the lowest lane's on ties),
+// with its value.
+OGJK_DEV int wave_best(float v, int i, float& top) {
+  top = group_max_f<64>(v);
+  return __builtin_amdgcn_readfirstlane(
+      shfl_i<64>(i, (int)__builtin_ctzll(__ballot(v == top) | (1ull << 63))));
+}
+
+// The two entries with the largest bounds of b[0, n): ub[j] keeps the bound of
+// entry lane + 64 j, later entries are bounded again.  second < 0: none.
+OGJK_DEV void two_best(const ClusterBound* b, int n, float dx, float dy, float dz, float dn,
+                       int lane, float (&ub)[2], int& first, int& second) {
+  float v = -INFINITY;
+  int i = 0;
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    const int c = lane + 64 * j;
+    ub[j] = c < n ? cluster_ub(b[c], dx, dy, dz, dn) : -INFINITY;
+    if (ub[j] > v) {
+      v = ub[j];
+      i = c;
+    }
+  }
+  for (int c = lane + 128; c < n; c += 64) {
+    const float u = cluster_ub(b[c], dx, dy, dz, dn);
+    if (u > v) {
+      v = u;
+      i = c;
+    }
+  }
+  float top;
+  first = wave_best(v, i, top);
+  v = -INFINITY;
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    const int c = lane + 64 * j;
+    if (c != first && ub[j] > v) {
+      v = ub[j];
+      i = c;
+    }
+  }
+  for (int c = lane + 128; c < n; c += 64) {
+    const float u = c != first ? cluster_ub(b[c], dx, dy, dz, dn) : -INFINITY;
+    if (u > v) {
+      v = u;
+      i = c;
+    }
+  }
+  second = wave_best(v, i, top);
+  if (!(top > -INFINITY)) second = -1;
+}
+
+template <bool TWO>
+OGJK_DEV Sup support_clustered64(const CBody& A, const Query& q, int lane) {
+  if (A.slot < 0) return support<64>(static_cast<const Body<float, 1>&>(A), q, lane);
   Sweep32 sw = sweep32_begin(q.dir);
   const float dx = sw.dx, dy = sw.dy, dz = sw.dz;
   const float dn = sqrtf(fmaf(dx, dx, fmaf(dy, dy, dz * dz))) * (1.0f + 0x1.0p-20f);
@@ -475,110 +588,108 @@ OGJK_DEV Sup support_clustered1(const CBody& A, const Query& q, int lane) {
   const float* sx = A.cv.x + A.slot;
   const float* sy = A.cv.y + A.slot;
   const float* sz = A.cv.z + A.slot;
+  const ClusterBound* sb = nullptr;
+  if constexpr (TWO) {
+    const int sup = first_super(cb);
+    if (sup >= 0) sb = A.cv.sbounds + sup;
+  }
+  // the build gives superclusters to every body of more clusters than this
+  if (sb == nullptr && nc > kSuperMinClusters)
+    return support_clustered<64, false>(A, q, lane);
 
-  // 1: every cluster's bound; the largest (lowest cluster on ties) is swept
-  // first.  Bounds past K per lane are recomputed in step 3.
-  float ub[K];
-  float bub = -INFINITY;
-  int bi = 0;
-#pragma unroll
-  for (int j = 0; j < K; j++) {
-    const int c = lane + j * LPP;
-    ub[j] = c < nc ? cluster_ub(cb[c], dx, dy, dz, dn) : -INFINITY;
-    if (ub[j] > bub) {
-      bub = ub[j];
-      bi = c;
-    }
-  }
-  for (int c = lane + K * LPP; c < nc; c += LPP) {
-    const float u = cluster_ub(cb[c], dx, dy, dz, dn);
-    if (u > bub) {
-      bub = u;
-      bi = c;
-    }
-  }
-  const float gub = group_max_f<LPP>(bub);
-  const int bc = shfl_i<LPP>(bi, (int)__builtin_ctzll(group_ballot<LPP>(bub == gub) | (1ull << 63)));
-  // A group of two clusters' width sweeps the cluster with the second largest
-  // bound in step 2 as well, on its upper half (idle otherwise): the threshold
-  // is then the maximum over both clusters (it can only rise), and step 3 has
-  // one cluster fewer to visit.
-  constexpr bool kPair = LPP == 2 * kCluster;
-  int bc2 = -1;
-  if constexpr (kPair) {
-    float sub = -INFINITY;
-    int si = 0;
-#pragma unroll
-    for (int j = 0; j < K; j++) {
-      const int c = lane + j * LPP;
-      if (c != bc && ub[j] > sub) {
-        sub = ub[j];
-        si = c;
-      }
-    }
-    for (int c = lane + K * LPP; c < nc; c += LPP) {
-      const float u = c != bc ? cluster_ub(cb[c], dx, dy, dz, dn) : -INFINITY;
-      if (u > sub) {
-        sub = u;
-        si = c;
-      }
-    }
-    const float g2 = group_max_f<LPP>(sub);
-    if (g2 > -INFINITY)
-      bc2 = shfl_i<LPP>(si, (int)__builtin_ctzll(group_ballot<LPP>(sub == g2) | (1ull << 63)));
-  }
-  // the slot of cluster bc (lower half) or bc2 (upper half) this lane sweeps
-  const int k2 = kPair ? ((lane < kCluster ? bc : bc2) * kCluster + (lane & (kCluster - 1))) : -1;
-  const bool has2 = kPair && (lane < kCluster || bc2 >= 0) && k2 < A.n;
-
-  auto sweep = [&](int k) {
-    const float px = sx[k], py = sy[k], pz = sz[k];
-    const float d = fmaf(px, dx, fmaf(py, dy, pz * dz));
-    sw.second = fmaxf(sw.second, fminf(sw.best, d));
-    if (d > sw.best) {
-      sw.best = d;
-      sw.bi = k;
-      sw.bx = px;
-      sw.by = py;
-      sw.bz = pz;
-    }
-  };
-  // 2: the best cluster (and the second, see above): the FP32 maximum m0 of
-  // what was swept gives the threshold L
-  if constexpr (kPair) {
-    if (has2) sweep(k2);
+  // 1: the two clusters with the largest bounds (of all, or of the two
+  // superclusters with the largest)
+  float ub[2], sub[2];
+  int bc, bc2;
+  const int half = lane >> 5, in = lane & (kCluster - 1);
+  const int ns = (nc + kSuper - 1) / kSuper;
+  if (!TWO || sb == nullptr) {
+    two_best(cb, nc, dx, dy, dz, dn, lane, ub, bc, bc2);
   } else {
-#pragma unroll
-    for (int t = lane; t < kCluster; t += LPP) {
-      const int k = bc * kCluster + t;
-      if (k < A.n) sweep(k);
-    }
+    int s1, s2;
+    two_best(sb, ns, dx, dy, dz, dn, lane, sub, s1, s2);
+    const int s = half ? s2 : s1;
+    const int c = s * kSuper + in;
+    const float v = s >= 0 && c < nc ? cluster_ub(cb[c], dx, dy, dz, dn) : -INFINITY;
+    float top;
+    bc = wave_best(v, c, top);
+    bc2 = wave_best(c == bc ? -INFINITY : v, c, top);
+    if (!(top > -INFINITY)) bc2 = -1;
   }
-  const float L = group_max_f<LPP>(sw.best) - 0x1.0p-15f * A.r1;
+
+  auto sweep = [&](int k, float px, float py, float pz, bool ok) {
+    const float d = fmaf(px, dx, fmaf(py, dy, pz * dz));
+    sweep32_take(sw, px, py, pz, ok ? d : -INFINITY, k);
+  };
+  // 2: sweep both; the FP32 maximum of what was swept gives the threshold L
+  {
+    const int c = half ? bc2 : bc;
+    const int k = c * kCluster + in;
+    const bool ok = c >= 0 && k < A.n;
+    const int at = ok ? k : 0;
+    sweep(k, sx[at], sy[at], sz[at], ok);
+  }
+  const float L = group_max_f<64>(sw.best) - 0x1.0p-15f * A.r1;
 
   // 3: the other clusters whose bound reaches L (the visit order does not
   // change the selection: ties are broken by input index below)
-  auto others = [&](auto&& f) {
+  if (!TWO || sb == nullptr) {
 #pragma unroll
-    for (int j = 0; j < K; j++) {
-      const int c = lane + j * LPP;
-      visit_mask<LPP>(A, j * LPP,
-                      group_ballot<LPP>(c < nc && c != bc && c != bc2 && !(ub[j] < L)), lane, f);
+    for (int j = 0; j < 2; j++) {
+      const int c = lane + 64 * j;
+      visit_live(c < nc && c != bc && c != bc2 && !(ub[j] < L), c, A.n, sx, sy, sz, lane, sweep);
     }
-    for (int base = K * LPP; base < nc; base += LPP) {
-      const int c = base + lane;
-      const bool live =
-          c < nc && c != bc && c != bc2 && !(cluster_ub(cb[c], dx, dy, dz, dn) < L);
-      visit_mask<LPP>(A, base, group_ballot<LPP>(live), lane, f);
+  } else {
+    for (int base = 0; base < ns; base += 64) {
+      const int s = base + lane;
+      float u = base == 0 ? sub[0] : sub[1];
+      if (base >= 128 && s < ns) u = cluster_ub(sb[s], dx, dy, dz, dn);
+      uint64_t live = __ballot(s < ns && !(u < L));
+      while (live != 0) {
+        // the clusters of up to 2 kBatch superclusters, one per half and step
+        int c[kBatch];
+        ClusterBound b[kBatch];
+#pragma unroll
+        for (int j = 0; j < kBatch; j++) {
+          c[j] = -1;
+          if (live != 0) {
+            int s0 = base + (int)__builtin_ctzll(live), s1 = -1;
+            live &= live - 1;
+            if (live != 0) {
+              s1 = base + (int)__builtin_ctzll(live);
+              live &= live - 1;
+            }
+            const int mine = half ? s1 : s0;
+            c[j] = mine >= 0 && mine * kSuper + in < nc ? mine * kSuper + in : -1;
+            b[j] = cb[max(c[j], 0)];
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < kBatch; j++) {
+          if (__ballot(c[j] >= 0) != 0)
+            visit_live(c[j] >= 0 && c[j] != bc && c[j] != bc2 &&
+                           !(cluster_ub(b[j], dx, dy, dz, dn) < L),
+                       c[j], A.n, sx, sy, sz, lane, sweep);
+        }
+      }
     }
-  };
-  others(sweep);
+  }
 
   const int32_t* orig = A.cv.orig + A.slot;
   const int oi = sw.bi >= 0 ? orig[sw.bi] : 0x7fffffff;
-  const float M = group_max_f<LPP>(sw.best);
+  const float M = group_max_f<64>(sw.best);
   const float T = M - 0x1.0p-19f * A.r1;
-  const bool multi = group_any<LPP>(sw.second >= T);
+  const bool multi = group_any<64>(sw.second >= T);
+  const uint64_t holders = __ballot(sw.bi >= 0 && sw.best >= T);
+  if (!multi && __popcll(holders) == 1) {  // as in support_f
+    const int src = (int)__builtin_ctzll(holders);
+    const Sup r = widen(SupF{shfl_i<64>(oi, src), shfl_f<64>(sw.bx, src), shfl_f<64>(sw.by, src),
+                             shfl_f<64>(sw.bz, src)});
+    const double v = dot(r.p, q.dir);
+    if (q.has_inc && !(v > dot(q.inc_pt, q.dir))) return Sup{q.inc_idx, q.inc_pt};
+    if (!q.has_inc && !(v > -1e10)) return Sup{-1, D3{0.0, 0.0, 0.0}};
+    return r;
+  }
 
   // FP64 re-rank of the window; ties go to the lowest input index
   Cand c{-INFINITY, 0x7fffffff, D3{0.0, 0.0, 0.0}};
@@ -589,7 +700,8 @@ OGJK_DEV Sup support_clustered1(const CBody& A, const Query& q, int lane) {
       c.i = oi;
     }
   } else {
-    auto rank = [&](int k) {
+    // every cluster that may hold a vertex of the window reaches L
+    visit_clusters<64, TWO>(A, cb, nc, sb, dx, dy, dz, dn, L, lane, [&](int k) {
       const float px = sx[k], py = sy[k], pz = sz[k];
       const float d = fmaf(px, dx, fmaf(py, dy, pz * dz));
       if (d >= T) {
@@ -602,36 +714,30 @@ OGJK_DEV Sup support_clustered1(const CBody& A, const Query& q, int lane) {
           c.p = p;
         }
       }
-    };
-    if constexpr (kPair) {
-      if (has2) rank(k2);
-    } else {
-#pragma unroll
-      for (int t = lane; t < kCluster; t += LPP) {
-        const int k = bc * kCluster + t;
-        if (k < A.n) rank(k);
-      }
-    }
-    others(rank);
+    });
   }
   if (!(c.v == c.v)) c.v = -INFINITY;
-  return finish1<LPP, false>(c, q);
+  return finish1<64, false>(c, q);
 }
 
-// The one-level query with cached bounds for whole-wave groups; narrower
-// groups would keep 128 / LPP bounds per lane, which costs the small-hull
-// kernels of the same scene more in spills than it saves.
+// Whole-wave groups take the form above; narrower groups would keep 128 / LPP
+// bounds per lane, which costs the small-hull kernels of the same scene more
+// in spills than it saves.
 template <int LPP>
 OGJK_DEV Sup support(const CBody& A, const Query& q, int lane) {
   if constexpr (LPP >= 64) {
-    return support_clustered1<LPP>(A, q, lane);
+    return support_clustered64<false>(A, q, lane);
   } else {
     return support_clustered<LPP, false>(A, q, lane);
   }
 }
 template <int LPP>
 OGJK_DEV Sup support(const CBody2& A, const Query& q, int lane) {
-  return support_clustered<LPP, true>(A, q, lane);
+  if constexpr (LPP >= 64) {
+    return support_clustered64<true>(A, q, lane);
+  } else {
+    return support_clustered<LPP, true>(A, q, lane);
+  }
 }
 
 // ------------------------------------------------------------ posed bodies
@@ -691,11 +797,21 @@ template <int LPP>
 OGJK_DEV Sup support(const PBody& A, const Query& q, int lane) {
   const Pose P = Pose::load(A.pose);
   Sweep32 sw = sweep32_begin(P.to_local(q.dir));
-  for (int i = lane; i < A.n; i += LPP) sweep32_step(A, i, sw);
+  sweep32<LPP>(static_cast<const Body<float, 1>&>(A), lane, sw);
   const float m = group_max_f<LPP>(sw.best);
   const float t1 = (float)(fabs(P.t[0]) + fabs(P.t[1]) + fabs(P.t[2]));
   const float T = m - (0x1.0p-19f * A.r1 + 0x1.0p-45f * (A.r1 + t1));
   const bool multi = group_any<LPP>(sw.second >= T);
+  const auto holders = lanes_where<LPP>(sw.bi >= 0 && sw.best >= T);
+  if (!multi && count_lanes<LPP>(holders) == 1) {  // as in support_f
+    const int src = first_lane<LPP>(holders);
+    const Sup r{shfl_i<LPP>(sw.bi, src), P.world(shfl_f<LPP>(sw.bx, src), shfl_f<LPP>(sw.by, src),
+                                                 shfl_f<LPP>(sw.bz, src))};
+    const double v = dot(r.p, q.dir);
+    if (q.has_inc && !(v > dot(q.inc_pt, q.dir))) return Sup{q.inc_idx, q.inc_pt};
+    if (!q.has_inc && !(v > -1e10)) return Sup{-1, D3{0.0, 0.0, 0.0}};
+    return r;
+  }
   Cand c{-INFINITY, 0x7fffffff, D3{0.0, 0.0, 0.0}};
   if (!multi) {
     if (sw.bi >= 0 && sw.best >= T) {
@@ -745,15 +861,19 @@ OGJK_DEV Query pick(bool c, const Query& a, const Query& b) {
                sel(c, a.inc_pt, b.inc_pt)};
 }
 
-// The support points of both bodies, one query after the other through one
-// copy of the sweep code (two sweeps in one loop keep two sweep states live;
-// two inlined copies double the code the register allocator sees).
 template <int LPP>
-OGJK_DEV Sup swap_halves(const Sup& r) {
-  Sup o;
-  o.i = xchg<LPP / 2>(r.i);
-  o.p = D3{xchg<LPP / 2>(r.p.x), xchg<LPP / 2>(r.p.y), xchg<LPP / 2>(r.p.z)};
-  return o;
+OGJK_DEV void both_halves(const Sup& r, Sup& lo, Sup& hi) {
+  both_halves<LPP>(r.i, lo.i, hi.i);
+  both_halves<LPP>(r.p.x, lo.p.x, hi.p.x);
+  both_halves<LPP>(r.p.y, lo.p.y, hi.p.y);
+  both_halves<LPP>(r.p.z, lo.p.z, hi.p.z);
+}
+template <int LPP>
+OGJK_DEV void both_halves(const SupF& r, SupF& lo, SupF& hi) {
+  both_halves<LPP>(r.i, lo.i, hi.i);
+  both_halves<LPP>(r.x, lo.x, hi.x);
+  both_halves<LPP>(r.y, lo.y, hi.y);
+  both_halves<LPP>(r.z, lo.z, hi.z);
 }
 
 // Split the group between the two queries for bodies swept whole (small
@@ -776,14 +896,21 @@ OGJK_DEV void support_pair(const BT& A, const Query& qa, const BT& B, const Quer
     // the lower half of the group answers A's query, the upper half B's, at
     // the same time; then each half takes the other's result
     const bool hi = lane >= LPP / 2;
-    const Sup r = support<LPP / 2>(pick(hi, B, A), pick(hi, qb, qa), lane & (LPP / 2 - 1));
-    // each half's result is uniform over the half, so any lane of the other
-    // half (the exchange partner) holds it
-    const Sup o = swap_halves<LPP>(r);
-    ra = Sup{hi ? o.i : r.i, sel(hi, o.p, r.p)};
-    rb = Sup{hi ? r.i : o.i, sel(hi, r.p, o.p)};
+    const BT& body = pick(hi, B, A);
+    const Query& q = pick(hi, qb, qa);
+    if constexpr (std::is_same_v<BT, PBody>) {
+      both_halves<LPP>(support<LPP / 2>(body, q, lane & (LPP / 2 - 1)), ra, rb);
+    } else {
+      SupF fa, fb;
+      both_halves<LPP>(support_f<LPP / 2>(body, q, lane & (LPP / 2 - 1)), fa, fb);
+      ra = widen(fa);
+      rb = widen(fb);
+    }
     return;
   }
+  // one query after the other through one copy of the sweep code (two sweeps
+  // in one loop keep two sweep states live; two inlined copies double the code
+  // the register allocator sees)
 #pragma clang loop unroll(disable)
   for (int w = 0; w < 2; w++) {
     const bool second = w != 0;

@@ -1,7 +1,7 @@
 // opengjk-amd device EPA for one pair on a group of LPP lanes (LPP <= 64).
 //
-// Layout: the polytope's vertex pool (<= 132 FP64 points and their body
-// indices), the horizon edge lists and the input witnesses live in LDS; the
+// Layout: the polytope's vertex pool (<= 68 FP64 points and their body
+// indices), the edge tables and the input witnesses live in LDS; the
 // 128 face slots are spread over the group's lanes, slot = q*LPP + lane,
 // FPL = 128/LPP faces per lane held in registers (normal, plane distance,
 // packed vertex ids).  Nothing else of the pair stays in registers through
@@ -13,7 +13,8 @@
 //   * closest face: min distance, lowest slot on ties (EPA.c:608-617);
 //   * horizon: edges of the faces removed this iteration, in slot order and
 //     (v0v1, v1v2, v2v0) order; an edge that occurs more than once is dropped
-//     (the pairwise cancellation of EPA.c:746-759 drops every occurrence);
+//     (the pairwise cancellation of EPA.c:746-759 drops every occurrence), found
+//     by two bit tables over the vertex pairs: met, and met again;
 //   * new faces take the lowest free slots in horizon order (EPA.c:762-775);
 //   * a face's normal is computed when it is created and a degenerate face is
 //     retired at the start of the next iteration, which is when the reference
@@ -25,16 +26,20 @@
 namespace ogjk {
 
 constexpr int kEpaMaxFaces = 128;
-constexpr int kEpaMaxVerts = kEpaMaxFaces + 4;
+constexpr int kEpaMaxIter = 64;
+// the tetrahedron and one vertex per iteration (below the reference's cap of
+// 132, EPA.c:44, which therefore never ends the loop)
+constexpr int kEpaMaxVerts = 4 + kEpaMaxIter;
+constexpr int kEdgeWords = (kEpaMaxVerts + 31) / 32;  // bits of one vertex's row
 
 struct EpaShared {
   double vx[kEpaMaxVerts], vy[kEpaMaxVerts], vz[kEpaMaxVerts];
   int via[kEpaMaxVerts], vib[kEpaMaxVerts];
-  // edges of the faces removed this iteration: directed edge v1 | v2 << 8 in
-  // the low half, its direction-free key in the high half
-  unsigned edir[kEpaMaxFaces * 3];
-  unsigned short surv[kEpaMaxFaces * 3];  // surviving horizon edges, in order
-  double w_in[6];                         // the witnesses EPA started from
+  // edges (a < b) of the faces removed this iteration, bit b of row a: those
+  // met, and those met more than once.  All zero between iterations.
+  unsigned met[kEpaMaxVerts * kEdgeWords], again[kEpaMaxVerts * kEdgeWords];
+  unsigned short surv[kEpaMaxFaces];  // surviving horizon edges, in order
+  double w_in[6];                     // the witnesses EPA started from
 };
 
 OGJK_DEV void wave_sync() {
@@ -42,11 +47,23 @@ OGJK_DEV void wave_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// Directed edge (a, b) packed as a | b << 8, with its direction-free key
-// (min | max << 8) in the high 16 bits.
-OGJK_DEV unsigned edge_word(int a, int b) {
-  const unsigned lo = a < b ? (unsigned)(a | (b << 8)) : (unsigned)(b | (a << 8));
-  return (unsigned)(a | (b << 8)) | (lo << 16);
+// Clears the edge tables: once before a group's first pair (epa() leaves them
+// clear).
+template <int LPP>
+OGJK_DEV void epa_shared_begin(EpaShared& sh, int lane) {
+  for (int i = lane; i < kEpaMaxVerts * kEdgeWords; i += LPP) sh.met[i] = sh.again[i] = 0u;
+  wave_sync();
+}
+
+// Place of the edge (a, b) in the edge tables.
+OGJK_DEV void edge_place(int a, int b, int& word, unsigned& bit) {
+  const int lo = min(a, b), hi = max(a, b);
+  word = lo * kEdgeWords + (hi >> 5);
+  bit = 1u << (hi & 31);
+}
+
+OGJK_DEV unsigned lds_or(unsigned* p, unsigned bits) {
+  return __hip_atomic_fetch_or(p, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
 }
 
 OGJK_DEV D3 lds_v(const EpaShared& sh, int i) { return D3{sh.vx[i], sh.vy[i], sh.vz[i]}; }
@@ -158,112 +175,206 @@ OGJK_DEV void put_face(Faces<FPL>& F, int q, const NewFace& f) {
   if (!f.ok) F.pend |= 1u << q;
 }
 
-// Exclusive rank of set flags in slot order (slot = q*LPP + lane).
+// Closest valid face with distance in [0, 1e10), lowest slot on ties: the
+// group's least distance, then the first slot that has it.  `many`: slots past
+// the first LPP are in use.
 template <int LPP, int FPL>
-OGJK_DEV int slot_rank(const bool (&flag)[FPL], int (&rank)[FPL]) {
-  int base = 0;
+OGJK_DEV int closest_face(const Faces<FPL>& F, bool many, double& cdist) {
+  double d[FPL];
+  double m = INFINITY;
 #pragma unroll
   for (int q = 0; q < FPL; q++) {
-    const uint64_t gb = group_ballot<LPP>(flag[q]);
-    rank[q] = base + group_prefix<LPP>(gb);
-    base += __popcll(gb);
-  }
-  return base;
-}
-
-// Closest valid face with distance in [0, 1e10), lowest slot on ties.
-template <int LPP, int FPL>
-OGJK_DEV int closest_face(const Faces<FPL>& F, int lane, double& cdist) {
-  double bv = INFINITY;
-  int bi = 0x7fffffff;
-#pragma unroll
-  for (int q = 0; q < FPL; q++) {
-    const double d = F.dist[q];
-    const bool ok = ((F.valid >> q) & 1u) && d >= 0.0 && d < 1e10;
-    if (ok && d < bv) {
-      bv = d;
-      bi = q * LPP + lane;
+    d[q] = INFINITY;
+    if (q == 0 || many) {
+      const double fd = F.dist[q];
+      if (((F.valid >> q) & 1u) && fd >= 0.0 && fd < 1e10) d[q] = fd;
+      m = d[q] < m ? d[q] : m;
     }
   }
-  group_argmin_d<LPP>(bv, bi);
-  cdist = bv;
-  return bi == 0x7fffffff ? -1 : bi;
+  m = group_min_d<LPP>(m);
+  cdist = m;
+  if (!(m < INFINITY)) return -1;
+  int slot = -1;
+#pragma unroll
+  for (int q = 0; q < FPL; q++) {
+    if (q == 0 || many) {
+      const auto has = lanes_where<LPP>(d[q] == m);
+      if (slot < 0 && has != 0) slot = q * LPP + first_lane<LPP>(has);
+    }
+  }
+  return slot;
 }
 
+// Normal, distance and vertices of the face in `slot`, on every lane.
 template <int LPP, int FPL>
-OGJK_DEV void fetch_face(const Faces<FPL>& F, int slot, D3& n, int& verts) {
+OGJK_DEV void fetch_face(const Faces<FPL>& F, int slot, bool many, D3& n, double& dist,
+                         int& verts) {
   const int q = slot / LPP, src = slot % LPP;
   // value selects over laundered registers (see keep_reg): no address select
   double x = keep_reg(F.nx[0]), y = keep_reg(F.ny[0]), z = keep_reg(F.nz[0]);
   int vv = keep_reg(F.verts[0]);
+  if (many) {
 #pragma unroll
-  for (int t = 1; t < FPL; t++) {
-    const bool h = (q == t);
-    x = h ? keep_reg(F.nx[t]) : x;
-    y = h ? keep_reg(F.ny[t]) : y;
-    z = h ? keep_reg(F.nz[t]) : z;
-    vv = h ? keep_reg(F.verts[t]) : vv;
+    for (int t = 1; t < FPL; t++) {
+      const bool h = (q == t);
+      x = h ? keep_reg(F.nx[t]) : x;
+      y = h ? keep_reg(F.ny[t]) : y;
+      z = h ? keep_reg(F.nz[t]) : z;
+      vv = h ? keep_reg(F.verts[t]) : vv;
+    }
   }
   n = D3{shfl_d<LPP>(x, src), shfl_d<LPP>(y, src), shfl_d<LPP>(z, src)};
   verts = shfl_i<LPP>(vv, src);
+  if (dist == 0.0) {  // a tie of zeros of either sign: the chosen face's own
+    double own = keep_reg(F.dist[0]);
+#pragma unroll
+    for (int t = 1; t < FPL; t++) own = (q == t) ? keep_reg(F.dist[t]) : own;
+    dist = shfl_d<LPP>(own, src);
+  }
 }
+
+// The two bodies as EPA holds them through its loop.  Where the group splits
+// into halves (see kSplit), a lane keeps its own half's body only (the lower
+// half A, the upper half B), half the registers, and each half works on its
+// body: the queries, and the blend of the witnesses, which the halves then
+// exchange.  Otherwise every lane keeps both.
+template <int LPP, class BT, bool SPLIT = LPP >= 16 && kSplit<LPP, BT>>
+struct PairView {
+  BT A, B;
+  OGJK_DEV PairView(const BT& a, const BT& b, int) : A(a), B(b) {}
+  OGJK_DEV void query(D3 dir, int lane, Sup& a, Sup& b) const {
+    const D3 zero{0.0, 0.0, 0.0};
+    support_pair<LPP>(A, Query{dir, false, 0, zero}, B, Query{neg(dir), false, 0, zero}, lane, a,
+                      b);
+    // The reference leaves its output unset when no vertex beats -1e10; such
+    // coordinates are out of any physical range, fall back to vertex 0.
+    if (a.i < 0) a = Sup{0, A.d(0)};
+    if (b.i < 0) b = Sup{0, B.d(0)};
+  }
+  // indices into A and B, clamped to vertex 0
+  OGJK_DEV void clamp(int& ia, int& ib) const {
+    ia = (ia >= 0 && ia < A.n) ? ia : 0;
+    ib = (ib >= 0 && ib < B.n) ? ib : 0;
+  }
+  OGJK_DEV void points(int ia, int ib, Wit& w) const {
+    w.w0 = A.d(ia);
+    w.w1 = B.d(ib);
+  }
+  OGJK_DEV void blend(const int* ia, const int* ib, const double* a, Wit& w) const {
+    w.w0 = D3{blend_c(A, ia, a, 3, 0), blend_c(A, ia, a, 3, 1), blend_c(A, ia, a, 3, 2)};
+    w.w1 = D3{blend_c(B, ib, a, 3, 0), blend_c(B, ib, a, 3, 1), blend_c(B, ib, a, 3, 2)};
+  }
+};
+
+template <int LPP, class BT>
+struct PairView<LPP, BT, true> {
+  BT own;
+  bool upper;
+  OGJK_DEV PairView(const BT& a, const BT& b, int lane)
+      : own(pick(lane >= LPP / 2, b, a)), upper(lane >= LPP / 2) {}
+  OGJK_DEV void query(D3 dir, int lane, Sup& a, Sup& b) const {
+    const Query q{sel(upper, neg(dir), dir), false, 0, D3{0.0, 0.0, 0.0}};
+    if constexpr (std::is_same_v<BT, PBody>) {
+      Sup r = support<LPP / 2>(own, q, lane & (LPP / 2 - 1));
+      if (r.i < 0) r = Sup{0, own.d(0)};
+      both_halves<LPP>(r, a, b);
+    } else {
+      SupF r = support_f<LPP / 2>(own, q, lane & (LPP / 2 - 1)), fa, fb;
+      if (r.i < 0) r = SupF{0, own.rx(0), own.ry(0), own.rz(0)};
+      both_halves<LPP>(r, fa, fb);
+      a = widen(fa);
+      b = widen(fb);
+    }
+  }
+  OGJK_DEV void clamp(int& ia, int& ib) const {
+    int na, nb;
+    both_halves<LPP>(own.n, na, nb);
+    ia = (ia >= 0 && ia < na) ? ia : 0;
+    ib = (ib >= 0 && ib < nb) ? ib : 0;
+  }
+  OGJK_DEV void exchange(D3 p, Wit& w) const {
+    both_halves<LPP>(p.x, w.w0.x, w.w1.x);
+    both_halves<LPP>(p.y, w.w0.y, w.w1.y);
+    both_halves<LPP>(p.z, w.w0.z, w.w1.z);
+  }
+  OGJK_DEV void points(int ia, int ib, Wit& w) const { exchange(own.d(upper ? ib : ia), w); }
+  OGJK_DEV void blend(const int* ia, const int* ib, const double* a, Wit& w) const {
+    const int i[3] = {upper ? ib[0] : ia[0], upper ? ib[1] : ia[1], upper ? ib[2] : ia[2]};
+    exchange(D3{blend_c(own, i, a, 3, 0), blend_c(own, i, a, 3, 1), blend_c(own, i, a, 3, 2)}, w);
+  }
+};
+
+// The plain FP64 path sweeps both bodies at once on the whole group.
+template <int LPP, int STRIDE>
+struct PairView<LPP, Body<double, STRIDE>, true> : PairView<LPP, Body<double, STRIDE>, false> {
+  using PairView<LPP, Body<double, STRIDE>, false>::PairView;
+};
 
 // support_epa (GJK/cpu/EPA.c:307-344): farthest vertex of A along dir and of
 // B along -dir; returns the Minkowski point A[ia] - B[ib].
-template <int LPP, class BT>
-OGJK_DEV D3 support_epa(const BT& A, const BT& B, D3 dir, int& ia, int& ib, int lane) {
-  const D3 zero{0.0, 0.0, 0.0};
+template <int LPP, class PV>
+OGJK_DEV D3 support_epa(const PV& V, D3 dir, int& ia, int& ib, int lane) {
   Sup a, b;
-  support_pair<LPP>(A, Query{dir, false, 0, zero}, B, Query{neg(dir), false, 0, zero}, lane, a,
-                    b);
-  // The reference leaves its output unset when no vertex beats -1e10; such
-  // coordinates are out of any physical range, fall back to vertex 0.
-  if (a.i < 0) a = Sup{0, A.d(0)};
-  if (b.i < 0) b = Sup{0, B.d(0)};
+  V.query(dir, lane, a, b);
   ia = a.i;
   ib = b.i;
   return sub(a.p, b.p);
 }
 
-// Is p farther than eps from every simplex vertex (GJK/cpu/EPA.c:453-463)?
-OGJK_DEV bool is_new_point(const Simplex& s, D3 p) {
+// Is p farther than eps from each of the first n pool vertices
+// (GJK/cpu/EPA.c:453-463, 654-684)?
+template <int LPP>
+OGJK_DEV bool is_new_point(const EpaShared& sh, int n, D3 p, int lane) {
   const double eps_sq = kEps64 * kEps64;
-  bool fresh = true;
-#pragma unroll
-  for (int t = 0; t < 4; t++) {
-    if (t < s.n) {
-      const D3 q = s.p[t];
-      const double dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-      if (dx * dx + dy * dy + dz * dz < eps_sq) fresh = false;
-    }
+  bool near = false;
+  for (int t = lane; t < n; t += LPP) {
+    const double dx = p.x - sh.vx[t], dy = p.y - sh.vy[t], dz = p.z - sh.vz[t];
+    if (dx * dx + dy * dy + dz * dz < eps_sq) near = true;
   }
-  return fresh;
+  return !group_any<LPP>(near);
 }
 
-template <class BT>
-OGJK_DEV void zero_depth(const BT& A, const BT& B, int ia, int ib,
-                         double& distance, Wit& w, D3& normal) {
+OGJK_DEV void put_vertex(EpaShared& sh, int i, D3 p, int ia, int ib) {
+  sh.vx[i] = p.x;
+  sh.vy[i] = p.y;
+  sh.vz[i] = p.z;
+  sh.via[i] = ia;
+  sh.vib[i] = ib;
+}
+
+// The simplex EPA returns: the tetrahedron it started from, pool slots 0-3.
+OGJK_DEV void simplex_back(const EpaShared& sh, Simplex& s, int n) {
+  s.n = n;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    s.p[k] = lds_v(sh, k);
+    s.ia[k] = sh.via[k];
+    s.ib[k] = sh.vib[k];
+  }
+}
+
+template <class PV>
+OGJK_DEV void zero_depth(const PV& V, int ia, int ib, double& distance, Wit& w, D3& normal) {
   distance = 0.0;
-  w.w0 = A.d(ia);
-  w.w1 = B.d(ib);
+  V.points(ia, ib, w);
   normal = contact_normal(w.w0, w.w1);
 }
 
-template <class BT>
-OGJK_DEV void face_result(const BT& A, const BT& B, const EpaShared& sh,
-                          int verts, D3 n, double cdist, double& distance, Wit& w, D3& normal) {
+template <class PV>
+OGJK_DEV void face_result(const PV& V, const EpaShared& sh, int verts, D3 n, double cdist,
+                          double& distance, Wit& w, D3& normal) {
   const int v0 = verts & 0xff, v1 = (verts >> 8) & 0xff, v2 = (verts >> 16) & 0xff;
   double a[3];
   bary_origin(lds_v(sh, v0), lds_v(sh, v1), lds_v(sh, v2), a[0], a[1], a[2]);
   const int ia[3] = {sh.via[v0], sh.via[v1], sh.via[v2]};
   const int ib[3] = {sh.vib[v0], sh.vib[v1], sh.vib[v2]};
-  w.w0 = D3{blend_c(A, ia, a, 3, 0), blend_c(A, ia, a, 3, 1), blend_c(A, ia, a, 3, 2)};
-  w.w1 = D3{blend_c(B, ib, a, 3, 0), blend_c(B, ib, a, 3, 1), blend_c(B, ib, a, 3, 2)};
+  V.blend(ia, ib, a, w);
   normal = n;
   distance = -cdist;
 }
 
-// computeCollisionInformation for one pair (GJK/cpu/EPA.c:362-864).
+// computeCollisionInformation for one pair (GJK/cpu/EPA.c:362-864).  The edge
+// tables of sh are clear before and after.
 template <int LPP, class BT>
 OGJK_DEV void epa(const BT& A, const BT& B, Simplex& s, double& distance, Wit& w, D3& normal,
                   EpaShared& sh, int lane) {
@@ -274,79 +385,11 @@ OGJK_DEV void epa(const BT& A, const BT& B, Simplex& s, double& distance, Wit& w
     normal = contact_normal(w.w0, w.w1);
     return;
   }
+  const PairView<LPP, BT> V(A, B, lane);
 
-  // -------- grow a degenerate GJK simplex to a tetrahedron (EPA.c:376-583)
-  if (s.n != 4) {
-    int ia, ib;
-    if (s.n == 1) {
-      const D3 nv = support_epa<LPP>(A, B, s.p[0], ia, ib, lane);
-      if (is_new_point(s, nv)) {
-        sset(s, 1, nv, ia, ib);
-        s.n = 2;
-      } else {
-        zero_depth(A, B, ia, ib, distance, w, normal);
-        return;
-      }
-    }
-    if (s.n == 2) {
-      const D3 edge = sub(s.p[1], s.p[0]);
-      D3 axis{1.0, 0.0, 0.0};
-      const double en = sqrt(norm2(edge));
-      if (en > kEps64 && fabs(edge.x) > (double)0.9f * en) axis = D3{0.0, 1.0, 0.0};
-      D3 dir = cross(edge, axis);
-      if (norm2(dir) < kEps64) {
-        axis = D3{0.0, 0.0, 1.0};
-        dir = cross(edge, axis);
-      }
-      const D3 nv = support_epa<LPP>(A, B, dir, ia, ib, lane);
-      if (is_new_point(s, nv)) {
-        sset(s, 2, nv, ia, ib);
-        s.n = 3;
-      } else {
-        zero_depth(A, B, ia, ib, distance, w, normal);
-        return;
-      }
-    }
-    if (s.n == 3) {
-      D3 dir = cross(sub(s.p[1], s.p[0]), sub(s.p[2], s.p[0]));
-      D3 nv = support_epa<LPP>(A, B, dir, ia, ib, lane);
-      if (is_new_point(s, nv)) {
-        sset(s, 3, nv, ia, ib);
-        s.n = 4;
-      } else {
-        dir = neg(dir);
-      }
-      if (s.n == 3) {
-        nv = support_epa<LPP>(A, B, dir, ia, ib, lane);
-        if (is_new_point(s, nv)) {
-          sset(s, 3, nv, ia, ib);
-          s.n = 4;
-        } else {
-          zero_depth(A, B, ia, ib, distance, w, normal);
-          return;
-        }
-      }
-    }
-    if (s.n != 4) {
-      int best = s.n > 0 ? s.n - 1 : 0;
-      best = best > 3 ? 3 : best;
-      int ba = sa(s, best), bb = sb(s, best);
-      ba = (ba >= 0 && ba < A.n) ? ba : 0;  // sanitise caller-provided indices
-      bb = (bb >= 0 && bb < B.n) ? bb : 0;
-      zero_depth(A, B, ba, bb, distance, w, normal);
-      return;
-    }
-  }
-
-  // -------- initial tetrahedron (init_epa_polytope, EPA.c:144-235)
-  if (lane < 4) {
-    const D3 p = sp(s, lane);
-    sh.vx[lane] = p.x;
-    sh.vy[lane] = p.y;
-    sh.vz[lane] = p.z;
-    sh.via[lane] = sa(s, lane);
-    sh.vib[lane] = sb(s, lane);
-  }
+  // the simplex and the witnesses wait in LDS: registers are what limits the
+  // waves in flight
+  if (lane < 4) put_vertex(sh, lane, sp(s, lane), sa(s, lane), sb(s, lane));
   if (lane == 0) {
     sh.w_in[0] = w.w0.x;
     sh.w_in[1] = w.w0.y;
@@ -356,12 +399,63 @@ OGJK_DEV void epa(const BT& A, const BT& B, Simplex& s, double& distance, Wit& w
     sh.w_in[5] = w.w1.z;
   }
   wave_sync();
+
+  // -------- grow a degenerate GJK simplex to a tetrahedron (EPA.c:376-583):
+  // one support query per turn, along the point, across the edge, along the
+  // triangle's normal, then against it
+  int ns = s.n;
+  bool against = false;
+  while (ns >= 1 && ns < 4) {
+    const D3 p0 = lds_v(sh, 0);
+    D3 dir;
+    if (ns == 1) {
+      dir = p0;
+    } else if (ns == 2) {
+      const D3 edge = sub(lds_v(sh, 1), p0);
+      D3 axis{1.0, 0.0, 0.0};
+      const double en = sqrt(norm2(edge));
+      if (en > kEps64 && fabs(edge.x) > (double)0.9f * en) axis = D3{0.0, 1.0, 0.0};
+      dir = cross(edge, axis);
+      if (norm2(dir) < kEps64) {
+        axis = D3{0.0, 0.0, 1.0};
+        dir = cross(edge, axis);
+      }
+    } else {
+      dir = cross(sub(lds_v(sh, 1), p0), sub(lds_v(sh, 2), p0));
+      if (against) dir = neg(dir);
+    }
+    int ia, ib;
+    const D3 nv = support_epa<LPP>(V, dir, ia, ib, lane);
+    if (is_new_point<LPP>(sh, ns, nv, lane)) {
+      if (lane == 0) put_vertex(sh, ns, nv, ia, ib);
+      wave_sync();
+      ns++;
+    } else if (ns == 3 && !against) {
+      against = true;
+    } else {
+      zero_depth(V, ia, ib, distance, w, normal);
+      simplex_back(sh, s, ns);
+      return;
+    }
+  }
+  if (ns != 4) {  // no simplex a GJK writes: caller-provided, sanitised
+    int best = ns > 0 ? ns - 1 : 0;
+    best = best > 3 ? 3 : best;
+    int ba = sh.via[best], bb = sh.vib[best];
+    V.clamp(ba, bb);
+    zero_depth(V, ba, bb, distance, w, normal);
+    simplex_back(sh, s, ns);
+    return;
+  }
+
+  // -------- initial tetrahedron (init_epa_polytope, EPA.c:144-235)
   D3 centroid{0.0, 0.0, 0.0};
 #pragma unroll
   for (int i = 0; i < 4; i++) {
-    centroid.x += s.p[i].x * 0.25;
-    centroid.y += s.p[i].y * 0.25;
-    centroid.z += s.p[i].z * 0.25;
+    const D3 p = lds_v(sh, i);
+    centroid.x += p.x * 0.25;
+    centroid.y += p.y * 0.25;
+    centroid.z += p.z * 0.25;
   }
   Faces<FPL> F;
   F.valid = 0;
@@ -383,51 +477,37 @@ OGJK_DEV void epa(const BT& A, const BT& B, Simplex& s, double& distance, Wit& w
   const double tol = kEps64 * 1e2;
   int nverts = 4;
   int iteration = 0;
-  bool wrote = false;  // w, distance and normal hold a face's result
-  while (iteration < 64 && nverts < kEpaMaxVerts - 1) {
+  int rverts = -1;  // the face whose result is returned, if any
+  D3 rn{0.0, 0.0, 0.0};
+  double rdist = 0.0;
+  while (iteration < kEpaMaxIter) {
     iteration++;
     F.valid &= ~F.pend;  // the reference's per-iteration recompute retires them
     F.pend = 0;
+    // slots past the first LPP are rarely in use: one ballot skips their share
+    // of every step (wave-uniform)
+    bool many = __ballot(F.valid > 1u) != 0;
 
     double cdist;
-    const int cf = closest_face<LPP>(F, lane, cdist);
+    const int cf = closest_face<LPP>(F, many, cdist);
     if (cf < 0) break;
     D3 n;
     int cverts;
-    fetch_face<LPP>(F, cf, n, cverts);
+    fetch_face<LPP>(F, cf, many, n, cdist, cverts);
 
     int ia, ib;
-    const D3 nv = support_epa<LPP>(A, B, n, ia, ib, lane);
+    const D3 nv = support_epa<LPP>(V, n, ia, ib, lane);
     const double improvement = dot(n, nv) - cdist;
-    if (improvement < tol) {
-      face_result(A, B, sh, cverts, n, cdist, distance, w, normal);
-      wrote = true;
-      break;
-    }
-
-    bool dup = false;
-    {
-      const double eps_sq = kEps64 * kEps64;
-      for (int t = lane; t < nverts; t += LPP) {
-        const double dx = nv.x - sh.vx[t], dy = nv.y - sh.vy[t], dz = nv.z - sh.vz[t];
-        if (dx * dx + dy * dy + dz * dz < eps_sq) dup = true;
-      }
-    }
-    if (group_any<LPP>(dup)) {
-      face_result(A, B, sh, cverts, n, cdist, distance, w, normal);
-      wrote = true;
+    if (improvement < tol || !is_new_point<LPP>(sh, nverts, nv, lane)) {
+      rverts = cverts;
+      rn = n;
+      rdist = cdist;
       break;
     }
 
     // add the vertex and update the running-mean centroid (EPA.c:686-699)
     const int nid = nverts;
-    if (lane == 0) {
-      sh.vx[nid] = nv.x;
-      sh.vy[nid] = nv.y;
-      sh.vz[nid] = nv.z;
-      sh.via[nid] = ia;
-      sh.vib[nid] = ib;
-    }
+    if (lane == 0) put_vertex(sh, nid, nv, ia, ib);
     nverts++;
     const double inv_n = 1.0 / (double)nverts;
     centroid.x += (nv.x - centroid.x) * inv_n;
@@ -435,92 +515,107 @@ OGJK_DEV void epa(const BT& A, const BT& B, Simplex& s, double& distance, Wit& w
     centroid.z += (nv.z - centroid.z) * inv_n;
     wave_sync();
 
-    // faces visible from the new vertex (is_face_visible, EPA.c:132-140)
-    bool vis[FPL];
+    // faces visible from the new vertex (is_face_visible, EPA.c:132-140); each
+    // marks its edges in the tables
+    unsigned vis = 0;
 #pragma unroll
     for (int q = 0; q < FPL; q++) {
-      vis[q] = false;
-      if ((F.valid >> q) & 1u) {
-        const D3 p0 = lds_v(sh, F.verts[q] & 0xff);
-        const D3 fn{F.nx[q], F.ny[q], F.nz[q]};
-        vis[q] = dot(fn, sub(nv, p0)) > kEps64;
-      }
-    }
-    int vrank[FPL];
-    const int nvis = slot_rank<LPP, FPL>(vis, vrank);
-#pragma unroll
-    for (int q = 0; q < FPL; q++) {
-      if (vis[q]) {
-        F.valid &= ~(1u << q);
+      if ((q == 0 || many) && ((F.valid >> q) & 1u)) {
         const int pv = F.verts[q];
         const int x0 = pv & 0xff, x1 = (pv >> 8) & 0xff, x2 = (pv >> 16) & 0xff;
-        const int e = 3 * vrank[q];
-        sh.edir[e + 0] = edge_word(x0, x1);
-        sh.edir[e + 1] = edge_word(x1, x2);
-        sh.edir[e + 2] = edge_word(x2, x0);
+        const D3 fn{F.nx[q], F.ny[q], F.nz[q]};
+        if (dot(fn, sub(nv, lds_v(sh, x0))) > kEps64) {
+          vis |= 1u << q;
+          int w0, w1, w2;
+          unsigned b0, b1, b2;
+          edge_place(x0, x1, w0, b0);
+          edge_place(x1, x2, w1, b1);
+          edge_place(x2, x0, w2, b2);
+          const unsigned o0 = lds_or(&sh.met[w0], b0), o1 = lds_or(&sh.met[w1], b1),
+                         o2 = lds_or(&sh.met[w2], b2);
+          if (o0 & b0) lds_or(&sh.again[w0], b0);
+          if (o1 & b1) lds_or(&sh.again[w1], b1);
+          if (o2 & b2) lds_or(&sh.again[w2], b2);
+        }
       }
     }
+    F.valid &= ~vis;
     wave_sync();
 
-    // horizon = edges that occur exactly once, kept in edge order
-    const int E = 3 * nvis;
+    // horizon = edges met once, in slot order, (v0v1, v1v2, v2v0) within a face
     int nsurv = 0;
-    for (int base = 0; base < E; base += LPP) {
-      const int e = base + lane;
-      bool keep = false;
-      unsigned mine = 0u;
-      if (e < E) {
-        mine = sh.edir[e];
-        const unsigned key = mine >> 16;
-        int c = 0;
-#pragma unroll 8
-        for (int f = 0; f < E; f++) c += (sh.edir[f] >> 16) == key;
-        keep = (c == 1);
-      }
-      const uint64_t gb = group_ballot<LPP>(keep);
-      if (keep) sh.surv[nsurv + group_prefix<LPP>(gb)] = (unsigned short)(mine & 0xffffu);
-      nsurv += __popcll(gb);
-    }
-    wave_sync();
-
-    // fan new faces into the lowest free slots (EPA.c:761-825)
-    bool fr[FPL];
-    int frank[FPL];
-#pragma unroll
-    for (int q = 0; q < FPL; q++) fr[q] = !((F.valid >> q) & 1u);
-    slot_rank<LPP, FPL>(fr, frank);
 #pragma unroll
     for (int q = 0; q < FPL; q++) {
-      if (fr[q] && frank[q] < nsurv) {
-        const int ed = sh.surv[frank[q]];
+      if (q == 0 || many) {
+        bool k0 = false, k1 = false, k2 = false;
+        const int pv = F.verts[q];
+        const int x0 = pv & 0xff, x1 = (pv >> 8) & 0xff, x2 = (pv >> 16) & 0xff;
+        if ((vis >> q) & 1u) {
+          int w0, w1, w2;
+          unsigned b0, b1, b2;
+          edge_place(x0, x1, w0, b0);
+          edge_place(x1, x2, w1, b1);
+          edge_place(x2, x0, w2, b2);
+          k0 = !(sh.again[w0] & b0);
+          k1 = !(sh.again[w1] & b1);
+          k2 = !(sh.again[w2] & b2);
+        }
+        const auto m0 = lanes_where<LPP>(k0), m1 = lanes_where<LPP>(k1), m2 = lanes_where<LPP>(k2);
+        int at = nsurv + lanes_below<LPP>(m0, lane) + lanes_below<LPP>(m1, lane) +
+                 lanes_below<LPP>(m2, lane);
+        // at most kEpaMaxFaces slots can take a new face
+        if (k0 && at < kEpaMaxFaces) sh.surv[at] = (unsigned short)(x0 | (x1 << 8));
+        at += k0;
+        if (k1 && at < kEpaMaxFaces) sh.surv[at] = (unsigned short)(x1 | (x2 << 8));
+        at += k1;
+        if (k2 && at < kEpaMaxFaces) sh.surv[at] = (unsigned short)(x2 | (x0 << 8));
+        nsurv += count_lanes<LPP>(m0) + count_lanes<LPP>(m1) + count_lanes<LPP>(m2);
+      }
+    }
+    wave_sync();
+    // leave the tables clear
+#pragma unroll
+    for (int q = 0; q < FPL; q++) {
+      if ((q == 0 || many) && ((vis >> q) & 1u)) {
+        const int pv = F.verts[q];
+        const int x0 = pv & 0xff, x1 = (pv >> 8) & 0xff, x2 = (pv >> 16) & 0xff;
+        int w0, w1, w2;
+        unsigned b;
+        edge_place(x0, x1, w0, b);
+        edge_place(x1, x2, w1, b);
+        edge_place(x2, x0, w2, b);
+        sh.met[w0] = sh.again[w0] = 0u;
+        sh.met[w1] = sh.again[w1] = 0u;
+        sh.met[w2] = sh.again[w2] = 0u;
+      }
+    }
+
+    // fan new faces into the lowest free slots (EPA.c:761-825)
+    int taken = 0;
+#pragma unroll
+    for (int q = 0; q < FPL; q++) {
+      if (q > 0 && __ballot(taken < nsurv) == 0) break;
+      const bool fr = !((F.valid >> q) & 1u);
+      const auto mf = lanes_where<LPP>(fr);
+      const int rank = taken + lanes_below<LPP>(mf, lane);
+      if (fr && rank < nsurv) {
+        const int ed = sh.surv[rank];
         put_face(F, q, build_face(sh, ed & 0xff, (ed >> 8) & 0xff, nid, centroid));
       }
+      taken += count_lanes<LPP>(mf);
     }
   }
 
-  if (iteration >= 64) {  // cap fallback (EPA.c:828-863)
+  if (iteration >= kEpaMaxIter) {  // cap fallback (EPA.c:828-863)
     F.valid &= ~F.pend;
     F.pend = 0;
-    double cdist;
-    const int cf = closest_face<LPP>(F, lane, cdist);
-    if (cf >= 0) {
-      D3 n;
-      int cverts;
-      fetch_face<LPP>(F, cf, n, cverts);
-      face_result(A, B, sh, cverts, n, cdist, distance, w, normal);
-      wrote = true;
-    }
+    const int cf = closest_face<LPP>(F, true, rdist);
+    if (cf >= 0) fetch_face<LPP>(F, cf, true, rn, rdist, rverts);
   }
-  // the starting tetrahedron (the simplex this call returns) and, when no
-  // face result was written, the witnesses EPA started from
-  s.n = 4;
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    s.p[k] = lds_v(sh, k);
-    s.ia[k] = sh.via[k];
-    s.ib[k] = sh.vib[k];
-  }
-  if (!wrote) {
+  simplex_back(sh, s, 4);
+  if (rverts >= 0) {
+    face_result(V, sh, rverts, rn, rdist, distance, w, normal);
+  } else {  // no face: the witnesses EPA started from
     w.w0 = D3{sh.w_in[0], sh.w_in[1], sh.w_in[2]};
     w.w1 = D3{sh.w_in[3], sh.w_in[4], sh.w_in[5]};
   }

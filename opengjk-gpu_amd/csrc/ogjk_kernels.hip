@@ -400,7 +400,10 @@ __global__ void __launch_bounds__(256) k_pairs(Src src, OutArgs out, int n) {
   } else {
     load_input(out, pair, A, B, s, w, dist);
   }
-  if constexpr (kEpa) epa<LPP>(A, B, s, dist, w, normal, sh[kEpa ? g : 0], lane);
+  if constexpr (kEpa) {
+    epa_shared_begin<LPP>(sh[g], lane);
+    epa<LPP>(A, B, s, dist, w, normal, sh[g], lane);
+  }
   if (lane == 0) store(out, pair, s, w, dist, normal, kEpa);
 }
 
@@ -673,6 +676,7 @@ __global__ void __launch_bounds__(256, Src::template kEpaWaves<LPP>)
   if (blockIdx.x * GPB >= njobs) return;
   const EpaJob* mine =
       jobs + __builtin_amdgcn_readfirstlane(plan.nb > 1 ? c[kClassStart + cls] : 0u);
+  epa_shared_begin<LPP>(sh[g], lane);
   int slice = blockIdx.x & (kSlices - 1), tried = 0;
   for (;;) {
     unsigned j = claim(c, kQueueEpa + cls, njobs, slice, tried, lane == 0);
@@ -741,6 +745,7 @@ __global__ void __launch_bounds__(256) k_epa_all(Src src, OutArgs out, int n, co
   typename Src::BodyT A, B;
   src.template load<LPP>(pair, lane, A, B);  // validated by the GJK kernel
   D3 normal{0.0, 0.0, 0.0};
+  epa_shared_begin<LPP>(sh[g], lane);
   epa<LPP>(A, B, s, dist, w, normal, sh[g], lane);
   if (lane == 0) store(out, pair, s, w, dist, normal, true);
 }

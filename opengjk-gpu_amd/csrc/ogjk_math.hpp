@@ -74,6 +74,11 @@ OGJK_DEV int count_lanes(lane_mask<LPP> m) {
   if constexpr (LPP == 64) return __popcll(m);
   else return __popc(m);
 }
+template <int LPP>
+OGJK_DEV int first_lane(lane_mask<LPP> m) {
+  if constexpr (LPP == 64) return (int)__builtin_ctzll(m);
+  else return (int)__builtin_ctz(m);
+}
 // Set bits of m below lane l of the group (l = this lane's index in it).
 template <int LPP>
 OGJK_DEV int lanes_below(lane_mask<LPP> m, int l) {
@@ -104,10 +109,10 @@ OGJK_DEV int group_prefix(uint64_t gb) {
 // rows through ds_bpermute.
 template <int M>
 OGJK_DEV int xchg_i32(int v) {
-  if constexpr (M == 1) return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false);
-  else if constexpr (M == 2) return __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, false);
-  else if constexpr (M == 4) return __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, false);
-  else if constexpr (M == 8) return __builtin_amdgcn_update_dpp(0, v, 0x140, 0xF, 0xF, false);
+  if constexpr (M == 1) return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, true);
+  else if constexpr (M == 2) return __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, true);
+  else if constexpr (M == 4) return __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, true);
+  else if constexpr (M == 8) return __builtin_amdgcn_update_dpp(0, v, 0x140, 0xF, 0xF, true);
   else if constexpr (M == 16) {
     // v_permlane16_swap with both operands = v: result 0 holds the even
     // 16-lane row's value, result 1 the odd row's, in both rows of a pair
@@ -175,6 +180,37 @@ OGJK_DEV void xpair(double v, double& a, double& b) {
   b = __builtin_bit_cast(double, ((uint64_t)(uint32_t)hi1 << 32) | (uint32_t)lo1);
 }
 
+// The values of a group's two halves, each uniform over its half, on every
+// lane.  Halves of 16 and 32 lanes: the swap with both operands = v is that
+// pair (see xpair_i32).
+template <int LPP>
+OGJK_DEV void both_halves(int v, int& lo, int& hi) {
+  if constexpr (LPP == 32 || LPP == 64) {
+    xpair_i32<LPP / 2>(v, lo, hi);
+  } else {
+    const int o = xchg_i32<LPP / 2>(v);
+    const bool up = (lane_id() & (LPP / 2)) != 0;
+    lo = up ? o : v;
+    hi = up ? v : o;
+  }
+}
+template <int LPP>
+OGJK_DEV void both_halves(float v, float& lo, float& hi) {
+  int a, b;
+  both_halves<LPP>(__builtin_bit_cast(int, v), a, b);
+  lo = __builtin_bit_cast(float, a);
+  hi = __builtin_bit_cast(float, b);
+}
+template <int LPP>
+OGJK_DEV void both_halves(double v, double& lo, double& hi) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  int lo0, lo1, hi0, hi1;
+  both_halves<LPP>((int)(uint32_t)u, lo0, lo1);
+  both_halves<LPP>((int)(uint32_t)(u >> 32), hi0, hi1);
+  lo = __builtin_bit_cast(double, ((uint64_t)(uint32_t)hi0 << 32) | (uint32_t)lo0);
+  hi = __builtin_bit_cast(double, ((uint64_t)(uint32_t)hi1 << 32) | (uint32_t)lo1);
+}
+
 template <int LPP>
 OGJK_DEV double shfl_d(double v, int src) {
   return __shfl(v, src, LPP);
@@ -195,6 +231,18 @@ OGJK_DEV float group_max_f(float v) {
     xpair<M>(v, a, b);
     v = fmaxf(a, b);
     return group_max_f<LPP, 2 * M>(v);
+  } else {
+    return v;
+  }
+}
+
+// Min over the group (no NaN).
+template <int LPP, int M = 1>
+OGJK_DEV double group_min_d(double v) {
+  if constexpr (M < LPP) {
+    double a, b;
+    xpair<M>(v, a, b);
+    return group_min_d<LPP, 2 * M>(b < a ? b : a);
   } else {
     return v;
   }
