@@ -76,6 +76,7 @@ struct Query {
   bool has_inc;
   int inc_idx;
   D3 inc_pt;
+  bool unit = false;  // |dir| = 1 up to rounding: no scaling needed
 };
 
 // A lane's FP64-exact candidate after the sweep: value, index, point.
@@ -95,15 +96,22 @@ struct Sweep32 {
 // Scale the direction by an exact power of two so its max-norm is in
 // [0.5, 1): the FP32 copy then carries a relative error <= 2^-24 per
 // component whatever the magnitude of dir (tiny GJK directions included).
-OGJK_DEV Sweep32 sweep32_begin(D3 dir) {
-  const double mx = fmax(fabs(dir.x), fmax(fabs(dir.y), fabs(dir.z)));
-  int e = 0;
-  (void)frexp(mx, &e);
-  const double sc = ldexp(1.0, -e);
+// A unit direction is taken as it is (max-norm in [0.57, 1 + 2^-50]).
+OGJK_DEV Sweep32 sweep32_begin(D3 dir, bool unit = false) {
   Sweep32 s;
-  s.dx = (float)(dir.x * sc);
-  s.dy = (float)(dir.y * sc);
-  s.dz = (float)(dir.z * sc);
+  if (unit) {
+    s.dx = (float)dir.x;
+    s.dy = (float)dir.y;
+    s.dz = (float)dir.z;
+  } else {
+    const double mx = fmax(fabs(dir.x), fmax(fabs(dir.y), fabs(dir.z)));
+    int e = 0;
+    (void)frexp(mx, &e);
+    const double sc = ldexp(1.0, -e);
+    s.dx = (float)(dir.x * sc);
+    s.dy = (float)(dir.y * sc);
+    s.dz = (float)(dir.z * sc);
+  }
   s.best = s.second = -INFINITY;
   s.bx = s.by = s.bz = 0.0f;
   s.bi = -1;
@@ -122,34 +130,37 @@ OGJK_DEV void sweep32_take(Sweep32& s, float px, float py, float pz, float d, in
   s.bz = better ? pz : s.bz;
 }
 
-// One lane's share of the FP32 sweep: vertices lane, lane + LPP, ...  Four of
-// them are loaded at a time: with one per trip the loop waits out a memory
-// round trip for every LPP vertices, and a sweep is little else.
+// U vertices of the sweep in flight: base + lane, base + LPP + lane, ...
+template <int LPP, int U, int STRIDE>
+OGJK_DEV void sweep32_batch(const Body<float, STRIDE>& b, int base, int lane, Sweep32& s) {
+  float px[U], py[U], pz[U];
+#pragma unroll
+  for (int k = 0; k < U; k++) {
+    const int i = min(base + k * LPP + lane, b.n - 1);
+    px[k] = b.rx(i);
+    py[k] = b.ry(i);
+    pz[k] = b.rz(i);
+  }
+#pragma unroll
+  for (int k = 0; k < U; k++) {
+    const int i = base + k * LPP + lane;
+    const float d = fmaf(px[k], s.dx, fmaf(py[k], s.dy, pz[k] * s.dz));
+    sweep32_take(s, px[k], py[k], pz[k], i < b.n ? d : -INFINITY, i);
+  }
+}
+
+// One lane's share of the FP32 sweep: vertices lane, lane + LPP, ...  Up to
+// four of them are loaded at a time: with one per trip the loop waits out a
+// memory round trip for every LPP vertices, and a sweep is little else.
 template <int LPP, int STRIDE>
 OGJK_DEV void sweep32(const Body<float, STRIDE>& b, int lane, Sweep32& s) {
-  constexpr int U = 4;
   int base = 0;
 #pragma clang loop unroll(disable)
-  for (; base + LPP < b.n; base += U * LPP) {
-    float px[U], py[U], pz[U];
-#pragma unroll
-    for (int k = 0; k < U; k++) {
-      const int i = min(base + k * LPP + lane, b.n - 1);
-      px[k] = b.rx(i);
-      py[k] = b.ry(i);
-      pz[k] = b.rz(i);
-    }
-#pragma unroll
-    for (int k = 0; k < U; k++) {
-      const int i = base + k * LPP + lane;
-      const float d = fmaf(px[k], s.dx, fmaf(py[k], s.dy, pz[k] * s.dz));
-      sweep32_take(s, px[k], py[k], pz[k], i < b.n ? d : -INFINITY, i);
-    }
-  }
-  if (base + lane < b.n) {
-    const int i = base + lane;
-    const float px = b.rx(i), py = b.ry(i), pz = b.rz(i);
-    sweep32_take(s, px, py, pz, fmaf(px, s.dx, fmaf(py, s.dy, pz * s.dz)), i);
+  for (; base + 2 * LPP < b.n; base += 4 * LPP) sweep32_batch<LPP, 4>(b, base, lane, s);
+  if (base + LPP < b.n) {
+    sweep32_batch<LPP, 2>(b, base, lane, s);
+  } else if (base < b.n) {
+    sweep32_batch<LPP, 1>(b, base, lane, s);
   }
 }
 
@@ -220,13 +231,29 @@ struct SupF {
 };
 OGJK_DEV Sup widen(const SupF& s) { return Sup{s.i, D3{(double)s.x, (double)s.y, (double)s.z}}; }
 
+// The acceptance rule for the only vertex r in the window of a float body's
+// query, t the window's lower end.  FP32 settles it nearly always: r is the
+// incumbent, or beats it by more than the window, or (EPA, unit direction: sweep
+// values are not scaled) the window lies far above -1e10.
+OGJK_DEV SupF accept(const SupF& r, const Query& q, const Sweep32& sw, float t) {
+  const D3 p{(double)r.x, (double)r.y, (double)r.z};
+  if (q.has_inc) {
+    const float ix = (float)q.inc_pt.x, iy = (float)q.inc_pt.y, iz = (float)q.inc_pt.z;
+    const float di = fmaf(ix, sw.dx, fmaf(iy, sw.dy, iz * sw.dz));
+    if (r.i != q.inc_idx && !(t > di) && !(dot(p, q.dir) > dot(q.inc_pt, q.dir)))
+      return SupF{q.inc_idx, ix, iy, iz};
+  } else if (!(q.unit && t > -1e9f) && !(dot(p, q.dir) > -1e10)) {
+    return SupF{-1, 0.0f, 0.0f, 0.0f};
+  }
+  return r;
+}
+
 // Support point of one body (FP32 sweep, FP64 re-rank of the window).  Nearly
 // always a single vertex lies in the window: its lane is known from one
-// ballot, its index and FP32 point are fetched, and every lane evaluates the
-// acceptance rule's FP64 product itself.
+// ballot, and its index and FP32 point are fetched.
 template <int LPP, int STRIDE>
 OGJK_DEV SupF support_f(const Body<float, STRIDE>& A, const Query& q, int lane) {
-  Sweep32 sw = sweep32_begin(q.dir);
+  Sweep32 sw = sweep32_begin(q.dir, q.unit);
   sweep32<LPP>(A, lane, sw);
   const float m = group_max_f<LPP>(sw.best);
   // |D32 - scale*D64| <= 16u * r1 (u = 2^-24): candidates lie within 2x that.
@@ -235,13 +262,9 @@ OGJK_DEV SupF support_f(const Body<float, STRIDE>& A, const Query& q, int lane) 
   const auto holders = lanes_where<LPP>(sw.bi >= 0 && sw.best >= t);
   if (!multi && count_lanes<LPP>(holders) == 1) {
     const int src = first_lane<LPP>(holders);
-    const SupF r{shfl_i<LPP>(sw.bi, src), shfl_f<LPP>(sw.bx, src), shfl_f<LPP>(sw.by, src),
-                 shfl_f<LPP>(sw.bz, src)};
-    const double v = dot(D3{(double)r.x, (double)r.y, (double)r.z}, q.dir);
-    if (q.has_inc && !(v > dot(q.inc_pt, q.dir)))
-      return SupF{q.inc_idx, (float)q.inc_pt.x, (float)q.inc_pt.y, (float)q.inc_pt.z};
-    if (!q.has_inc && !(v > -1e10)) return SupF{-1, 0.0f, 0.0f, 0.0f};
-    return r;
+    return accept(SupF{shfl_i<LPP>(sw.bi, src), shfl_f<LPP>(sw.bx, src),
+                       shfl_f<LPP>(sw.by, src), shfl_f<LPP>(sw.bz, src)},
+                  q, sw, t);
   }
   const Sup r = finish1<LPP>(candidates32<LPP>(A, sw, t, multi, q.dir, lane), q);
   return SupF{r.i, (float)r.p.x, (float)r.p.y, (float)r.p.z};
@@ -529,8 +552,7 @@ OGJK_DEV void visit_live(bool live, int c, int n, const float* sx, const float* 
 // with its value.
 OGJK_DEV int wave_best(float v, int i, float& top) {
   top = group_max_f<64>(v);
-  return __builtin_amdgcn_readfirstlane(
-      shfl_i<64>(i, (int)__builtin_ctzll(__ballot(v == top) | (1ull << 63))));
+  return lane_value(i, (int)__builtin_ctzll(__ballot(v == top) | (1ull << 63)));
 }
 
 // The two entries with the largest bounds of b[0, n): ub[j] keeps the bound of
@@ -580,7 +602,7 @@ OGJK_DEV void two_best(const ClusterBound* b, int n, float dx, float dy, float d
 template <bool TWO>
 OGJK_DEV Sup support_clustered64(const CBody& A, const Query& q, int lane) {
   if (A.slot < 0) return support<64>(static_cast<const Body<float, 1>&>(A), q, lane);
-  Sweep32 sw = sweep32_begin(q.dir);
+  Sweep32 sw = sweep32_begin(q.dir, q.unit);
   const float dx = sw.dx, dy = sw.dy, dz = sw.dz;
   const float dn = sqrtf(fmaf(dx, dx, fmaf(dy, dy, dz * dz))) * (1.0f + 0x1.0p-20f);
   const int nc = (A.n + kCluster - 1) / kCluster;
@@ -683,12 +705,9 @@ OGJK_DEV Sup support_clustered64(const CBody& A, const Query& q, int lane) {
   const uint64_t holders = __ballot(sw.bi >= 0 && sw.best >= T);
   if (!multi && __popcll(holders) == 1) {  // as in support_f
     const int src = (int)__builtin_ctzll(holders);
-    const Sup r = widen(SupF{shfl_i<64>(oi, src), shfl_f<64>(sw.bx, src), shfl_f<64>(sw.by, src),
-                             shfl_f<64>(sw.bz, src)});
-    const double v = dot(r.p, q.dir);
-    if (q.has_inc && !(v > dot(q.inc_pt, q.dir))) return Sup{q.inc_idx, q.inc_pt};
-    if (!q.has_inc && !(v > -1e10)) return Sup{-1, D3{0.0, 0.0, 0.0}};
-    return r;
+    return widen(accept(SupF{lane_value(oi, src), lane_value(sw.bx, src),
+                             lane_value(sw.by, src), lane_value(sw.bz, src)},
+                        q, sw, T));
   }
 
   // FP64 re-rank of the window; ties go to the lowest input index
@@ -858,7 +877,7 @@ OGJK_DEV PBody pick(bool c, const PBody& a, const PBody& b) {
 }
 OGJK_DEV Query pick(bool c, const Query& a, const Query& b) {
   return Query{sel(c, a.dir, b.dir), c ? a.has_inc : b.has_inc, c ? a.inc_idx : b.inc_idx,
-               sel(c, a.inc_pt, b.inc_pt)};
+               sel(c, a.inc_pt, b.inc_pt), c ? a.unit : b.unit};
 }
 
 template <int LPP>

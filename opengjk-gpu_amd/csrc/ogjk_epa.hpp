@@ -1,12 +1,14 @@
 // opengjk-amd device EPA for one pair on a group of LPP lanes (LPP <= 64).
 //
 // Layout: the polytope's vertex pool (<= 68 FP64 points and their body
-// indices), the edge tables and the input witnesses live in LDS; the
-// 128 face slots are spread over the group's lanes, slot = q*LPP + lane,
-// FPL = 128/LPP faces per lane held in registers (normal, plane distance,
-// packed vertex ids).  Nothing else of the pair stays in registers through
-// the expansion loop: the starting tetrahedron is slots 0-3 of the vertex
-// pool and is read back from there when the loop ends.
+// indices), the edge tables and the input witnesses live in LDS.  The 128 face
+// slots are spread over the group's lanes, slot = q * LPP + lane.  A polytope
+// seldom has more than 30 faces, so each lane holds the face of its first slot
+// (q = 0) in registers and those of the others in LDS: with all of them in
+// registers the 32-lane kernel wanted 190 of the 168 that three waves per SIMD
+// leave it.  Nothing else of the pair stays in registers through the expansion
+// loop: the starting tetrahedron is slots 0-3 of the vertex pool and is read
+// back from there when the loop ends.
 //
 // The reference EPA (GJK/cpu/EPA.c:362-864) is sequential; its discrete
 // choices are reproduced exactly with ballots:
@@ -30,16 +32,26 @@ constexpr int kEpaMaxIter = 64;
 // the tetrahedron and one vertex per iteration (below the reference's cap of
 // 132, EPA.c:44, which therefore never ends the loop)
 constexpr int kEpaMaxVerts = 4 + kEpaMaxIter;
-constexpr int kEdgeWords = (kEpaMaxVerts + 31) / 32;  // bits of one vertex's row
+constexpr int kEdgeWords = (kEpaMaxVerts * (kEpaMaxVerts - 1) / 2 + 31) / 32;
 
+template <int LPP>
 struct EpaShared {
   double vx[kEpaMaxVerts], vy[kEpaMaxVerts], vz[kEpaMaxVerts];
+  double w_in[6];  // the witnesses EPA started from
+  // faces of the slots past the first LPP
+  static constexpr int kFar = kEpaMaxFaces - LPP;
+  double nx[kFar], ny[kFar], nz[kFar], dist[kFar];
+  int verts[kFar];
   int via[kEpaMaxVerts], vib[kEpaMaxVerts];
-  // edges (a < b) of the faces removed this iteration, bit b of row a: those
-  // met, and those met more than once.  All zero between iterations.
-  unsigned met[kEpaMaxVerts * kEdgeWords], again[kEpaMaxVerts * kEdgeWords];
+  // a bit per edge of the faces removed this iteration: those met, and those
+  // met more than once.  All zero between iterations.
+  unsigned met[kEdgeWords], again[kEdgeWords];
   unsigned short surv[kEpaMaxFaces];  // surviving horizon edges, in order
-  double w_in[6];                     // the witnesses EPA started from
+};
+
+// Per block: 1 / (5 + i), the weights of the centroid's running mean.
+struct EpaTable {
+  double inv[kEpaMaxIter];
 };
 
 OGJK_DEV void wave_sync() {
@@ -50,23 +62,79 @@ OGJK_DEV void wave_sync() {
 // Clears the edge tables: once before a group's first pair (epa() leaves them
 // clear).
 template <int LPP>
-OGJK_DEV void epa_shared_begin(EpaShared& sh, int lane) {
-  for (int i = lane; i < kEpaMaxVerts * kEdgeWords; i += LPP) sh.met[i] = sh.again[i] = 0u;
+OGJK_DEV void epa_shared_begin(EpaShared<LPP>& sh, int lane) {
+  for (int i = lane; i < kEdgeWords; i += LPP) sh.met[i] = sh.again[i] = 0u;
   wave_sync();
+}
+// By every thread of the block.
+OGJK_DEV void epa_table_begin(EpaTable& tb) {
+  if (threadIdx.x < kEpaMaxIter) tb.inv[threadIdx.x] = 1.0 / (double)(5 + (int)threadIdx.x);
+  __syncthreads();
 }
 
 // Place of the edge (a, b) in the edge tables.
 OGJK_DEV void edge_place(int a, int b, int& word, unsigned& bit) {
   const int lo = min(a, b), hi = max(a, b);
-  word = lo * kEdgeWords + (hi >> 5);
-  bit = 1u << (hi & 31);
+  const unsigned at = ((unsigned)__mul24(hi, hi - 1) >> 1) + (unsigned)lo;
+  word = (int)(at >> 5);
+  bit = 1u << (at & 31u);
+}
+
+// Places of a face's edges (v0v1, v1v2, v2v0), from its packed vertices.
+OGJK_DEV void face_edges(int packed, int (&w)[3], unsigned (&b)[3]) {
+  const int x0 = packed & 0xff, x1 = (packed >> 8) & 0xff, x2 = (packed >> 16) & 0xff;
+  edge_place(x0, x1, w[0], b[0]);
+  edge_place(x1, x2, w[1], b[1]);
+  edge_place(x2, x0, w[2], b[2]);
 }
 
 OGJK_DEV unsigned lds_or(unsigned* p, unsigned bits) {
   return __hip_atomic_fetch_or(p, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
 }
 
-OGJK_DEV D3 lds_v(const EpaShared& sh, int i) { return D3{sh.vx[i], sh.vy[i], sh.vz[i]}; }
+template <int LPP>
+OGJK_DEV void mark_edges(EpaShared<LPP>& sh, const int (&w)[3], const unsigned (&b)[3]) {
+  unsigned old[3];
+#pragma unroll
+  for (int k = 0; k < 3; k++) old[k] = lds_or(&sh.met[w[k]], b[k]);
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    const unsigned twice = old[k] & b[k];
+    if (twice) lds_or(&sh.again[w[k]], twice);
+  }
+}
+
+// Appends the edges of the lanes' removed faces (`mine`) that were met once to
+// the surviving ones, of which there are n; returns how many.
+template <int LPP>
+OGJK_DEV int keep_edges(EpaShared<LPP>& sh, bool mine, int packed, const int (&w)[3],
+                        const unsigned (&b)[3], int n, int lane) {
+  bool k0 = false, k1 = false, k2 = false;
+  if (mine) {
+    k0 = !(sh.again[w[0]] & b[0]);
+    k1 = !(sh.again[w[1]] & b[1]);
+    k2 = !(sh.again[w[2]] & b[2]);
+  }
+  const int x0 = packed & 0xff, x1 = (packed >> 8) & 0xff, x2 = (packed >> 16) & 0xff;
+  const auto m0 = lanes_where<LPP>(k0), m1 = lanes_where<LPP>(k1), m2 = lanes_where<LPP>(k2);
+  int at = n + lanes_below<LPP>(m0, lane) + lanes_below<LPP>(m1, lane) + lanes_below<LPP>(m2, lane);
+  // at most kEpaMaxFaces slots can take a new face
+  if (k0 && at < kEpaMaxFaces) sh.surv[at] = (unsigned short)(x0 | (x1 << 8));
+  at += k0;
+  if (k1 && at < kEpaMaxFaces) sh.surv[at] = (unsigned short)(x1 | (x2 << 8));
+  at += k1;
+  if (k2 && at < kEpaMaxFaces) sh.surv[at] = (unsigned short)(x2 | (x0 << 8));
+  return count_lanes<LPP>(m0) + count_lanes<LPP>(m1) + count_lanes<LPP>(m2);
+}
+
+template <int LPP>
+OGJK_DEV void clear_edges(EpaShared<LPP>& sh, const int (&w)[3]) {
+#pragma unroll
+  for (int k = 0; k < 3; k++) sh.met[w[k]] = sh.again[w[k]] = 0u;
+}
+
+template <int LPP>
+OGJK_DEV D3 lds_v(const EpaShared<LPP>& sh, int i) { return D3{sh.vx[i], sh.vy[i], sh.vz[i]}; }
 
 // set_contact_normal: GJK/cpu/EPA.c:350-360
 OGJK_DEV D3 contact_normal(D3 w1, D3 w2) {
@@ -116,10 +184,10 @@ OGJK_DEV void bary_origin(D3 v0, D3 v1, D3 v2, double& a0, double& a1, double& a
   }
 }
 
-template <int FPL>
+// A lane's faces: the first slot's in registers, and which slots are in use.
 struct Faces {
-  double nx[FPL], ny[FPL], nz[FPL], dist[FPL];
-  int verts[FPL];  // v0 | v1 << 8 | v2 << 16
+  double nx, ny, nz, dist;
+  int verts;       // v0 | v1 << 8 | v2 << 16
   unsigned valid;  // bit q
   unsigned pend;   // bit q: degenerate, retire at the next iteration start
 };
@@ -140,7 +208,8 @@ struct NewFace {
 // p1 - p0) is exactly -cross(p1 - p0, p2 - p0) (products commute exactly,
 // x - y = -(y - x)), so the swapped face's normal is the negated one, bit for
 // bit.
-OGJK_DEV NewFace build_face(const EpaShared& sh, int v0, int v1, int v2, D3 centroid) {
+template <int LPP>
+OGJK_DEV NewFace build_face(const EpaShared<LPP>& sh, int v0, int v1, int v2, D3 centroid) {
   const D3 p0 = lds_v(sh, v0);
   D3 n = cross(sub(lds_v(sh, v1), p0), sub(lds_v(sh, v2), p0));
   const bool swap = dot(n, sub(centroid, p0)) > 0;
@@ -164,72 +233,68 @@ OGJK_DEV NewFace build_face(const EpaShared& sh, int v0, int v1, int v2, D3 cent
   return f;
 }
 
-template <int FPL>
-OGJK_DEV void put_face(Faces<FPL>& F, int q, const NewFace& f) {
-  F.nx[q] = f.n.x;
-  F.ny[q] = f.n.y;
-  F.nz[q] = f.n.z;
-  F.dist[q] = f.d;
-  F.verts[q] = f.packed;
+template <int LPP>
+OGJK_DEV void put_face(EpaShared<LPP>& sh, Faces& F, int q, int lane, const NewFace& f) {
+  if (q == 0) {
+    F.nx = f.n.x;
+    F.ny = f.n.y;
+    F.nz = f.n.z;
+    F.dist = f.d;
+    F.verts = f.packed;
+  } else {
+    const int k = (q - 1) * LPP + lane;
+    sh.nx[k] = f.n.x;
+    sh.ny[k] = f.n.y;
+    sh.nz[k] = f.n.z;
+    sh.dist[k] = f.d;
+    sh.verts[k] = f.packed;
+  }
   F.valid |= 1u << q;
   if (!f.ok) F.pend |= 1u << q;
 }
 
-// Closest valid face with distance in [0, 1e10), lowest slot on ties: the
-// group's least distance, then the first slot that has it.  `many`: slots past
-// the first LPP are in use.
-template <int LPP, int FPL>
-OGJK_DEV int closest_face(const Faces<FPL>& F, bool many, double& cdist) {
-  double d[FPL];
+// Closest valid face with distance in [0, 1e10), lowest slot on ties: the lanes
+// with the group's least distance, then the first slot that has it.  `many`:
+// slots past the first LPP are in use.
+template <int LPP>
+OGJK_DEV int closest_face(const EpaShared<LPP>& sh, const Faces& F, bool many, int lane) {
+  constexpr int FPL = kEpaMaxFaces / LPP;
   double m = INFINITY;
-#pragma unroll
-  for (int q = 0; q < FPL; q++) {
-    d[q] = INFINITY;
-    if (q == 0 || many) {
-      const double fd = F.dist[q];
-      if (((F.valid >> q) & 1u) && fd >= 0.0 && fd < 1e10) d[q] = fd;
-      m = d[q] < m ? d[q] : m;
+  int slot = lane;
+  if ((F.valid & 1u) && F.dist >= 0.0 && F.dist < 1e10) m = F.dist;
+  if (many) {
+#pragma clang loop unroll(disable)
+    for (int q = 1; q < FPL; q++) {
+      if ((F.valid >> q) & 1u) {
+        const double fd = sh.dist[(q - 1) * LPP + lane];
+        if (fd >= 0.0 && fd < 1e10 && fd < m) {
+          m = fd;
+          slot = q * LPP + lane;
+        }
+      }
     }
   }
-  m = group_min_d<LPP>(m);
-  cdist = m;
-  if (!(m < INFINITY)) return -1;
-  int slot = -1;
-#pragma unroll
-  for (int q = 0; q < FPL; q++) {
-    if (q == 0 || many) {
-      const auto has = lanes_where<LPP>(d[q] == m);
-      if (slot < 0 && has != 0) slot = q * LPP + first_lane<LPP>(has);
-    }
-  }
-  return slot;
+  const auto least = lanes_of_least<LPP>(m);
+  const bool mine = ((least >> lane) & 1) != 0 && m < INFINITY;
+  const auto hold = lanes_where<LPP>(mine);
+  if (hold == 0) return -1;
+  if (!many) return first_lane<LPP>(hold);
+  return (int)group_min_u<LPP>(mine ? (uint32_t)slot : 0xffffffffu);
 }
 
 // Normal, distance and vertices of the face in `slot`, on every lane.
-template <int LPP, int FPL>
-OGJK_DEV void fetch_face(const Faces<FPL>& F, int slot, bool many, D3& n, double& dist,
+template <int LPP>
+OGJK_DEV void fetch_face(const EpaShared<LPP>& sh, const Faces& F, int slot, D3& n, double& dist,
                          int& verts) {
-  const int q = slot / LPP, src = slot % LPP;
-  // value selects over laundered registers (see keep_reg): no address select
-  double x = keep_reg(F.nx[0]), y = keep_reg(F.ny[0]), z = keep_reg(F.nz[0]);
-  int vv = keep_reg(F.verts[0]);
-  if (many) {
-#pragma unroll
-    for (int t = 1; t < FPL; t++) {
-      const bool h = (q == t);
-      x = h ? keep_reg(F.nx[t]) : x;
-      y = h ? keep_reg(F.ny[t]) : y;
-      z = h ? keep_reg(F.nz[t]) : z;
-      vv = h ? keep_reg(F.verts[t]) : vv;
-    }
-  }
-  n = D3{shfl_d<LPP>(x, src), shfl_d<LPP>(y, src), shfl_d<LPP>(z, src)};
-  verts = shfl_i<LPP>(vv, src);
-  if (dist == 0.0) {  // a tie of zeros of either sign: the chosen face's own
-    double own = keep_reg(F.dist[0]);
-#pragma unroll
-    for (int t = 1; t < FPL; t++) own = (q == t) ? keep_reg(F.dist[t]) : own;
-    dist = shfl_d<LPP>(own, src);
+  if (slot < LPP) {
+    n = D3{shfl_d<LPP>(F.nx, slot), shfl_d<LPP>(F.ny, slot), shfl_d<LPP>(F.nz, slot)};
+    dist = shfl_d<LPP>(F.dist, slot);
+    verts = shfl_i<LPP>(F.verts, slot);
+  } else {
+    const int k = slot - LPP;
+    n = D3{sh.nx[k], sh.ny[k], sh.nz[k]};
+    dist = sh.dist[k];
+    verts = sh.verts[k];
   }
 }
 
@@ -242,10 +307,10 @@ template <int LPP, class BT, bool SPLIT = LPP >= 16 && kSplit<LPP, BT>>
 struct PairView {
   BT A, B;
   OGJK_DEV PairView(const BT& a, const BT& b, int) : A(a), B(b) {}
-  OGJK_DEV void query(D3 dir, int lane, Sup& a, Sup& b) const {
+  OGJK_DEV void query(D3 dir, bool unit, int lane, Sup& a, Sup& b) const {
     const D3 zero{0.0, 0.0, 0.0};
-    support_pair<LPP>(A, Query{dir, false, 0, zero}, B, Query{neg(dir), false, 0, zero}, lane, a,
-                      b);
+    support_pair<LPP>(A, Query{dir, false, 0, zero, unit}, B,
+                      Query{neg(dir), false, 0, zero, unit}, lane, a, b);
     // The reference leaves its output unset when no vertex beats -1e10; such
     // coordinates are out of any physical range, fall back to vertex 0.
     if (a.i < 0) a = Sup{0, A.d(0)};
@@ -272,8 +337,8 @@ struct PairView<LPP, BT, true> {
   bool upper;
   OGJK_DEV PairView(const BT& a, const BT& b, int lane)
       : own(pick(lane >= LPP / 2, b, a)), upper(lane >= LPP / 2) {}
-  OGJK_DEV void query(D3 dir, int lane, Sup& a, Sup& b) const {
-    const Query q{sel(upper, neg(dir), dir), false, 0, D3{0.0, 0.0, 0.0}};
+  OGJK_DEV void query(D3 dir, bool unit, int lane, Sup& a, Sup& b) const {
+    const Query q{sel(upper, neg(dir), dir), false, 0, D3{0.0, 0.0, 0.0}, unit};
     if constexpr (std::is_same_v<BT, PBody>) {
       Sup r = support<LPP / 2>(own, q, lane & (LPP / 2 - 1));
       if (r.i < 0) r = Sup{0, own.d(0)};
@@ -313,9 +378,9 @@ struct PairView<LPP, Body<double, STRIDE>, true> : PairView<LPP, Body<double, ST
 // support_epa (GJK/cpu/EPA.c:307-344): farthest vertex of A along dir and of
 // B along -dir; returns the Minkowski point A[ia] - B[ib].
 template <int LPP, class PV>
-OGJK_DEV D3 support_epa(const PV& V, D3 dir, int& ia, int& ib, int lane) {
+OGJK_DEV D3 support_epa(const PV& V, D3 dir, bool unit, int& ia, int& ib, int lane) {
   Sup a, b;
-  V.query(dir, lane, a, b);
+  V.query(dir, unit, lane, a, b);
   ia = a.i;
   ib = b.i;
   return sub(a.p, b.p);
@@ -324,7 +389,7 @@ OGJK_DEV D3 support_epa(const PV& V, D3 dir, int& ia, int& ib, int lane) {
 // Is p farther than eps from each of the first n pool vertices
 // (GJK/cpu/EPA.c:453-463, 654-684)?
 template <int LPP>
-OGJK_DEV bool is_new_point(const EpaShared& sh, int n, D3 p, int lane) {
+OGJK_DEV bool is_new_point(const EpaShared<LPP>& sh, int n, D3 p, int lane) {
   const double eps_sq = kEps64 * kEps64;
   bool near = false;
   for (int t = lane; t < n; t += LPP) {
@@ -334,7 +399,8 @@ OGJK_DEV bool is_new_point(const EpaShared& sh, int n, D3 p, int lane) {
   return !group_any<LPP>(near);
 }
 
-OGJK_DEV void put_vertex(EpaShared& sh, int i, D3 p, int ia, int ib) {
+template <int LPP>
+OGJK_DEV void put_vertex(EpaShared<LPP>& sh, int i, D3 p, int ia, int ib) {
   sh.vx[i] = p.x;
   sh.vy[i] = p.y;
   sh.vz[i] = p.z;
@@ -343,7 +409,8 @@ OGJK_DEV void put_vertex(EpaShared& sh, int i, D3 p, int ia, int ib) {
 }
 
 // The simplex EPA returns: the tetrahedron it started from, pool slots 0-3.
-OGJK_DEV void simplex_back(const EpaShared& sh, Simplex& s, int n) {
+template <int LPP>
+OGJK_DEV void simplex_back(const EpaShared<LPP>& sh, Simplex& s, int n) {
   s.n = n;
 #pragma unroll
   for (int k = 0; k < 4; k++) {
@@ -360,8 +427,8 @@ OGJK_DEV void zero_depth(const PV& V, int ia, int ib, double& distance, Wit& w, 
   normal = contact_normal(w.w0, w.w1);
 }
 
-template <class PV>
-OGJK_DEV void face_result(const PV& V, const EpaShared& sh, int verts, D3 n, double cdist,
+template <int LPP, class PV>
+OGJK_DEV void face_result(const PV& V, const EpaShared<LPP>& sh, int verts, D3 n, double cdist,
                           double& distance, Wit& w, D3& normal) {
   const int v0 = verts & 0xff, v1 = (verts >> 8) & 0xff, v2 = (verts >> 16) & 0xff;
   double a[3];
@@ -377,7 +444,7 @@ OGJK_DEV void face_result(const PV& V, const EpaShared& sh, int verts, D3 n, dou
 // tables of sh are clear before and after.
 template <int LPP, class BT>
 OGJK_DEV void epa(const BT& A, const BT& B, Simplex& s, double& distance, Wit& w, D3& normal,
-                  EpaShared& sh, int lane) {
+                  EpaShared<LPP>& sh, const EpaTable& tb, int lane) {
   constexpr int FPL = kEpaMaxFaces / LPP;
   static_assert(FPL * LPP == kEpaMaxFaces, "LPP must divide 128");
 
@@ -425,7 +492,7 @@ OGJK_DEV void epa(const BT& A, const BT& B, Simplex& s, double& distance, Wit& w
       if (against) dir = neg(dir);
     }
     int ia, ib;
-    const D3 nv = support_epa<LPP>(V, dir, ia, ib, lane);
+    const D3 nv = support_epa<LPP>(V, dir, false, ia, ib, lane);
     if (is_new_point<LPP>(sh, ns, nv, lane)) {
       if (lane == 0) put_vertex(sh, ns, nv, ia, ib);
       wave_sync();
@@ -457,21 +524,13 @@ OGJK_DEV void epa(const BT& A, const BT& B, Simplex& s, double& distance, Wit& w
     centroid.y += p.y * 0.25;
     centroid.z += p.z * 0.25;
   }
-  Faces<FPL> F;
-  F.valid = 0;
-  F.pend = 0;
-#pragma unroll
-  for (int q = 0; q < FPL; q++) {
-    F.nx[q] = F.ny[q] = F.nz[q] = 0.0;
-    F.dist[q] = 0.0;
-    F.verts[q] = 0;
-  }
+  Faces F{0.0, 0.0, 0.0, 0.0, 0, 0u, 0u};
   if (lane < 4) {
     // faces (0,1,2) (0,3,1) (0,2,3) (1,3,2)
     const int a = lane == 3 ? 1 : 0;
     const int b = lane == 0 ? 1 : (lane == 1 ? 3 : (lane == 2 ? 2 : 3));
     const int c = lane == 0 ? 2 : (lane == 1 ? 1 : (lane == 2 ? 3 : 2));
-    put_face(F, 0, build_face(sh, a, b, c, centroid));
+    put_face(sh, F, 0, lane, build_face(sh, a, b, c, centroid));
   }
 
   const double tol = kEps64 * 1e2;
@@ -486,17 +545,17 @@ OGJK_DEV void epa(const BT& A, const BT& B, Simplex& s, double& distance, Wit& w
     F.pend = 0;
     // slots past the first LPP are rarely in use: one ballot skips their share
     // of every step (wave-uniform)
-    bool many = __ballot(F.valid > 1u) != 0;
+    const bool many = __ballot(F.valid > 1u) != 0;
 
-    double cdist;
-    const int cf = closest_face<LPP>(F, many, cdist);
+    const int cf = closest_face(sh, F, many, lane);
     if (cf < 0) break;
     D3 n;
+    double cdist;
     int cverts;
-    fetch_face<LPP>(F, cf, many, n, cdist, cverts);
+    fetch_face(sh, F, cf, n, cdist, cverts);
 
     int ia, ib;
-    const D3 nv = support_epa<LPP>(V, n, ia, ib, lane);
+    const D3 nv = support_epa<LPP>(V, n, true, ia, ib, lane);
     const double improvement = dot(n, nv) - cdist;
     if (improvement < tol || !is_new_point<LPP>(sh, nverts, nv, lane)) {
       rverts = cverts;
@@ -508,8 +567,8 @@ OGJK_DEV void epa(const BT& A, const BT& B, Simplex& s, double& distance, Wit& w
     // add the vertex and update the running-mean centroid (EPA.c:686-699)
     const int nid = nverts;
     if (lane == 0) put_vertex(sh, nid, nv, ia, ib);
+    const double inv_n = tb.inv[nverts - 4];
     nverts++;
-    const double inv_n = 1.0 / (double)nverts;
     centroid.x += (nv.x - centroid.x) * inv_n;
     centroid.y += (nv.y - centroid.y) * inv_n;
     centroid.z += (nv.z - centroid.z) * inv_n;
@@ -518,24 +577,27 @@ OGJK_DEV void epa(const BT& A, const BT& B, Simplex& s, double& distance, Wit& w
     // faces visible from the new vertex (is_face_visible, EPA.c:132-140); each
     // marks its edges in the tables
     unsigned vis = 0;
-#pragma unroll
-    for (int q = 0; q < FPL; q++) {
-      if ((q == 0 || many) && ((F.valid >> q) & 1u)) {
-        const int pv = F.verts[q];
-        const int x0 = pv & 0xff, x1 = (pv >> 8) & 0xff, x2 = (pv >> 16) & 0xff;
-        const D3 fn{F.nx[q], F.ny[q], F.nz[q]};
-        if (dot(fn, sub(nv, lds_v(sh, x0))) > kEps64) {
-          vis |= 1u << q;
-          int w0, w1, w2;
-          unsigned b0, b1, b2;
-          edge_place(x0, x1, w0, b0);
-          edge_place(x1, x2, w1, b1);
-          edge_place(x2, x0, w2, b2);
-          const unsigned o0 = lds_or(&sh.met[w0], b0), o1 = lds_or(&sh.met[w1], b1),
-                         o2 = lds_or(&sh.met[w2], b2);
-          if (o0 & b0) lds_or(&sh.again[w0], b0);
-          if (o1 & b1) lds_or(&sh.again[w1], b1);
-          if (o2 & b2) lds_or(&sh.again[w2], b2);
+    int w[3];  // the first slot's edge places; the others' are found again
+    unsigned b[3];
+    if ((F.valid & 1u) &&
+        dot(D3{F.nx, F.ny, F.nz}, sub(nv, lds_v(sh, F.verts & 0xff))) > kEps64) {
+      vis = 1u;
+      face_edges(F.verts, w, b);
+      mark_edges(sh, w, b);
+    }
+    if (many) {
+#pragma clang loop unroll(disable)
+      for (int q = 1; q < FPL; q++) {
+        if ((F.valid >> q) & 1u) {
+          const int k = (q - 1) * LPP + lane;
+          const int pv = sh.verts[k];
+          if (dot(D3{sh.nx[k], sh.ny[k], sh.nz[k]}, sub(nv, lds_v(sh, pv & 0xff))) > kEps64) {
+            vis |= 1u << q;
+            int fw[3];
+            unsigned fb[3];
+            face_edges(pv, fw, fb);
+            mark_edges(sh, fw, fb);
+          }
         }
       }
     }
@@ -543,64 +605,44 @@ OGJK_DEV void epa(const BT& A, const BT& B, Simplex& s, double& distance, Wit& w
     wave_sync();
 
     // horizon = edges met once, in slot order, (v0v1, v1v2, v2v0) within a face
-    int nsurv = 0;
-#pragma unroll
-    for (int q = 0; q < FPL; q++) {
-      if (q == 0 || many) {
-        bool k0 = false, k1 = false, k2 = false;
-        const int pv = F.verts[q];
-        const int x0 = pv & 0xff, x1 = (pv >> 8) & 0xff, x2 = (pv >> 16) & 0xff;
-        if ((vis >> q) & 1u) {
-          int w0, w1, w2;
-          unsigned b0, b1, b2;
-          edge_place(x0, x1, w0, b0);
-          edge_place(x1, x2, w1, b1);
-          edge_place(x2, x0, w2, b2);
-          k0 = !(sh.again[w0] & b0);
-          k1 = !(sh.again[w1] & b1);
-          k2 = !(sh.again[w2] & b2);
-        }
-        const auto m0 = lanes_where<LPP>(k0), m1 = lanes_where<LPP>(k1), m2 = lanes_where<LPP>(k2);
-        int at = nsurv + lanes_below<LPP>(m0, lane) + lanes_below<LPP>(m1, lane) +
-                 lanes_below<LPP>(m2, lane);
-        // at most kEpaMaxFaces slots can take a new face
-        if (k0 && at < kEpaMaxFaces) sh.surv[at] = (unsigned short)(x0 | (x1 << 8));
-        at += k0;
-        if (k1 && at < kEpaMaxFaces) sh.surv[at] = (unsigned short)(x1 | (x2 << 8));
-        at += k1;
-        if (k2 && at < kEpaMaxFaces) sh.surv[at] = (unsigned short)(x2 | (x0 << 8));
-        nsurv += count_lanes<LPP>(m0) + count_lanes<LPP>(m1) + count_lanes<LPP>(m2);
+    int nsurv = keep_edges(sh, (vis & 1u) != 0, F.verts, w, b, 0, lane);
+    if (many) {
+#pragma clang loop unroll(disable)
+      for (int q = 1; q < FPL; q++) {
+        const bool mine = ((vis >> q) & 1u) != 0;
+        const int pv = sh.verts[(q - 1) * LPP + lane];
+        int fw[3];
+        unsigned fb[3];
+        face_edges(mine ? pv : 0x020100, fw, fb);
+        nsurv += keep_edges(sh, mine, pv, fw, fb, nsurv, lane);
       }
     }
     wave_sync();
     // leave the tables clear
-#pragma unroll
-    for (int q = 0; q < FPL; q++) {
-      if ((q == 0 || many) && ((vis >> q) & 1u)) {
-        const int pv = F.verts[q];
-        const int x0 = pv & 0xff, x1 = (pv >> 8) & 0xff, x2 = (pv >> 16) & 0xff;
-        int w0, w1, w2;
-        unsigned b;
-        edge_place(x0, x1, w0, b);
-        edge_place(x1, x2, w1, b);
-        edge_place(x2, x0, w2, b);
-        sh.met[w0] = sh.again[w0] = 0u;
-        sh.met[w1] = sh.again[w1] = 0u;
-        sh.met[w2] = sh.again[w2] = 0u;
+    if (vis & 1u) clear_edges(sh, w);
+    if (many) {
+#pragma clang loop unroll(disable)
+      for (int q = 1; q < FPL; q++) {
+        if ((vis >> q) & 1u) {
+          int fw[3];
+          unsigned fb[3];
+          face_edges(sh.verts[(q - 1) * LPP + lane], fw, fb);
+          clear_edges(sh, fw);
+        }
       }
     }
 
     // fan new faces into the lowest free slots (EPA.c:761-825)
     int taken = 0;
-#pragma unroll
+#pragma clang loop unroll(disable)
     for (int q = 0; q < FPL; q++) {
-      if (q > 0 && __ballot(taken < nsurv) == 0) break;
+      if (__ballot(taken < nsurv) == 0) break;
       const bool fr = !((F.valid >> q) & 1u);
       const auto mf = lanes_where<LPP>(fr);
       const int rank = taken + lanes_below<LPP>(mf, lane);
       if (fr && rank < nsurv) {
         const int ed = sh.surv[rank];
-        put_face(F, q, build_face(sh, ed & 0xff, (ed >> 8) & 0xff, nid, centroid));
+        put_face(sh, F, q, lane, build_face(sh, ed & 0xff, (ed >> 8) & 0xff, nid, centroid));
       }
       taken += count_lanes<LPP>(mf);
     }
@@ -609,8 +651,8 @@ OGJK_DEV void epa(const BT& A, const BT& B, Simplex& s, double& distance, Wit& w
   if (iteration >= kEpaMaxIter) {  // cap fallback (EPA.c:828-863)
     F.valid &= ~F.pend;
     F.pend = 0;
-    const int cf = closest_face<LPP>(F, true, rdist);
-    if (cf >= 0) fetch_face<LPP>(F, cf, true, rn, rdist, rverts);
+    const int cf = closest_face(sh, F, true, lane);
+    if (cf >= 0) fetch_face(sh, F, cf, rn, rdist, rverts);
   }
   simplex_back(sh, s, 4);
   if (rverts >= 0) {

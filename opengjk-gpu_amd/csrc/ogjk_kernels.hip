@@ -379,7 +379,9 @@ template <int LPP, int MODE, class Src>
 __global__ void __launch_bounds__(256) k_pairs(Src src, OutArgs out, int n) {
   constexpr int GPB = 256 / LPP;
   constexpr bool kEpa = (MODE & 2) != 0;
-  __shared__ EpaShared sh[kEpa ? GPB : 1];
+  __shared__ EpaShared<LPP> sh[kEpa ? GPB : 1];
+  __shared__ EpaTable tb;
+  if constexpr (kEpa) epa_table_begin(tb);
   const int lane = threadIdx.x & (LPP - 1);
   const int g = threadIdx.x / LPP;
   const int pair = blockIdx.x * GPB + g;
@@ -402,7 +404,7 @@ __global__ void __launch_bounds__(256) k_pairs(Src src, OutArgs out, int n) {
   }
   if constexpr (kEpa) {
     epa_shared_begin<LPP>(sh[g], lane);
-    epa<LPP>(A, B, s, dist, w, normal, sh[g], lane);
+    epa<LPP>(A, B, s, dist, w, normal, sh[g], tb, lane);
   }
   if (lane == 0) store(out, pair, s, w, dist, normal, kEpa);
 }
@@ -668,7 +670,8 @@ template <int LPP, class Src>
 __global__ void __launch_bounds__(256, Src::template kEpaWaves<LPP>)
     k_epa_list(Src src, OutArgs out, BucketPlan plan, int cls, unsigned* c, const EpaJob* jobs) {
   const int GPB = (int)blockDim.x / LPP;  // groups per block: 1, 2 or 4 waves of them
-  EpaShared* sh = (EpaShared*)ogjk_lds;
+  EpaTable& tb = *(EpaTable*)ogjk_lds;
+  EpaShared<LPP>* sh = (EpaShared<LPP>*)(ogjk_lds + sizeof(EpaTable));
   const int lane = threadIdx.x & (LPP - 1);
   const int g = threadIdx.x / LPP;
   const unsigned njobs =
@@ -676,6 +679,7 @@ __global__ void __launch_bounds__(256, Src::template kEpaWaves<LPP>)
   if (blockIdx.x * GPB >= njobs) return;
   const EpaJob* mine =
       jobs + __builtin_amdgcn_readfirstlane(plan.nb > 1 ? c[kClassStart + cls] : 0u);
+  epa_table_begin(tb);
   epa_shared_begin<LPP>(sh[g], lane);
   int slice = blockIdx.x & (kSlices - 1), tried = 0;
   for (;;) {
@@ -692,7 +696,7 @@ __global__ void __launch_bounds__(256, Src::template kEpaWaves<LPP>)
     typename Src::BodyT A, B;
     src.template load<LPP>(pair, lane, A, B);  // validated by the GJK kernel
     D3 normal{0.0, 0.0, 0.0};
-    epa<LPP>(A, B, s, dist, w, normal, sh[g], lane);
+    epa<LPP>(A, B, s, dist, w, normal, sh[g], tb, lane);
     if (lane == 0) store(out, pair, s, w, dist, normal, true);
   }
 }
@@ -733,7 +737,9 @@ __global__ void __launch_bounds__(256) k_gjk_all(Src src, OutArgs out, int n, Ep
 template <int LPP, class Src>
 __global__ void __launch_bounds__(256) k_epa_all(Src src, OutArgs out, int n, const EpaJob* jobs) {
   constexpr int GPB = 256 / LPP;
-  __shared__ EpaShared sh[GPB];
+  __shared__ EpaShared<LPP> sh[GPB];
+  __shared__ EpaTable tb;
+  epa_table_begin(tb);
   const int lane = threadIdx.x & (LPP - 1);
   const int g = threadIdx.x / LPP;
   const int pair = blockIdx.x * GPB + g;
@@ -746,7 +752,7 @@ __global__ void __launch_bounds__(256) k_epa_all(Src src, OutArgs out, int n, co
   src.template load<LPP>(pair, lane, A, B);  // validated by the GJK kernel
   D3 normal{0.0, 0.0, 0.0};
   epa_shared_begin<LPP>(sh[g], lane);
-  epa<LPP>(A, B, s, dist, w, normal, sh[g], lane);
+  epa<LPP>(A, B, s, dist, w, normal, sh[g], tb, lane);
   if (lane == 0) store(out, pair, s, w, dist, normal, true);
 }
 
@@ -869,6 +875,16 @@ static hipError_t launch_pairs(const Src& src, const OutArgs& o, int n, hipStrea
   return hipGetLastError();
 }
 
+// Lanes per pair of a launch over n pairs: the configured number, doubled while
+// the launch would still leave a SIMD idle (one wave for each, 1,024 on the
+// chip).  Nothing else runs there, so a wider group only shortens its pair's
+// chain: no waiting for the other pairs of the wave and fewer sweep steps.
+constexpr int64_t kChipLanes = 1024 * 64;
+static int fill_lanes(int lanes, int n) {
+  while (lanes < 64 && 2 * (int64_t)lanes * n <= kChipLanes) lanes *= 2;
+  return lanes;
+}
+
 // Resident grid for a persistent launch over at most n items.
 static unsigned persistent_blocks(int n, int gpb, unsigned cap = 4096u) {
   const unsigned want = (unsigned)((n + gpb - 1) / gpb);
@@ -899,7 +915,7 @@ static hipError_t launch_epa_list(const Src& src, const OutArgs& o, int n, const
   const EpaJob* jobs = (const EpaJob*)((char*)ws + ws_jobs_off(n));
   const int gpb = 64 * wpb / LPP;
   hipLaunchKernelGGL((k_epa_list<LPP, Src>), dim3(persistent_blocks(n, gpb, 16384u / wpb)),
-                     dim3(64 * wpb), (size_t)gpb * sizeof(EpaShared), st, src, o, p, cls, c,
+                     dim3(64 * wpb), sizeof(EpaTable) + (size_t)gpb * sizeof(EpaShared<LPP>), st, src, o, p, cls, c,
                      jobs);
   return hipGetLastError();
 }
@@ -917,7 +933,7 @@ static hipError_t gjk_by_lanes(int lanes, const Src& src, const OutArgs& o, int 
 
 template <int MODE, class Src>
 static hipError_t pairs_by_lanes(const Src& src, const OutArgs& o, int n, hipStream_t st) {
-  switch (g_cfg.epa_lanes[0]) {
+  switch (fill_lanes(g_cfg.epa_lanes[0], n)) {
     case 16: return launch_pairs<16, MODE>(src, o, n, st);
     case 32: return launch_pairs<32, MODE>(src, o, n, st);
     default: return launch_pairs<64, MODE>(src, o, n, st);
@@ -929,7 +945,11 @@ static hipError_t pairs_by_lanes(const Src& src, const OutArgs& o, int n, hipStr
 template <class Src>
 static hipError_t launch_bucketed(int mode, const Src& src, const OutArgs& o, int n, void* ws,
                                   hipStream_t st) {
-  const LaunchConfig cfg = g_cfg;
+  LaunchConfig cfg = g_cfg;
+  for (int b = 0; b < cfg.nb; b++) {
+    cfg.gjk_lanes[b] = fill_lanes(cfg.gjk_lanes[b], n);
+    cfg.epa_lanes[b] = fill_lanes(cfg.epa_lanes[b], n);
+  }
   const BucketPlan p = plan_of(cfg);
   unsigned* c = (unsigned*)ws;
   // GJK alone over a single bucket reads and writes no counter (no

@@ -90,6 +90,11 @@ OGJK_DEV int lanes_below(lane_mask<LPP> m, int l) {
 }
 
 template <int LPP>
+OGJK_DEV int lane_in() {
+  return lane_id() & (LPP - 1);
+}
+
+template <int LPP>
 OGJK_DEV bool group_any(bool p) {
   return group_ballot<LPP>(p) != 0;
 }
@@ -211,6 +216,12 @@ OGJK_DEV void both_halves(double v, double& lo, double& hi) {
   hi = __builtin_bit_cast(double, ((uint64_t)(uint32_t)hi1 << 32) | (uint32_t)lo1);
 }
 
+// The value of a wave-uniform lane, without an LDS round trip.
+OGJK_DEV int lane_value(int v, int src) { return __builtin_amdgcn_readlane(v, src); }
+OGJK_DEV float lane_value(float v, int src) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), src));
+}
+
 template <int LPP>
 OGJK_DEV double shfl_d(double v, int src) {
   return __shfl(v, src, LPP);
@@ -236,16 +247,33 @@ OGJK_DEV float group_max_f(float v) {
   }
 }
 
-// Min over the group (no NaN).
 template <int LPP, int M = 1>
-OGJK_DEV double group_min_d(double v) {
+OGJK_DEV uint32_t group_min_u(uint32_t v) {
   if constexpr (M < LPP) {
-    double a, b;
-    xpair<M>(v, a, b);
-    return group_min_d<LPP, 2 * M>(b < a ? b : a);
+    int a, b;
+    xpair<M>((int)v, a, b);
+    return group_min_u<LPP, 2 * M>(min((uint32_t)a, (uint32_t)b));
   } else {
     return v;
   }
+}
+
+// The lanes that hold the group's least value, for values >= 0 (or +inf, no
+// NaN; the two zeros are equal): such doubles order as their bit patterns, so
+// one 32-bit reduction over the high words decides unless several lanes share
+// the least.
+template <int LPP>
+OGJK_DEV lane_mask<LPP> lanes_of_least(double v) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v + 0.0);  // -0 -> +0
+  const uint32_t hi = (uint32_t)(u >> 32);
+  const bool first = hi == group_min_u<LPP>(hi);
+  lane_mask<LPP> m = lanes_where<LPP>(first);
+  if (count_lanes<LPP>(m) > 1) {
+    const uint32_t lo = first ? (uint32_t)u : 0xffffffffu;
+    const uint32_t least = group_min_u<LPP>(lo);  // by every lane of the group
+    m = lanes_where<LPP>(first && lo == least);
+  }
+  return m;
 }
 
 // Max of (value, index) with the lowest index winning ties.  NaN values must
@@ -261,21 +289,6 @@ OGJK_DEV void group_argmax_d(double& v, int& i) {
     v = tb ? vb : va;
     i = tb ? ib : ia;
     group_argmax_d<LPP, 2 * M>(v, i);
-  }
-}
-
-// Min of (value, index), lowest index on ties; NaN must be mapped to +inf.
-template <int LPP, int M = 1>
-OGJK_DEV void group_argmin_d(double& v, int& i) {
-  if constexpr (M < LPP) {
-    double va, vb;
-    int ia, ib;
-    xpair<M>(v, va, vb);
-    xpair<M>(i, ia, ib);
-    const bool tb = vb < va || (vb == va && ib < ia);  // symmetric in (a, b)
-    v = tb ? vb : va;
-    i = tb ? ib : ia;
-    group_argmin_d<LPP, 2 * M>(v, i);
   }
 }
 

@@ -37,19 +37,27 @@ def _join(batches):
 
 
 def _exact(torch, b, shape, cluster_min=None):
+    # launches that would leave SIMDs idle use wider groups than configured:
+    # as it is, and repeated until the configured ones run
     ref = oracle_run(oracle.GJK_EPA, b)
-    ogjk.set_config(*shape, 0)
-    try:
-        sc = ogjk.DeviceScene(b)
-        if cluster_min is not None:
-            sc.build_clusters(cluster_min)
-        out = sc.collide(oracle.GJK_EPA, b.n_pairs, f64_record=True)
-        torch.cuda.synchronize()
-    finally:
-        ogjk.set_config(8, 32, 0)
-    res = compare_f64(out["f64"].cpu().numpy(), ogjk.simplices_from_device(out["simplices"]), ref,
-                      oracle.GJK_EPA)
-    assert res["exact"] == res["n"], res
+    once = np.stack([b.pa, b.pb], 1).astype(np.int32)
+    for reps in (1, 1 + 65536 // (2 * shape[0] * b.n_pairs)):
+        pairs = torch.from_numpy(np.ascontiguousarray(np.tile(once, (reps, 1)))).cuda()
+        ogjk.set_config(*shape, 0)
+        try:
+            sc = ogjk.DeviceScene(b)
+            if cluster_min is not None:
+                sc.build_clusters(cluster_min)
+            out = sc.collide(oracle.GJK_EPA, len(pairs), pairs=pairs, f64_record=True)
+            torch.cuda.synchronize()
+        finally:
+            ogjk.set_config(8, 32, 0)
+        rec = out["f64"].cpu().numpy()
+        simp = ogjk.simplices_from_device(out["simplices"])
+        for k in range(reps):
+            at = slice(k * b.n_pairs, (k + 1) * b.n_pairs)
+            res = compare_f64(rec[at], simp[at], ref, oracle.GJK_EPA)
+            assert res["exact"] == res["n"], (reps, k, res)
     assert (ref.distances < 0).any()
 
 
