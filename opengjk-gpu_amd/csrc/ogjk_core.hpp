@@ -1005,16 +1005,6 @@ OGJK_DEV int sb(const Simplex& s, int k) {
             b3 = keep_reg(s.ib[3]);
   return k == 0 ? b0 : (k == 1 ? b1 : (k == 2 ? b2 : b3));
 }
-// Write slot k: every slot is rewritten with a value select (no address select).
-OGJK_DEV void sset(Simplex& s, int k, D3 p, int a, int b) {
-#pragma unroll
-  for (int t = 0; t < 4; t++) {
-    const bool h = (k == t);
-    s.p[t] = sel(h, p, keep_reg(s.p[t]));
-    s.ia[t] = h ? a : keep_reg(s.ia[t]);
-    s.ib[t] = h ? b : keep_reg(s.ib[t]);
-  }
-}
 template <int DST, int SRC>
 OGJK_DEV void smove(Simplex& s) {
   s.p[DST] = s.p[SRC];
@@ -1022,338 +1012,169 @@ OGJK_DEV void smove(Simplex& s) {
   s.ib[DST] = s.ib[SRC];
 }
 
-struct Pt {  // a simplex vertex with its pair of body indices
-  D3 p;
+// ---------------------------------------------------- sub-distance (FP64)
+//
+// S1D, S2D and S3D (GJK/cpu/openGJK.c:257-613) as one straight piece of code.
+// Written as the reference's tree, with a projection at each of some twenty
+// leaves, a wave of eight pairs walked nearly all of it in every iteration.  All
+// leaves are of four kinds: keep the newest vertex s1, project on the line to
+// one older vertex, on the plane through two, or stop inside.  So every
+// predicate is evaluated once, from the edges e_x = q_x - s1 and their cross
+// products, the tree is walked over the resulting bits, and one projection is
+// made at the end, with one division.
+//
+// The values are the reference's bit for bit:
+//   hff2(s1, x, y) = s1.(e_x x (e_x x e_y)) < 0, and e_y x e_x is the exact
+//   negative of e_x x e_y, so both orders of a pair share one cross product;
+//   projectOnPlane's normal (s1 - x) x (s1 - y) is e_x x e_y, and
+//   projectOnLine's s1 - x is -e_x: a sign on both factors of X * t;
+//   the determinant of (e_1, e_0, e_2) is -(e_1 . (e_2 x e_0)).
+// (A zero component of v may take the other sign; no output depends on it.)
+//
+// The simplex itself is in LDS: four places, and a map of its slots to places
+// (2 bits each), so that the reference's copies between slots, which leave the
+// old vertices in the slots above the count, are changes of the map.
+
+struct SimplexVertex {
+  double x, y, z;
   int a, b;
 };
-OGJK_DEV Pt spt(const Simplex& s, int k) { return Pt{sp(s, k), sa(s, k), sb(s, k)}; }
+struct GjkShared {
+  SimplexVertex v[4];
+  int pad[4];  // neighbouring groups' vertices fall on other banks
+};
 
-// select_1ik / 1ij / 1jk (GJK/cpu/openGJK.c:53-78): {newest, a, b}
-OGJK_DEV void keep3(Simplex& s, const Pt& a, const Pt& b) {
-  s.n = 3;
-  smove<2, 3>(s);
-  s.p[1] = a.p; s.ia[1] = a.a; s.ib[1] = a.b;
-  s.p[0] = b.p; s.ia[0] = b.a; s.ib[0] = b.b;
-}
-// select_1i / 1j / 1k (GJK/cpu/openGJK.c:80-99): {newest, a}
-OGJK_DEV void keep2(Simplex& s, const Pt& a) {
-  s.n = 2;
-  smove<1, 3>(s);
-  s.p[0] = a.p; s.ia[0] = a.a; s.ib[0] = a.b;
+OGJK_DEV D3 point(const SimplexVertex& v) { return D3{v.x, v.y, v.z}; }
+
+// hff1: GJK/cpu/openGJK.c:219-230
+OGJK_DEV bool hff1(D3 p, D3 q) {
+  return (p.x * p.x - p.x * q.x) + (p.y * p.y - p.y * q.y) + (p.z * p.z - p.z * q.z) > 0;
 }
 
-// ------------------------------------------------------- predicates (FP64)
+OGJK_DEV int map_at(int map, int slot) { return (map >> (2 * slot)) & 3; }
+OGJK_DEV int map_set(int map, int slot, int place) {
+  return (map & ~(3 << (2 * slot))) | (place << (2 * slot));
+}
 
-// determinant: GJK/cpu/openGJK.c:167-173
-OGJK_DEV double det3(D3 p, D3 q, D3 r) {
-  return p.x * ((q.y * r.z) - (r.y * q.z)) - p.y * (q.x * r.z - r.x * q.z) +
-         p.z * (q.x * r.y - r.x * q.y);
-}
-// projectOnLine: GJK/cpu/openGJK.c:183-196
-OGJK_DEV D3 proj_line(D3 p, D3 q) {
-  const D3 pq = sub(p, q);
-  const double t = dot(p, pq) / dot(pq, pq);
-  return D3{p.x - pq.x * t, p.y - pq.y * t, p.z - pq.z * t};
-}
-// projectOnPlane: GJK/cpu/openGJK.c:198-217
-OGJK_DEV D3 proj_plane(D3 p, D3 q, D3 r) {
-  const D3 n = cross(sub(p, q), sub(p, r));
-  const double t = dot(n, p) / dot(n, n);
-  return D3{n.x * t, n.y * t, n.z * t};
-}
-// hff1: GJK/cpu/openGJK.c:219-230 (sum starts at 0, as in the reference)
-OGJK_DEV int hff1(D3 p, D3 q) {
-  double t = 0;
-  t += (p.x * p.x - p.x * q.x);
-  t += (p.y * p.y - p.y * q.y);
-  t += (p.z * p.z - p.z * q.z);
-  return t > 0;
-}
-// hff2: GJK/cpu/openGJK.c:232-248
-OGJK_DEV int hff2(D3 p, D3 q, D3 r) {
-  const D3 pq = sub(q, p);
-  const D3 nt = cross(pq, sub(r, p));
-  const D3 n = cross(pq, nt);
-  return dot(p, n) < 0;
-}
-// hff3: GJK/cpu/openGJK.c:250-255
-OGJK_DEV int hff3(D3 p, D3 q, D3 r) { return dot(p, cross(q, r)) <= 0; }
+// x for label 0, 1, 2 of q[]
+OGJK_DEV D3 sel3(int x, D3 q0, D3 q1, D3 q2) { return sel(x == 0, q0, sel(x == 1, q1, q2)); }
 
-// ------------------------------------------------------- S1D / S2D / S3D
+// The tree of S3D below "origin outside" (openGJK.c:390-608) over the bits of
+// its predicates, for one or no face plane containing the origin's side.  H:
+// hff1 of the older vertices; F bit x: hff2(s1, x, x - 1 mod 3); G bit x: hff2(s1, x,
+// x + 1 mod 3); k: the reference's k (i = k - 1, j = k + 1 mod 3).  Returns x | y
+// << 2 | kind << 4 with kind 2: line to x, 3: plane through x and y (slots 1 and
+// 0 of the triangle).
+OGJK_DEV int s3d_leaf(int H, int F, int G, int k, bool one_plane) {
+  const int i = k == 0 ? 2 : k - 1, j = k == 2 ? 0 : k + 1;
+  const bool hk = (H >> k) & 1, hi = (H >> i) & 1;
+  const bool Tki = (F >> k) & 1, Tjk = (F >> j) & 1, Tij = (F >> i) & 1;
+  const bool Tkj = (G >> k) & 1, Tji = (G >> j) & 1, Tik = (G >> i) & 1;
+  const int Lk = k | 32, Li = i | 32, Lj = j | 32;
+  const int Pik = i | (k << 2) | 48, Pjk = j | (k << 2) | 48, Pij = i | (j << 2) | 48;
+  const int dt = __popc((unsigned)H);
+  const int one = dt == 1 ? (hk ? (!Tki ? Pik : (!Tkj ? Pjk : Lk))
+                                : (hi ? (!Tik ? Pik : Li) : (!Tjk ? Pjk : Lj)))
+                : dt == 2 ? (hi ? (!Tki ? (!Tik ? Pik : Lk) : (!Tkj ? Pjk : Lk))
+                                : (!Tkj ? (!Tjk ? Pjk : Lj) : (!Tki ? Pik : Lk)))
+                          : (Tki ? (Tkj ? Lk : (Tjk ? Lj : Pjk)) : (Tik ? Li : Pik));
+  const int none = dt == 1 ? (!Tij ? Pij : (!Tik ? Pik : Li))
+                           : (!Tjk ? (!Tkj ? Pjk : (!Tki ? Pik : Lk)) : (!Tji ? Pij : Lj));
+  return one_plane ? one : none;
+}
 
-// S1D: GJK/cpu/openGJK.c:257-268
-OGJK_DEV void S1D(Simplex& s, D3& v) {
-  if (hff1(s.p[1], s.p[0])) {
-    v = proj_line(s.p[1], s.p[0]);
+// subalgorithm (openGJK.c:641-656) after vertex s1 (place f) joined the n older
+// ones: n, map and v are updated.
+OGJK_DEV void subdistance(const GjkShared& sh, D3 s1, int f, int& n, int& map, D3& v) {
+  const D3 q0 = point(sh.v[map_at(map, 0)]), q1 = point(sh.v[map_at(map, 1)]),
+           q2 = point(sh.v[map_at(map, 2)]);
+  const D3 e0 = sub(q0, s1), e1 = sub(q1, s1), e2 = sub(q2, s1);
+  int H = hff1(s1, q0) ? 1 : 0;
+  // kind 0: v and the simplex stay, 1: s1 alone, 2: line to x, 3: plane x, y,
+  // 4: inside.  tri: the reference reduced a tetrahedron to the triangle (s1, a, b)
+  // first, or it was one.
+  int kind, x = 0, y = 0, a = 1, b = 0;
+  bool tri = n == 2;
+  D3 c10 = e0, c20 = e0, c21 = e0;
+  if (n == 1) {
+    kind = H ? 2 : 1;  // S1D
   } else {
-    v = s.p[1];
-    s.n = 1;
-    smove<0, 1>(s);
-  }
-}
-
-// S2D: GJK/cpu/openGJK.c:270-313
-OGJK_DEV void S2D(Simplex& s, D3& v) {
-  const D3 s1 = s.p[2], s2 = s.p[1], s3 = s.p[0];
-  const int h12 = hff1(s1, s2);
-  const int h13 = hff1(s1, s3);
-  if (h12) {
-    if (!hff2(s1, s2, s3)) {
-      if (h13) {
-        if (!hff2(s1, s3, s2)) {
-          v = proj_plane(s1, s2, s3);
-        } else {
-          v = proj_line(s1, s3);
-          s.n = 2;
-          smove<1, 2>(s);
-        }
-      } else {
-        v = proj_plane(s1, s2, s3);
+    H |= hff1(s1, q1) ? 2 : 0;
+    c10 = cross(e1, e0);
+    const bool T10 = dot(s1, cross(e1, c10)) < 0, T01 = dot(s1, cross(e0, c10)) > 0;
+    bool Ta = T10, Tb = T01;
+    kind = 0;
+    if (n == 3) {
+      H |= hff1(s1, q2) ? 4 : 0;
+      c20 = cross(e2, e0);
+      c21 = cross(e2, e1);
+      const bool T20 = dot(s1, cross(e2, c20)) < 0, T02 = dot(s1, cross(e0, c20)) > 0;
+      const bool T21 = dot(s1, cross(e2, c21)) < 0, T12 = dot(s1, cross(e1, c21)) > 0;
+      const bool sss = dot(e1, c20) >= 0;
+      const bool p2 = (dot(s1, cross(q1, q0)) <= 0) != sss;
+      const bool p3 = (dot(s1, cross(q0, q2)) <= 0) != sss;
+      const bool p4 = (dot(s1, cross(q2, q1)) <= 0) != sss;
+      const int planes = (int)p2 + (int)p3 + (int)p4;
+      const int dt = __popc((unsigned)H);
+      if (dt == 0) {
+        kind = 1;
+      } else if (planes == 3) {
+        kind = 4;
+      } else if (planes == 2) {
+        tri = true;
+        a = !p2 ? 1 : 2;
+        b = !p4 ? 1 : 0;
+        Ta = !p2 ? T10 : (!p3 ? T20 : T21);
+        Tb = !p2 ? T01 : (!p3 ? T02 : T12);
+      } else if (planes == 1 || dt != 3) {
+        const int F = (T02 ? 1 : 0) | (T10 ? 2 : 0) | (T21 ? 4 : 0);
+        const int G = (T01 ? 1 : 0) | (T12 ? 2 : 0) | (T20 ? 4 : 0);
+        const bool h0 = H & 1, h1 = H & 2;
+        const int k = planes == 1 ? (p2 ? 2 : (p3 ? 1 : 0))
+                                  : (dt == 1 ? (h1 ? 2 : (h0 ? 1 : 0)) : (!h1 ? 2 : (!h0 ? 1 : 0)));
+        const int leaf = s3d_leaf(H, F, G, k, planes == 1);
+        x = leaf & 3;
+        y = (leaf >> 2) & 3;
+        kind = leaf >> 4;
       }
-    } else {
-      v = proj_line(s1, s2);
-      s.n = 2;
-      smove<0, 2>(s);
     }
-  } else if (h13) {
-    if (!hff2(s1, s3, s2)) {
-      v = proj_plane(s1, s2, s3);
-    } else {
-      v = proj_line(s1, s3);
-      s.n = 2;
-      smove<1, 2>(s);
+    if (tri) {  // S2D over (s1, a, b)
+      const bool ha = (H >> a) & 1, hb = (H >> b) & 1;
+      x = a;
+      y = b;
+      kind = !(ha || hb) ? 1 : (ha && Ta ? 2 : (hb && Tb ? 2 : 3));
+      if (kind == 2 && !(ha && Ta)) x = b;
     }
-  } else {
-    v = s.p[2];
-    s.n = 1;
-    smove<0, 2>(s);
   }
-}
-
-// S3D: GJK/cpu/openGJK.c:315-613.  (k, i, j) name the three older vertices
-// with k opposite the face under test, as in the reference.
-OGJK_DEV void S3D(Simplex& s, D3& v) {
-  const Pt P1{s.p[3], s.ia[3], s.ib[3]};
-  const D3 s1 = P1.p, s2 = s.p[2], s3 = s.p[1], s4 = s.p[0];
-  const Pt P2{s2, s.ia[2], s.ib[2]};
-  const Pt P3{s3, s.ia[1], s.ib[1]};
-  const D3 s1s2 = sub(s2, s1), s1s3 = sub(s3, s1), s1s4 = sub(s4, s1);
-
-  const int h1_2 = hff1(s1, s2);
-  const int h1_1 = hff1(s1, s3);
-  const int h1_0 = hff1(s1, s4);
-  const int line3 = h1_1, line4 = h1_0;
-  const int dot_total = h1_2 + line3 + line4;
-
-  if (dot_total == 0) {
-    v = s1;
-    s.n = 1;
-    s.p[0] = s1; s.ia[0] = P1.a; s.ib[0] = P1.b;
+  if (kind == 0) {  // outside all faces and towards every vertex: no branch there
+    n = 4;
     return;
   }
 
-  const double det134 = det3(s1s3, s1s4, s1s2);
-  const int sss = (det134 <= 0);
-  int p2 = hff3(s1, s3, s4) - sss;
-  p2 = p2 * p2;
-  int p3 = hff3(s1, s4, s2) - sss;
-  p3 = p3 * p3;
-  int p4 = hff3(s1, s2, s3) - sss;
-  p4 = p4 * p4;
-  const int planes = p2 + p3 + p4;
+  // the one projection: X the edge, or the plane's normal
+  const int other = 3 - x - y;  // of a plane's pair: the vertex left out
+  const D3 X = sel(kind == 3, sel3(other, c21, c20, c10), sel3(x, e0, e1, e2));
+  const double t = dot(s1, X) / dot(X, X);
+  const D3 Xt{X.x * t, X.y * t, X.z * t};
+  v = kind == 3 ? Xt : (kind == 2 ? sub(s1, Xt) : (kind == 1 ? s1 : D3{0.0, 0.0, 0.0}));
 
-  if (planes == 3) {
-    v = D3{0.0, 0.0, 0.0};
-    s.n = 4;
-    return;
+  // the slots, as the reference leaves them
+  const int px = map_at(map, x), py = map_at(map, y);
+  if (n == 1) {
+    if (kind == 1) map = map_set(map, 0, f);
+  } else if (tri) {
+    const int pa = map_at(map, a), pb = map_at(map, b);
+    map = map_set(map_set(map_set(map, 2, f), 1, pa), 0, pb);
+    if (kind == 1 || (kind == 2 && x == a)) map = map_set(map, 0, f);
+    if (kind == 2 && x == b) map = map_set(map, 1, f);
+  } else if (kind == 3) {
+    map = map_set(map_set(map_set(map, 2, f), 1, px), 0, py);
+  } else if (kind == 2) {
+    map = map_set(map_set(map, 1, f), 0, px);
+  } else if (kind == 1) {
+    map = map_set(map, 0, f);
   }
-  if (planes == 2) {
-    s.n = 3;
-    if (!p2) {
-      smove<2, 3>(s);
-    } else if (!p3) {
-      s.p[1] = P2.p; s.ia[1] = P2.a; s.ib[1] = P2.b;
-      smove<2, 3>(s);
-    } else if (!p4) {
-      s.p[0] = P3.p; s.ia[0] = P3.a; s.ib[0] = P3.b;
-      s.p[1] = P2.p; s.ia[1] = P2.a; s.ib[1] = P2.b;
-      smove<2, 3>(s);
-    }
-    S2D(s, v);
-    return;
-  }
-  if (planes == 1) {
-    s.n = 3;
-    int k, i, j;
-    if (p2) {
-      k = 2; i = 1; j = 0;
-    } else if (p3) {
-      k = 1; i = 0; j = 2;
-    } else {
-      k = 0; i = 2; j = 1;
-    }
-    const Pt si = spt(s, i), sj = spt(s, j), sk = spt(s, k);
-    const int hk = (k == 2) ? h1_2 : (k == 1 ? h1_1 : h1_0);
-    const int hi = (i == 2) ? h1_2 : (i == 1 ? h1_1 : h1_0);
-    const int hj = (j == 2) ? h1_2 : (j == 1 ? h1_1 : h1_0);
-    if (dot_total == 1) {
-      if (hk) {
-        if (!hff2(s1, sk.p, si.p)) {
-          keep3(s, si, sk);
-          v = proj_plane(s1, si.p, sk.p);
-        } else if (!hff2(s1, sk.p, sj.p)) {
-          keep3(s, sj, sk);
-          v = proj_plane(s1, sj.p, sk.p);
-        } else {
-          keep2(s, sk);
-          v = proj_line(s1, sk.p);
-        }
-      } else if (hi) {
-        if (!hff2(s1, si.p, sk.p)) {
-          keep3(s, si, sk);
-          v = proj_plane(s1, si.p, sk.p);
-        } else {
-          keep2(s, si);
-          v = proj_line(s1, si.p);
-        }
-      } else {
-        if (!hff2(s1, sj.p, sk.p)) {
-          keep3(s, sj, sk);
-          v = proj_plane(s1, sj.p, sk.p);
-        } else {
-          keep2(s, sj);
-          v = proj_line(s1, sj.p);
-        }
-      }
-    } else if (dot_total == 2) {
-      if (hi) {
-        if (!hff2(s1, sk.p, si.p)) {
-          if (!hff2(s1, si.p, sk.p)) {
-            keep3(s, si, sk);
-            v = proj_plane(s1, si.p, sk.p);
-          } else {
-            keep2(s, sk);
-            v = proj_line(s1, sk.p);
-          }
-        } else {
-          if (!hff2(s1, sk.p, sj.p)) {
-            keep3(s, sj, sk);
-            v = proj_plane(s1, sj.p, sk.p);
-          } else {
-            keep2(s, sk);
-            v = proj_line(s1, sk.p);
-          }
-        }
-      } else if (hj) {
-        if (!hff2(s1, sk.p, sj.p)) {
-          if (!hff2(s1, sj.p, sk.p)) {
-            keep3(s, sj, sk);
-            v = proj_plane(s1, sj.p, sk.p);
-          } else {
-            keep2(s, sj);
-            v = proj_line(s1, sj.p);
-          }
-        } else {
-          if (!hff2(s1, sk.p, si.p)) {
-            keep3(s, si, sk);
-            v = proj_plane(s1, si.p, sk.p);
-          } else {
-            keep2(s, sk);
-            v = proj_line(s1, sk.p);
-          }
-        }
-      }
-      // else: no region; v and the 3-vertex prefix stay (openGJK.c:494-496)
-    } else {  // dot_total == 3
-      const int h2ik = hff2(s1, si.p, sk.p);
-      const int h2jk = hff2(s1, sj.p, sk.p);
-      const int h2ki = hff2(s1, sk.p, si.p);
-      const int h2kj = hff2(s1, sk.p, sj.p);
-      if (h2ki == 1 && h2kj == 1) {
-        keep2(s, sk);
-        v = proj_line(s1, sk.p);
-      } else if (h2ki) {
-        if (h2jk) {
-          keep2(s, sj);
-          v = proj_line(s1, sj.p);
-        } else {
-          keep3(s, sj, sk);
-          v = proj_plane(s1, sk.p, sj.p);
-        }
-      } else {
-        if (h2ik) {
-          keep2(s, si);
-          v = proj_line(s1, si.p);
-        } else {
-          keep3(s, si, sk);
-          v = proj_plane(s1, sk.p, si.p);
-        }
-      }
-    }
-    return;
-  }
-  // planes == 0: origin outside all three faces (openGJK.c:538-608)
-  if (dot_total == 1) {
-    int k, i, j;
-    if (line3) {
-      k = 2; i = 1; j = 0;
-    } else if (line4) {
-      k = 1; i = 0; j = 2;
-    } else {
-      k = 0; i = 2; j = 1;
-    }
-    const Pt si = spt(s, i), sj = spt(s, j), sk = spt(s, k);
-    if (!hff2(s1, si.p, sj.p)) {
-      keep3(s, si, sj);
-      v = proj_plane(s1, si.p, sj.p);
-    } else if (!hff2(s1, si.p, sk.p)) {
-      keep3(s, si, sk);
-      v = proj_plane(s1, si.p, sk.p);
-    } else {
-      keep2(s, si);
-      v = proj_line(s1, si.p);
-    }
-  } else if (dot_total == 2) {
-    s.n = 3;
-    int k, i, j;
-    if (!line3) {
-      k = 2; i = 1; j = 0;
-    } else if (!line4) {
-      k = 1; i = 0; j = 2;
-    } else {
-      k = 0; i = 2; j = 1;
-    }
-    const Pt si = spt(s, i), sj = spt(s, j), sk = spt(s, k);
-    if (!hff2(s1, sj.p, sk.p)) {
-      if (!hff2(s1, sk.p, sj.p)) {
-        keep3(s, sj, sk);
-        v = proj_plane(s1, sj.p, sk.p);
-      } else if (!hff2(s1, sk.p, si.p)) {
-        keep3(s, si, sk);
-        v = proj_plane(s1, sk.p, si.p);
-      } else {
-        keep2(s, sk);
-        v = proj_line(s1, sk.p);
-      }
-    } else if (!hff2(s1, sj.p, si.p)) {
-      keep3(s, si, sj);
-      v = proj_plane(s1, si.p, sj.p);
-    } else {
-      keep2(s, sj);
-      v = proj_line(s1, sj.p);
-    }
-  }
-  // dot_total == 3 with planes == 0: nothing (the reference has no branch)
-}
-
-// subalgorithm: GJK/cpu/openGJK.c:641-656
-OGJK_DEV void subalgorithm(Simplex& s, D3& v) {
-  if (s.n == 4)
-    S3D(s, v);
-  else if (s.n == 3)
-    S2D(s, v);
-  else if (s.n == 2)
-    S1D(s, v);
+  n = kind;  // 1, 2, 3 or 4 vertices
 }
 
 // ------------------------------------------------------- witnesses W*D
@@ -1487,7 +1308,7 @@ OGJK_DEV void witnesses(const BT& A, const BT& B, Simplex& s, Wit& w) {
 
 // compute_minimum_distance: GJK/cpu/openGJK.c:952-1056.  Returns ||v||.
 template <int LPP, class BT>
-OGJK_DEV double gjk(const BT& A, const BT& B, Simplex& s, Wit& w, int lane) {
+OGJK_DEV double gjk(const BT& A, const BT& B, Simplex& s, Wit& w, GjkShared& sh, int lane) {
   const double eps_rel = kEps64 * 1e4;  // (gkFloat)DBL_EPSILON * 1e4f
   const double eps_tot = kEps64 * 1e2;
   const double eps_rel2 = eps_rel * eps_rel;
@@ -1495,10 +1316,12 @@ OGJK_DEV double gjk(const BT& A, const BT& B, Simplex& s, Wit& w, int lane) {
   D3 pa = A.d(0), pb = B.d(0);
   int ia = 0, ib = 0;
   D3 v = sub(pa, pb);
-  s.n = 1;
-  s.p[0] = v;
-  s.ia[0] = 0;
-  s.ib[0] = 0;
+  int n = 1, map = 0xE4;  // slot i in place i
+  if (lane == 0) {
+    sh.v[0] = SimplexVertex{v.x, v.y, v.z, 0, 0};
+    for (int k = 1; k < 4; k++) sh.v[k] = SimplexVertex{0.0, 0.0, 0.0, 0, 0};
+  }
+  const double n0 = norm2(v);
   double norm2Wmax = 0.0;
   unsigned k = 0;
   do {
@@ -1514,20 +1337,35 @@ OGJK_DEV double gjk(const BT& A, const BT& B, Simplex& s, Wit& w, int lane) {
     if (gap <= eps_rel * norm2(v) || gap < eps_tot) break;
     if (norm2(v) < eps_rel2) break;
 
-    sset(s, s.n, wv, ia, ib);
-    s.n++;
-    subalgorithm(s, v);
-
+    // slot n gets the new vertex, in a place that no other slot names
+    int used = 0;
 #pragma unroll
-    for (int jj = 0; jj < 4; jj++) {
-      if (jj < s.n) {
-        const double tn = norm2(s.p[jj]);
-        if (tn > norm2Wmax) norm2Wmax = tn;
-      }
-    }
-    if (norm2(v) <= eps_tot * eps_tot * norm2Wmax) break;
-  } while (s.n != 4 && k != 25u);
+    for (int t = 0; t < 4; t++) used |= t == n ? 0 : 1 << map_at(map, t);
+    const int f = __builtin_ctz(~(unsigned)used);
+    wave_sync();
+    if (lane == 0) sh.v[f] = SimplexVertex{wv.x, wv.y, wv.z, ia, ib};
+    map = map_set(map, n, f);
+    wave_sync();
+    subdistance(sh, wv, f, n, map, v);
 
+    // the largest vertex of any simplex so far: the newest vertex always stays,
+    // the older ones were counted when they were new, the first one in the
+    // first turn if it stayed
+    const double tn = norm2(wv);
+    if (k == 1u && n == 2 && n0 > norm2Wmax) norm2Wmax = n0;
+    if (tn > norm2Wmax) norm2Wmax = tn;
+    if (norm2(v) <= eps_tot * eps_tot * norm2Wmax) break;
+  } while (n != 4 && k != 25u);
+
+  wave_sync();
+  s.n = n;
+#pragma unroll
+  for (int t = 0; t < 4; t++) {
+    const SimplexVertex& q = sh.v[map_at(map, t)];
+    s.p[t] = point(q);
+    s.ia[t] = q.a;
+    s.ib[t] = q.b;
+  }
   witnesses(A, B, s, w);
   return sqrt(norm2(v));
 }

@@ -54,11 +54,6 @@ struct EpaTable {
   double inv[kEpaMaxIter];
 };
 
-OGJK_DEV void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 // Clears the edge tables: once before a group's first pair (epa() leaves them
 // clear).
 template <int LPP>

@@ -380,6 +380,7 @@ __global__ void __launch_bounds__(256) k_pairs(Src src, OutArgs out, int n) {
   constexpr int GPB = 256 / LPP;
   constexpr bool kEpa = (MODE & 2) != 0;
   __shared__ EpaShared<LPP> sh[kEpa ? GPB : 1];
+  __shared__ GjkShared gs[(MODE & 1) ? GPB : 1];
   __shared__ EpaTable tb;
   if constexpr (kEpa) epa_table_begin(tb);
   const int lane = threadIdx.x & (LPP - 1);
@@ -398,7 +399,7 @@ __global__ void __launch_bounds__(256) k_pairs(Src src, OutArgs out, int n) {
   double dist = 0.0;
   D3 normal{0.0, 0.0, 0.0};
   if constexpr ((MODE & 1) != 0) {
-    dist = gjk<LPP>(A, B, s, w, lane);
+    dist = gjk<LPP>(A, B, s, w, gs[g], lane);
   } else {
     load_input(out, pair, A, B, s, w, dist);
   }
@@ -646,12 +647,13 @@ __global__ void __launch_bounds__(256, Src::kGjkWaves)
     return;
   }
   if constexpr (Src::kStage) {
-    float* stg = (float*)ogjk_lds + (threadIdx.x / LPP) * (3 * kStageGjk);
+    float* stg = (float*)(ogjk_lds + GPB * sizeof(GjkShared)) +
+                 (threadIdx.x / LPP) * (3 * kStageGjk);
     stage_pair<LPP, kStageGjk>(A, B, stg, lane);
   }
   Simplex s = {};
   Wit w = {};
-  const double dist = gjk<LPP>(A, B, s, w, lane);
+  const double dist = gjk<LPP>(A, B, s, w, ((GjkShared*)ogjk_lds)[threadIdx.x / LPP], lane);
   const bool pen = EMIT && !(dist > kEps64);
   const int cls = plan.epa_class[bucket];
   const unsigned k = wave_fetch_add(job_counter(c, cls), lane == 0 && pen);
@@ -710,6 +712,7 @@ __global__ void __launch_bounds__(256, Src::template kEpaWaves<LPP>)
 template <int LPP, bool EMIT, class Src>
 __global__ void __launch_bounds__(256) k_gjk_all(Src src, OutArgs out, int n, EpaJob* jobs) {
   constexpr int GPB = 256 / LPP;
+  __shared__ GjkShared gs[GPB];
   const int lane = threadIdx.x & (LPP - 1);
   const int pair = blockIdx.x * GPB + threadIdx.x / LPP;
   if (pair >= n) return;
@@ -724,7 +727,7 @@ __global__ void __launch_bounds__(256) k_gjk_all(Src src, OutArgs out, int n, Ep
   }
   Simplex s = {};
   Wit w = {};
-  const double dist = gjk<LPP>(A, B, s, w, lane);
+  const double dist = gjk<LPP>(A, B, s, w, gs[threadIdx.x / LPP], lane);
   if (lane != 0) return;
   if (EMIT && !(dist > kEps64)) {
     job_store(jobs + pair, pair, s, w, dist);
@@ -900,7 +903,8 @@ static hipError_t launch_gjk(const Src& src, const OutArgs& o, int n, const Buck
   const int* list = (const int*)((char*)ws + ws_list_off());
   EpaJob* jobs = (EpaJob*)((char*)ws + ws_jobs_off(n));
   const int gpb = 64 * wpb / LPP;
-  const size_t lds = Src::kStage ? (size_t)gpb * 3 * kStageGjk * sizeof(float) : 0;
+  const size_t lds =
+      gpb * (sizeof(GjkShared) + (Src::kStage ? 3 * kStageGjk * sizeof(float) : size_t(0)));
   hipLaunchKernelGGL((k_gjk<LPP, EMIT, Src>), dim3((unsigned)((n + gpb - 1) / gpb)),
                      dim3(64 * wpb), lds, st, src, o, n, p, b, c, list, jobs);
   return hipGetLastError();

@@ -42,6 +42,11 @@ OGJK_DEV D3 sel(bool c, D3 a, D3 b) { return D3{c ? a.x : b.x, c ? a.y : b.y, c 
 
 OGJK_DEV int lane_id() { return __lane_id(); }
 
+OGJK_DEV void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 template <int LPP>
 OGJK_DEV uint64_t group_ballot(bool p) {
   const uint64_t b = __ballot(p);
