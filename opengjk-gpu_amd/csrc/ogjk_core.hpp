@@ -769,39 +769,44 @@ OGJK_DEV Sup support(const CBody2& A, const Query& q, int lane) {
 // their FP64 world coordinates, so the selection is that of a sweep over the
 // FP64 world vertices.
 
+// A pose as the kernels hold it, in LDS: one lane per body makes the rotation
+// matrix once per pair (it was made again for every query, some 45 FP64
+// operations and the quaternion's loads).
 struct Pose {
   double r[9];
   double t[3];
-  OGJK_DEV static Pose load(const float* p) {
-    const double w = p[0], x = p[1], y = p[2], z = p[3];
-    Pose P;
-    P.r[0] = 1.0 - 2.0 * (y * y + z * z);
-    P.r[1] = 2.0 * (x * y - w * z);
-    P.r[2] = 2.0 * (x * z + w * y);
-    P.r[3] = 2.0 * (x * y + w * z);
-    P.r[4] = 1.0 - 2.0 * (x * x + z * z);
-    P.r[5] = 2.0 * (y * z - w * x);
-    P.r[6] = 2.0 * (x * z - w * y);
-    P.r[7] = 2.0 * (y * z + w * x);
-    P.r[8] = 1.0 - 2.0 * (x * x + y * y);
-    P.t[0] = p[4];
-    P.t[1] = p[5];
-    P.t[2] = p[6];
-    return P;
-  }
-  OGJK_DEV D3 world(double x, double y, double z) const {
-    return D3{((r[0] * x + r[1] * y) + r[2] * z) + t[0], ((r[3] * x + r[4] * y) + r[5] * z) + t[1],
-              ((r[6] * x + r[7] * y) + r[8] * z) + t[2]};
-  }
-  OGJK_DEV D3 to_local(D3 d) const {  // R^T d
-    return D3{(r[0] * d.x + r[3] * d.y) + r[6] * d.z, (r[1] * d.x + r[4] * d.y) + r[7] * d.z,
-              (r[2] * d.x + r[5] * d.y) + r[8] * d.z};
-  }
 };
+using LdsPose = const __attribute__((address_space(3))) Pose*;
+
+OGJK_DEV void make_pose(const float* p, Pose* P) {
+  const double w = p[0], x = p[1], y = p[2], z = p[3];
+  P->r[0] = 1.0 - 2.0 * (y * y + z * z);
+  P->r[1] = 2.0 * (x * y - w * z);
+  P->r[2] = 2.0 * (x * z + w * y);
+  P->r[3] = 2.0 * (x * y + w * z);
+  P->r[4] = 1.0 - 2.0 * (x * x + z * z);
+  P->r[5] = 2.0 * (y * z - w * x);
+  P->r[6] = 2.0 * (x * z - w * y);
+  P->r[7] = 2.0 * (y * z + w * x);
+  P->r[8] = 1.0 - 2.0 * (x * x + y * y);
+  P->t[0] = p[4];
+  P->t[1] = p[5];
+  P->t[2] = p[6];
+}
 
 struct PBody : Body<float, 1> {
-  const float* pose;  // 7 floats: quaternion w, x, y, z, then translation
-  OGJK_DEV D3 d(int i) const { return Pose::load(pose).world(rx(i), ry(i), rz(i)); }
+  LdsPose P;
+  OGJK_DEV D3 world(double x, double y, double z) const {
+    return D3{((P->r[0] * x + P->r[1] * y) + P->r[2] * z) + P->t[0],
+              ((P->r[3] * x + P->r[4] * y) + P->r[5] * z) + P->t[1],
+              ((P->r[6] * x + P->r[7] * y) + P->r[8] * z) + P->t[2]};
+  }
+  OGJK_DEV D3 to_local(D3 d) const {  // R^T d
+    return D3{(P->r[0] * d.x + P->r[3] * d.y) + P->r[6] * d.z,
+              (P->r[1] * d.x + P->r[4] * d.y) + P->r[7] * d.z,
+              (P->r[2] * d.x + P->r[5] * d.y) + P->r[8] * d.z};
+  }
+  OGJK_DEV D3 d(int i) const { return world(rx(i), ry(i), rz(i)); }
   OGJK_DEV double c(int i, int k) const {
     const D3 p = d(i);
     return k == 0 ? p.x : (k == 1 ? p.y : p.z);
@@ -813,18 +818,19 @@ struct PBody : Body<float, 1> {
 // (R x + t).d by at most u64 (45 r1 + 15 |t|_1) scaled, < 2^-46 (r1 + |t|_1):
 // the window widens by twice that.
 template <int LPP>
-OGJK_DEV Sup support(const PBody& A, const Query& q, int lane) {
-  const Pose P = Pose::load(A.pose);
-  Sweep32 sw = sweep32_begin(P.to_local(q.dir));
+OGJK_DEV Sup support(PBody A, const Query& q, int lane) {
+  // read from LDS for each query: kept across them, two poses are 24 registers
+  asm volatile("" : "+v"(A.P));
+  Sweep32 sw = sweep32_begin(A.to_local(q.dir));
   sweep32<LPP>(static_cast<const Body<float, 1>&>(A), lane, sw);
   const float m = group_max_f<LPP>(sw.best);
-  const float t1 = (float)(fabs(P.t[0]) + fabs(P.t[1]) + fabs(P.t[2]));
+  const float t1 = (float)(fabs(A.P->t[0]) + fabs(A.P->t[1]) + fabs(A.P->t[2]));
   const float T = m - (0x1.0p-19f * A.r1 + 0x1.0p-45f * (A.r1 + t1));
   const bool multi = group_any<LPP>(sw.second >= T);
   const auto holders = lanes_where<LPP>(sw.bi >= 0 && sw.best >= T);
   if (!multi && count_lanes<LPP>(holders) == 1) {  // as in support_f
     const int src = first_lane<LPP>(holders);
-    const Sup r{shfl_i<LPP>(sw.bi, src), P.world(shfl_f<LPP>(sw.bx, src), shfl_f<LPP>(sw.by, src),
+    const Sup r{shfl_i<LPP>(sw.bi, src), A.world(shfl_f<LPP>(sw.bx, src), shfl_f<LPP>(sw.by, src),
                                                  shfl_f<LPP>(sw.bz, src))};
     const double v = dot(r.p, q.dir);
     if (q.has_inc && !(v > dot(q.inc_pt, q.dir))) return Sup{q.inc_idx, q.inc_pt};
@@ -834,7 +840,7 @@ OGJK_DEV Sup support(const PBody& A, const Query& q, int lane) {
   Cand c{-INFINITY, 0x7fffffff, D3{0.0, 0.0, 0.0}};
   if (!multi) {
     if (sw.bi >= 0 && sw.best >= T) {
-      c.p = P.world(sw.bx, sw.by, sw.bz);
+      c.p = A.world(sw.bx, sw.by, sw.bz);
       c.v = dot(c.p, q.dir);
       c.i = sw.bi;
     }
@@ -843,7 +849,7 @@ OGJK_DEV Sup support(const PBody& A, const Query& q, int lane) {
       const float px = A.rx(i), py = A.ry(i), pz = A.rz(i);
       const float d = fmaf(px, sw.dx, fmaf(py, sw.dy, pz * sw.dz));
       if (d >= T) {
-        const D3 p = P.world(px, py, pz);
+        const D3 p = A.world(px, py, pz);
         const double v = dot(p, q.dir);
         if (v > c.v) {  // ascending i within the lane keeps the lowest index
           c.v = v;
@@ -873,7 +879,7 @@ OGJK_DEV CBody2 pick(bool c, const CBody2& a, const CBody2& b) {
 }
 OGJK_DEV PBody pick(bool c, const PBody& a, const PBody& b) {
   return PBody{pick(c, static_cast<const Body<float, 1>&>(a), static_cast<const Body<float, 1>&>(b)),
-               c ? a.pose : b.pose};
+               c ? a.P : b.P};
 }
 OGJK_DEV Query pick(bool c, const Query& a, const Query& b) {
   return Query{sel(c, a.dir, b.dir), c ? a.has_inc : b.has_inc, c ? a.inc_idx : b.inc_idx,
@@ -901,17 +907,10 @@ OGJK_DEV void both_halves(const SupF& r, SupF& lo, SupF& hi) {
 // slower on the uneven 1M-pair workload, 8% faster on 64-vertex pairs).
 template <class BT>
 constexpr bool kSplitQueries = !std::is_base_of_v<CBody, BT>;
-// Posed bodies in a 64-lane group (the wave) also query one after the other:
-// each query's pose is then wave-uniform and stays in scalar registers (the
-// posed GJK kernel's scratch 60 -> 12 B/lane; 10,000 posed pairs 0.186 ->
-// 0.181 ms).
-template <int LPP, class BT>
-constexpr bool kSplit = kSplitQueries<BT> && !(LPP == 64 && std::is_same_v<BT, PBody>);
-
 template <int LPP, class BT>
 OGJK_DEV void support_pair(const BT& A, const Query& qa, const BT& B, const Query& qb, int lane,
                            Sup& ra, Sup& rb) {
-  if constexpr (LPP >= 8 && kSplit<LPP, BT>) {
+  if constexpr (LPP >= 8 && kSplitQueries<BT>) {
     // the lower half of the group answers A's query, the upper half B's, at
     // the same time; then each half takes the other's result
     const bool hi = lane >= LPP / 2;

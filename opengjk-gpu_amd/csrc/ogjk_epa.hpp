@@ -294,11 +294,11 @@ OGJK_DEV void fetch_face(const EpaShared<LPP>& sh, const Faces& F, int slot, D3&
 }
 
 // The two bodies as EPA holds them through its loop.  Where the group splits
-// into halves (see kSplit), a lane keeps its own half's body only (the lower
+// into halves (see kSplitQueries), a lane keeps its own half's body only (the lower
 // half A, the upper half B), half the registers, and each half works on its
 // body: the queries, and the blend of the witnesses, which the halves then
 // exchange.  Otherwise every lane keeps both.
-template <int LPP, class BT, bool SPLIT = LPP >= 16 && kSplit<LPP, BT>>
+template <int LPP, class BT, bool SPLIT = LPP >= 16 && kSplitQueries<BT>>
 struct PairView {
   BT A, B;
   OGJK_DEV PairView(const BT& a, const BT& b, int) : A(a), B(b) {}

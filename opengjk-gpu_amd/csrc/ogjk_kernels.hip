@@ -16,7 +16,7 @@
 #define OGJK_GJK_WAVES_WIDE 3
 #endif
 #ifndef OGJK_GJK_WAVES_POSED
-#define OGJK_GJK_WAVES_POSED 3
+#define OGJK_GJK_WAVES_POSED 4
 #endif
 // EPA: float scenes swept whole run faster at 3 waves/SIMD even though the
 // compiler then spills 80 B/lane (100K x 64: 1.22 -> 1.12 ms); the 64-lane
@@ -64,6 +64,7 @@ struct SceneSrc {
   // descriptors in vector registers (10K x 100K: 4.7 vs 5.3 ms)
   static constexpr bool kEpaScalarPair = CL != 2;
   // GJK stages small pairs in LDS (float scenes without clusters)
+  static constexpr int kLds = 0;  // bytes of LDS that load() needs per group
   static constexpr bool kStage = std::is_same_v<T, float> && CL == 0;
 
   // max(nA, nB) of pair i, or 0 for an invalid pair (it goes to bucket 0)
@@ -74,7 +75,7 @@ struct SceneSrc {
   }
 
   template <int LPP>
-  OGJK_DEV bool load(int i, int lane, BodyT& A, BodyT& B) const {
+  OGJK_DEV bool load(int i, int lane, BodyT& A, BodyT& B, void* lds) const {
     int a, b;
     if (pairs) {
       a = pairs[2 * i];
@@ -118,6 +119,7 @@ struct PoseSrc {
   template <int LPP>
   static constexpr int kEpaWaves = OGJK_EPA_WAVES;
   static constexpr bool kEpaScalarPair = false;  // posed pairs: measured no faster
+  static constexpr int kLds = 2 * sizeof(Pose);
   static constexpr bool kStage = false;
 
   OGJK_DEV int pair_size(int i) const {
@@ -127,14 +129,18 @@ struct PoseSrc {
   }
 
   template <int LPP>
-  OGJK_DEV bool load(int i, int lane, BodyT& A, BodyT& B) const {
+  OGJK_DEV bool load(int i, int lane, BodyT& A, BodyT& B, void* lds) const {
     const int a = pairs[2 * i], b = pairs[2 * i + 1];
     if (a < 0 || a >= nb || b < 0 || b >= nb) return false;
     const int64_t oa = off[a], ob = off[b];
     const float* pa = by_body ? poses + 7 * (int64_t)a : poses + 14 * (int64_t)i;
     const float* pb = by_body ? poses + 7 * (int64_t)b : poses + 14 * (int64_t)i + 7;
-    A = PBody{{x + oa, y + oa, z + oa, cnt[a], r1[a]}, pa};
-    B = PBody{{x + ob, y + ob, z + ob, cnt[b], r1[b]}, pb};
+    Pose* P = (Pose*)lds;
+    wave_sync();
+    if (lane < 2) make_pose(lane ? pb : pa, P + lane);
+    wave_sync();
+    A = PBody{{x + oa, y + oa, z + oa, cnt[a], r1[a]}, (LdsPose)P};
+    B = PBody{{x + ob, y + ob, z + ob, cnt[b], r1[b]}, (LdsPose)(P + 1)};
     return true;
   }
 };
@@ -149,6 +155,7 @@ struct PolySrc {
   template <int LPP>
   static constexpr int kEpaWaves = OGJK_EPA_WAVES;
   static constexpr bool kEpaScalarPair = false;
+  static constexpr int kLds = 0;  // bytes of LDS that load() needs per group
   static constexpr bool kStage = false;
 
   OGJK_DEV int pair_size(int i) const {
@@ -166,7 +173,7 @@ struct PolySrc {
   }
 
   template <int LPP>
-  OGJK_DEV bool load(int i, int lane, BodyT& A, BodyT& B) const {
+  OGJK_DEV bool load(int i, int lane, BodyT& A, BodyT& B, void* lds) const {
     const gkPolytope* pa;
     const gkPolytope* pb;
     if (pairs) {
@@ -203,6 +210,7 @@ struct Aos64Src {
   template <int LPP>
   static constexpr int kEpaWaves = OGJK_EPA_WAVES;
   static constexpr bool kEpaScalarPair = false;
+  static constexpr int kLds = 0;  // bytes of LDS that load() needs per group
   static constexpr bool kStage = false;
 
   OGJK_DEV int pair_size(int i) const {
@@ -212,7 +220,7 @@ struct Aos64Src {
   }
 
   template <int LPP>
-  OGJK_DEV bool load(int i, int lane, BodyT& A, BodyT& B) const {
+  OGJK_DEV bool load(int i, int lane, BodyT& A, BodyT& B, void* lds) const {
     const int a = pairs ? pairs[2 * i] : 2 * i, b = pairs ? pairs[2 * i + 1] : 2 * i + 1;
     if (a < 0 || a >= nb || b < 0 || b >= nb) return false;
     const double* pa = xyz + 3 * off[a];
@@ -382,6 +390,7 @@ __global__ void __launch_bounds__(256) k_pairs(Src src, OutArgs out, int n) {
   __shared__ EpaShared<LPP> sh[kEpa ? GPB : 1];
   __shared__ GjkShared gs[(MODE & 1) ? GPB : 1];
   __shared__ EpaTable tb;
+  __shared__ __attribute__((aligned(16))) unsigned char own[Src::kLds ? GPB * Src::kLds : 1];
   if constexpr (kEpa) epa_table_begin(tb);
   const int lane = threadIdx.x & (LPP - 1);
   const int g = threadIdx.x / LPP;
@@ -389,7 +398,8 @@ __global__ void __launch_bounds__(256) k_pairs(Src src, OutArgs out, int n) {
   if (pair >= n) return;
 
   typename Src::BodyT A, B;
-  const bool ok = src.template load<LPP>(pair, lane, A, B) && A.n > 0 && B.n > 0;
+  const bool ok =
+      src.template load<LPP>(pair, lane, A, B, own + g * Src::kLds) && A.n > 0 && B.n > 0;
   if (!ok) {
     if (lane == 0) store_invalid(out, pair, kEpa);
     return;
@@ -641,14 +651,15 @@ __global__ void __launch_bounds__(256, Src::kGjkWaves)
   const int pair = multi ? list[__builtin_amdgcn_readfirstlane(c[kBucketStart + bucket]) + j]
                          : (int)j;
   typename Src::BodyT A, B;
-  const bool ok = src.template load<LPP>(pair, lane, A, B) && A.n > 0 && B.n > 0;
+  unsigned char* own = ogjk_lds + GPB * sizeof(GjkShared);  // the sources' or the stage's part
+  const bool ok = src.template load<LPP>(pair, lane, A, B, own + (threadIdx.x / LPP) * Src::kLds) &&
+                  A.n > 0 && B.n > 0;
   if (!ok) {
     if (lane == 0) store_invalid(out, pair, EMIT);
     return;
   }
   if constexpr (Src::kStage) {
-    float* stg = (float*)(ogjk_lds + GPB * sizeof(GjkShared)) +
-                 (threadIdx.x / LPP) * (3 * kStageGjk);
+    float* stg = (float*)own + (threadIdx.x / LPP) * (3 * kStageGjk);
     stage_pair<LPP, kStageGjk>(A, B, stg, lane);
   }
   Simplex s = {};
@@ -696,7 +707,8 @@ __global__ void __launch_bounds__(256, Src::template kEpaWaves<LPP>)
     // registers
     if constexpr (LPP == 64 && Src::kEpaScalarPair) pair = __builtin_amdgcn_readfirstlane(pair);
     typename Src::BodyT A, B;
-    src.template load<LPP>(pair, lane, A, B);  // validated by the GJK kernel
+    // validated by the GJK kernel
+    src.template load<LPP>(pair, lane, A, B, (unsigned char*)(sh + GPB) + g * Src::kLds);
     D3 normal{0.0, 0.0, 0.0};
     epa<LPP>(A, B, s, dist, w, normal, sh[g], tb, lane);
     if (lane == 0) store(out, pair, s, w, dist, normal, true);
@@ -717,7 +729,7 @@ __global__ void __launch_bounds__(256) k_gjk_all(Src src, OutArgs out, int n, Ep
   const int pair = blockIdx.x * GPB + threadIdx.x / LPP;
   if (pair >= n) return;
   typename Src::BodyT A, B;
-  const bool ok = src.template load<LPP>(pair, lane, A, B) && A.n > 0 && B.n > 0;
+  const bool ok = src.template load<LPP>(pair, lane, A, B, nullptr) && A.n > 0 && B.n > 0;
   if (!ok) {
     if (lane == 0) {
       store_invalid(out, pair, EMIT);
@@ -752,7 +764,7 @@ __global__ void __launch_bounds__(256) k_epa_all(Src src, OutArgs out, int n, co
   double dist;
   job_load(jobs + pair, s, w, dist);
   typename Src::BodyT A, B;
-  src.template load<LPP>(pair, lane, A, B);  // validated by the GJK kernel
+  src.template load<LPP>(pair, lane, A, B, nullptr);  // validated by the GJK kernel
   D3 normal{0.0, 0.0, 0.0};
   epa_shared_begin<LPP>(sh[g], lane);
   epa<LPP>(A, B, s, dist, w, normal, sh[g], tb, lane);
@@ -904,7 +916,8 @@ static hipError_t launch_gjk(const Src& src, const OutArgs& o, int n, const Buck
   EpaJob* jobs = (EpaJob*)((char*)ws + ws_jobs_off(n));
   const int gpb = 64 * wpb / LPP;
   const size_t lds =
-      gpb * (sizeof(GjkShared) + (Src::kStage ? 3 * kStageGjk * sizeof(float) : size_t(0)));
+      gpb * (sizeof(GjkShared) + Src::kLds +
+             (Src::kStage ? 3 * kStageGjk * sizeof(float) : size_t(0)));
   hipLaunchKernelGGL((k_gjk<LPP, EMIT, Src>), dim3((unsigned)((n + gpb - 1) / gpb)),
                      dim3(64 * wpb), lds, st, src, o, n, p, b, c, list, jobs);
   return hipGetLastError();
@@ -919,7 +932,7 @@ static hipError_t launch_epa_list(const Src& src, const OutArgs& o, int n, const
   const EpaJob* jobs = (const EpaJob*)((char*)ws + ws_jobs_off(n));
   const int gpb = 64 * wpb / LPP;
   hipLaunchKernelGGL((k_epa_list<LPP, Src>), dim3(persistent_blocks(n, gpb, 16384u / wpb)),
-                     dim3(64 * wpb), sizeof(EpaTable) + (size_t)gpb * sizeof(EpaShared<LPP>), st, src, o, p, cls, c,
+                     dim3(64 * wpb), sizeof(EpaTable) + gpb * (sizeof(EpaShared<LPP>) + Src::kLds), st, src, o, p, cls, c,
                      jobs);
   return hipGetLastError();
 }
