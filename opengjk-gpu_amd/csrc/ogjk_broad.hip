@@ -36,6 +36,13 @@ __device__ __forceinline__ int cell_axis(float p, float boundary, float cell, in
   return (int)f;
 }
 
+__device__ __forceinline__ uint32_t cell_key(const float4 s, float cell, float boundary, int g) {
+  const uint32_t cx = cell_axis(s.x, boundary, cell, g);
+  const uint32_t cy = cell_axis(s.y, boundary, cell, g);
+  const uint32_t cz = cell_axis(s.z, boundary, cell, g);
+  return cx + (uint32_t)g * (cy + (uint32_t)g * cz);
+}
+
 __device__ __forceinline__ bool overlap(const float4 a, const float4 b) {
   const float dx = a.x - b.x, dy = a.y - b.y, dz = a.z - b.z;
   const float d2 = (dx * dx + dy * dy) + dz * dz;
@@ -58,10 +65,7 @@ __global__ __launch_bounds__(kBlock) void k_bp_hist(const float4* __restrict__ s
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
   const float4 s = sph[i];
-  const uint32_t cx = cell_axis(s.x, boundary, cell, g);
-  const uint32_t cy = cell_axis(s.y, boundary, cell, g);
-  const uint32_t cz = cell_axis(s.z, boundary, cell, g);
-  const uint32_t k = cx + (uint32_t)g * (cy + (uint32_t)g * cz);
+  const uint32_t k = cell_key(s, cell, boundary, g);
   keys[i] = k;
   slot[i] = atomicAdd(count + k, 1);
 }
@@ -102,40 +106,54 @@ __device__ __forceinline__ bool gated_off(const int32_t* gate) {
   return gate != nullptr && *gate != 0;
 }
 
-// Object i goes to start[cell] + (number of lower indices in its cell): cells
-// list their objects in ascending index.  pos[i] = that position.
+// Workgroups go to the 8 XCDs round-robin; a grid of a multiple of 8 blocks
+// is remapped so that each XCD takes one contiguous eighth (a slab of cells
+// whose neighbour rows mostly stay in that XCD's L2).
+constexpr int kXcds = 8;
+__device__ __forceinline__ int xcd_block() {
+  const int per = gridDim.x / kXcds;
+  return (blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
+}
+unsigned xcd_blocks(int64_t threads) {
+  const int64_t b = (threads + kBlock - 1) / kBlock;
+  return (unsigned)((b + kXcds - 1) / kXcds * kXcds);
+}
+
+// The object at place t of the cell order (its cell's objects in order of
+// arrival) goes to start[cell] + (number of lower indices in its cell): cells
+// list their objects in ascending index.  Threads in cell order, not in index
+// order: the cell's bounds, its list and the record then lie next to the
+// neighbouring threads', and the sphere is the only line fetched at random (1M
+// spheres: 47 us in index order, with four such lines each).
 // An object of a cell holding more than kRankScanMax objects ranks nothing
 // and sets *crowded (one atomic per wave); the host then sorts instead.
-__global__ __launch_bounds__(kBlock) void k_bp_rank(const float4* __restrict__ sph,
-                                                    const uint32_t* __restrict__ keys,
+// Launched on xcd_blocks(n) blocks.
+__global__ __launch_bounds__(kBlock) void k_bp_rank(const float4* __restrict__ sph, float cell,
+                                                    float boundary, int g,
                                                     const int32_t* __restrict__ start,
                                                     const int32_t* __restrict__ tmp, int n,
                                                     BpRec* __restrict__ rec,
-                                                    int32_t* __restrict__ pos,
                                                     int32_t* __restrict__ crowded) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  const uint32_t k = i < n ? keys[i] : 0u;
-  const int lo = i < n ? start[k] : 0, hi = i < n ? start[k + 1] : 0;
-  const bool big = hi - lo > kRankScanMax;
+  const int t = xcd_block() * kBlock + threadIdx.x;
+  BpRec e;
+  e.id = t < n ? tmp[t] : 0;
+  e.s = sph[e.id];
+  e.key = cell_key(e.s, cell, boundary, g);
+  e.pad[0] = e.pad[1] = 0;
+  const int lo = start[e.key], hi = start[e.key + 1];
+  const bool big = t < n && hi - lo > kRankScanMax;
   const uint64_t any = __ballot(big);
   if (any != 0 && (threadIdx.x & 63) == (unsigned)__builtin_ctzll(any)) atomicOr(crowded, 1);
-  if (i >= n || big) return;
+  if (t >= n || big) return;
   int r = 0;
-  for (int t = lo; t < hi; t++) r += tmp[t] < i;
-  BpRec e;
-  e.s = sph[i];
-  e.id = i;
-  e.key = k;
-  e.pad[0] = e.pad[1] = 0;
+  for (int u = lo; u < hi; u++) r += tmp[u] < e.id;
   rec[lo + r] = e;
-  pos[i] = lo + r;
 }
 
 __global__ __launch_bounds__(kBlock) void k_bp_from_sorted(const float4* __restrict__ sph,
                                                            const uint32_t* __restrict__ okeys,
                                                            const int32_t* __restrict__ order,
-                                                           int n, BpRec* __restrict__ rec,
-                                                           int32_t* __restrict__ pos) {
+                                                           int n, BpRec* __restrict__ rec) {
   const int t = blockIdx.x * kBlock + threadIdx.x;
   if (t >= n) return;
   const int i = order[t];
@@ -145,18 +163,19 @@ __global__ __launch_bounds__(kBlock) void k_bp_from_sorted(const float4* __restr
   e.key = okeys[t];
   e.pad[0] = e.pad[1] = 0;
   rec[t] = e;
-  pos[i] = t;
 }
 
-// Partners of an object the count pass keeps for the emit pass.
-constexpr int kKeep = 8;
+// Partners of an object the count pass keeps for the emit pass (an object with
+// more walks its neighbours a second time).
+constexpr int kKeep = 16;
 
 // Calls f(j) for every j > o overlapping the object at sorted position s, in
 // neighbour-cell order (z, y, x from -1 to +1), ascending j within a cell.
+// rows: the block's 9 * kBlock entries of LDS.
 template <typename F>
 __device__ __forceinline__ void bp_walk(const BpRec* __restrict__ rec,
                                         const int32_t* __restrict__ start, int s, int g, int cap,
-                                        F&& f) {
+                                        int2* rows, F&& f) {
   const BpRec me = rec[s];
   const int o = me.id;
   const uint32_t k = me.key;
@@ -166,8 +185,13 @@ __device__ __forceinline__ void bp_walk(const BpRec* __restrict__ rec,
   const int x0 = cx > 0 ? cx - 1 : 0, x1 = cx < g - 1 ? cx + 1 : g - 1;
   if (cap == 0) {
     // uncapped: the x-neighbours of each of the 9 rows are one contiguous
-    // range; all 18 bounds are loaded before any candidate (indices clamped
-    // into the grid, rows outside it emptied)
+    // range (indices clamped into the grid, rows outside it emptied).  The
+    // rows' lengths differ from lane to lane, so a wave that took them one by
+    // one would wait for its longest lane nine times over; each lane instead
+    // runs through its own rows as one sequence, kept as (end in the sequence,
+    // position minus sequence index) per row that holds anything.
+    int2* my = rows + threadIdx.x;
+    int total = 0, nrow = 0;
     int lo[9], hi[9];
 #pragma unroll
     for (int r = 0; r < 9; r++) {
@@ -179,22 +203,35 @@ __device__ __forceinline__ void bp_walk(const BpRec* __restrict__ rec,
       hi[r] = in ? start[row + x1 + 1] : lo[r];
     }
 #pragma unroll
-    for (int r = 0; r < 9; r++)
-      for (int t = lo[r]; t < hi[r]; t += 4) {
-        // four candidates in flight; indices past the row repeat its last
-        // entry and are skipped
-        float4 q[4];
-        int j[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-          const int tu = t + u < hi[r] ? t + u : hi[r] - 1;
-          q[u] = rec[tu].s;
-          j[u] = rec[tu].id;
-        }
-#pragma unroll
-        for (int u = 0; u < 4; u++)
-          if (t + u < hi[r] && j[u] > o && overlap(me.s, q[u])) f(j[u]);
+    for (int r = 0; r < 9; r++) {
+      if (hi[r] > lo[r]) {
+        const int from = lo[r] - total;
+        total += hi[r] - lo[r];
+        my[nrow++ * kBlock] = int2{total, from};
       }
+    }
+    int2 cur = my[0];  // never empty: the object's own row holds it
+    int at = 0;
+    for (int m = 0; m < total; m += 4) {
+      // four candidates in flight; indices past the last repeat it and are
+      // skipped.  An index is loaded only for an overlapping sphere.
+      int t[4];
+      float4 q[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int mu = m + u < total ? m + u : total - 1;
+        if (mu >= cur.x) cur = my[++at * kBlock];
+        t[u] = mu + cur.y;
+        q[u] = rec[t[u]].s;
+      }
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        if (m + u < total && t[u] != s && overlap(me.s, q[u])) {
+          const int j = rec[t[u]].id;
+          if (j > o) f(j);
+        }
+      }
+    }
     return;
   }
   for (int dz = -1; dz <= 1; dz++) {
@@ -218,43 +255,36 @@ __device__ __forceinline__ void bp_walk(const BpRec* __restrict__ rec,
   }
 }
 
-// Workgroups go to the 8 XCDs round-robin; a grid of a multiple of 8 blocks
-// is remapped so that each XCD takes one contiguous eighth (a slab of cells
-// whose neighbour rows mostly stay in that XCD's L2).
-constexpr int kXcds = 8;
-__device__ __forceinline__ int xcd_block() {
-  const int per = gridDim.x / kXcds;
-  return (blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
-}
-unsigned xcd_blocks(int64_t threads) {
-  const int64_t b = (threads + kBlock - 1) / kBlock;
-  return (unsigned)((b + kXcds - 1) / kXcds * kXcds);
-}
-
 // Count pass, one thread per object in cell order: counts[o] = number of
 // pairs (o, j), j > o (counts[n] = 0, so the exclusive scan's last entry is
-// the total), and the first kKeep partners in keep[kKeep o ..].  Launched on
-// xcd_blocks(n + 1) blocks.
+// the total), and the first kKeep partners in keep[kKeep o ..]; pos[o] = s where
+// there are more.  *flag: the gate, next to the total for one copy to the host.
+// Launched on xcd_blocks(n + 1) blocks.
 __global__ __launch_bounds__(kBlock) void k_bp_count(const BpRec* __restrict__ rec,
                                                      const int32_t* __restrict__ start, int n,
                                                      int g, int cap,
                                                      int64_t* __restrict__ counts,
                                                      int32_t* __restrict__ keep,
+                                                     int32_t* __restrict__ pos,
+                                                     int64_t* __restrict__ flag,
                                                      const int32_t* __restrict__ gate) {
+  __shared__ int2 rows[9 * kBlock];
   const int s = xcd_block() * kBlock + threadIdx.x;
-  if (gated_off(gate)) return;
-  if (s >= n) {
-    if (s == n) counts[n] = 0;
-    return;
+  const bool off = gated_off(gate);
+  if (s == n) {
+    counts[n] = 0;
+    *flag = off ? 1 : 0;
   }
+  if (s >= n || off) return;
   const int o = rec[s].id;
   int64_t cnt = 0;
   int32_t* kp = keep + (int64_t)kKeep * o;
-  bp_walk(rec, start, s, g, cap, [&](int j) {
+  bp_walk(rec, start, s, g, cap, rows, [&](int j) {
     if (cnt < kKeep) kp[cnt] = j;
     cnt++;
   });
   counts[o] = cnt;
+  if (cnt > kKeep) pos[o] = s;
 }
 
 // Emit pass, one thread per object in index order (the output is in index
@@ -270,6 +300,7 @@ __global__ __launch_bounds__(kBlock) void k_bp_emit(const BpRec* __restrict__ re
                                                     gkCollisionPair* __restrict__ pairs,
                                                     int64_t max_pairs,
                                                     const int32_t* __restrict__ gate) {
+  __shared__ int2 rows[9 * kBlock];
   const int o = blockIdx.x * kBlock + threadIdx.x;
   if (o >= n || gated_off(gate)) return;
   int64_t w = offsets[o];
@@ -279,7 +310,7 @@ __global__ __launch_bounds__(kBlock) void k_bp_emit(const BpRec* __restrict__ re
     for (int q = 0; q < c && w < max_pairs; q++, w++) pairs[w] = gkCollisionPair{o, kp[q]};
     return;
   }
-  bp_walk(rec, start, pos[o], g, cap, [&](int j) {
+  bp_walk(rec, start, pos[o], g, cap, rows, [&](int j) {
     if (w < max_pairs) pairs[w] = gkCollisionPair{o, j};
     w++;
   });
@@ -376,7 +407,8 @@ hipError_t bp_layout_query(int n, int64_t cells, BpLayout* L) {
   L->pos = o;     o += up256(sizeof(int32_t) * (size_t)n);
   L->keep = o;    o += up256(sizeof(int32_t) * kKeep * (size_t)n);
   L->counts = o;  o += up256(sizeof(int64_t) * ((size_t)n + 1));
-  L->offsets = o; o += up256(sizeof(int64_t) * ((size_t)n + 1));
+  // offsets[n] is the total, offsets[n + 1] the crowded-cell flag again
+  L->offsets = o; o += up256(sizeof(int64_t) * ((size_t)n + 2));
   L->okeys = o;   o += up256(sizeof(uint32_t) * (size_t)n);
   L->temp = o;    o += up256(L->temp_bytes);
   L->total = o;
@@ -494,15 +526,14 @@ ogjk_status ogjk_broad_phase(const float* d_spheres, int32_t n_objects, const og
   // objects with the radix sort below and counts and emits again.
   hipLaunchKernelGGL(k_bp_place, dim3(blocks_for(n)), dim3(kBlock), 0, st_, keys, slot, start,
                      n, tmp);
-  hipLaunchKernelGGL(k_bp_rank, dim3(blocks_for(n)), dim3(kBlock), 0, st_, sph, keys, start, tmp,
-                     n, rec, pos, crowded);
+  hipLaunchKernelGGL(k_bp_rank, dim3(xcd_blocks(n)), dim3(kBlock), 0, st_, sph,
+                     grid->cell_size, grid->boundary, g, start, tmp, n, rec, crowded);
   BP_HIP(hipGetLastError(), "cell sort");
-  int64_t total = 0;
-  int32_t is_crowded = 0;
+  int64_t found[2] = {0, 0};  // the total, and whether a cell was too crowded
   for (int pass = 0; pass < 2; pass++) {
     const int32_t* gate = pass == 0 ? crowded : nullptr;
     hipLaunchKernelGGL(k_bp_count, dim3(xcd_blocks((int64_t)n + 1)), dim3(kBlock), 0, st_, rec,
-                       start, n, g, grid->max_per_cell, counts, keep, gate);
+                       start, n, g, grid->max_per_cell, counts, keep, pos, offsets + n + 1, gate);
     BP_HIP(hipGetLastError(), "pair count");
     tb = L.temp_bytes;
     BP_HIP(hipcub::DeviceScan::ExclusiveSum(temp, tb, counts, offsets, n + 1, st_), "pair scan");
@@ -512,13 +543,10 @@ ogjk_status ogjk_broad_phase(const float* d_spheres, int32_t n_objects, const og
                          (int64_t)max_pairs, gate);
       BP_HIP(hipGetLastError(), "pair emit");
     }
-    BP_HIP(hipMemcpyAsync(&total, offsets + n, sizeof(int64_t), hipMemcpyDeviceToHost, st_),
+    BP_HIP(hipMemcpyAsync(found, offsets + n, sizeof(found), hipMemcpyDeviceToHost, st_),
            "pair total");
-    if (pass == 0)
-      BP_HIP(hipMemcpyAsync(&is_crowded, crowded, sizeof(int32_t), hipMemcpyDeviceToHost, st_),
-             "cell occupancy");
     BP_HIP(hipStreamSynchronize(st_), "broad phase");
-    if (!is_crowded) break;
+    if (!found[1]) break;
     if (pass == 0) {
       // crowded cells: a stable radix sort by cell lists each cell's objects
       // in ascending index
@@ -529,10 +557,11 @@ ogjk_status ogjk_broad_phase(const float* d_spheres, int32_t n_objects, const og
                                                 L.key_bits, st_),
              "cell radix sort");
       hipLaunchKernelGGL(k_bp_from_sorted, dim3(blocks_for(n)), dim3(kBlock), 0, st_, sph, okeys,
-                         tmp, n, rec, pos);
+                         tmp, n, rec);
       BP_HIP(hipGetLastError(), "cell sort");
     }
   }
+  const int64_t total = found[0];
   if (n_found) *n_found = total;
   if (n_pairs) *n_pairs = (int32_t)(total < max_pairs ? total : max_pairs);
   return OGJK_OK;
