@@ -206,14 +206,17 @@ ogjk_status run_host(int mode, const gkPolytope* const* lists, const int* counts
   int64_t o = 0;
   for (int64_t b = 0; b < nb; b++) {
     const gkPolytope& p = body_at(b);
-    float m = 0.0f;
+    // four running maxima: one alone is a chain of a compare per vertex
+    float m4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int i = 0; i < p.numpoints; i++) {
       const float vx = p.coord[3 * i], vy = p.coord[3 * i + 1], vz = p.coord[3 * i + 2];
       hx[o + i] = vx;
       hy[o + i] = vy;
       hz[o + i] = vz;
-      m = std::fmax(m, std::fabs(vx) + std::fabs(vy) + std::fabs(vz));
+      const float l1 = std::fabs(vx) + std::fabs(vy) + std::fabs(vz);
+      m4[i & 3] = l1 > m4[i & 3] ? l1 : m4[i & 3];  // NaN is passed over
     }
+    const float m = std::fmax(std::fmax(m4[0], m4[1]), std::fmax(m4[2], m4[3]));
     hoff[b] = o;
     hcnt[b] = p.numpoints;
     hr1[b] = m * (1.0f + 0x1.0p-22f);  // per-body L1 bound, rounded up
