@@ -941,6 +941,33 @@ OGJK_DEV void support_pair(const BT& A, const Query& qa, const BT& B, const Quer
   }
 }
 
+// A clustered body of a pair that two waves work on together, a block of 128:
+// the first wave answers every query of A, the second of B, and they exchange
+// the results.  Everything else both do alike, each in its own LDS, so their
+// control flow is one and the barriers meet.
+struct DuoShared {
+  SupF r[2];
+};
+template <class BT>
+struct Duo : BT {
+  DuoShared* ex;
+};
+
+template <int LPP, class BT>
+OGJK_DEV void support_pair(const Duo<BT>& A, const Query& qa, const Duo<BT>& B, const Query& qb,
+                           int lane, Sup& ra, Sup& rb) {
+  static_assert(LPP == 64, "one wave per body");
+  const bool second = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) != 0;
+  const BT& a = A;
+  const BT& b = B;
+  const Sup r = support<64>(pick(second, b, a), pick(second, qb, qa), lane);
+  if (lane == 0) A.ex->r[second] = SupF{r.i, (float)r.p.x, (float)r.p.y, (float)r.p.z};
+  __syncthreads();
+  ra = widen(A.ex->r[0]);
+  rb = widen(A.ex->r[1]);
+  __syncthreads();  // read by both before the next query overwrites it
+}
+
 // Plain FP64 path over double storage: the same selection rules computed
 // directly in FP64 (the comparison baseline; no FP32 pass).
 template <int LPP, int STRIDE>

@@ -66,6 +66,8 @@ struct SceneSrc {
   // GJK stages small pairs in LDS (float scenes without clusters)
   static constexpr int kLds = 0;  // bytes of LDS that load() needs per group
   static constexpr bool kStage = std::is_same_v<T, float> && CL == 0;
+  // few pairs of clustered bodies: two waves to a pair
+  static constexpr bool kDuo = CL != 0;
 
   // max(nA, nB) of pair i, or 0 for an invalid pair (it goes to bucket 0)
   OGJK_DEV int pair_size(int i) const {
@@ -121,6 +123,7 @@ struct PoseSrc {
   static constexpr bool kEpaScalarPair = false;  // posed pairs: measured no faster
   static constexpr int kLds = 2 * sizeof(Pose);
   static constexpr bool kStage = false;
+  static constexpr bool kDuo = false;
 
   OGJK_DEV int pair_size(int i) const {
     const int a = pairs[2 * i], b = pairs[2 * i + 1];
@@ -157,6 +160,7 @@ struct PolySrc {
   static constexpr bool kEpaScalarPair = false;
   static constexpr int kLds = 0;  // bytes of LDS that load() needs per group
   static constexpr bool kStage = false;
+  static constexpr bool kDuo = false;
 
   OGJK_DEV int pair_size(int i) const {
     const gkPolytope *pa, *pb;
@@ -212,6 +216,7 @@ struct Aos64Src {
   static constexpr bool kEpaScalarPair = false;
   static constexpr int kLds = 0;  // bytes of LDS that load() needs per group
   static constexpr bool kStage = false;
+  static constexpr bool kDuo = false;
 
   OGJK_DEV int pair_size(int i) const {
     const int a = pairs ? pairs[2 * i] : 2 * i, b = pairs ? pairs[2 * i + 1] : 2 * i + 1;
@@ -715,6 +720,73 @@ __global__ void __launch_bounds__(256, Src::template kEpaWaves<LPP>)
   }
 }
 
+// Clustered pairs, a block of two waves each (see Duo).  A whole-wave query of
+// a large body is a chain of some ten memory round trips and a lone wave on its
+// SIMD takes about ten cycles an instruction, so where the pairs are too few to
+// fill the chip a second wave takes half of the queries.
+template <bool EMIT, class Src>
+__global__ void __launch_bounds__(128)
+    k_gjk_duo(Src src, OutArgs out, int n, BucketPlan plan, int bucket, unsigned* c,
+              const int* list, EpaJob* jobs) {
+  __shared__ GjkShared gs[2];
+  __shared__ DuoShared ex;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const bool multi = plan.nb > 1;
+  const unsigned count = multi ? c[kCntBucket + bucket] : (unsigned)n;
+  if (blockIdx.x >= count) return;
+  const int pair = multi ? list[c[kBucketStart + bucket] + blockIdx.x] : (int)blockIdx.x;
+  using BT = typename Src::BodyT;
+  Duo<BT> A, B;
+  const bool ok = src.template load<64>(pair, lane, A, B, nullptr) && A.n > 0 && B.n > 0;
+  if (!ok) {
+    if (threadIdx.x == 0) store_invalid(out, pair, EMIT);
+    return;
+  }
+  A.ex = B.ex = &ex;
+  Simplex s = {};
+  Wit w = {};
+  const double dist = gjk<64>(A, B, s, w, gs[wave], lane);
+  if (wave != 0) return;
+  const bool pen = EMIT && !(dist > kEps64);
+  const int cls = plan.epa_class[bucket];
+  const unsigned k = wave_fetch_add(job_counter(c, cls), lane == 0 && pen);
+  if (lane != 0) return;
+  if (pen) {
+    job_store(jobs + (multi ? c[kClassStart + cls] : 0u) + k, pair, s, w, dist);
+  } else {
+    store(out, pair, s, w, dist, EMIT ? contact_normal(w.w0, w.w1) : D3{0.0, 0.0, 0.0}, EMIT);
+  }
+}
+
+// One block per job: the launch covers every pair, so no job is left over.
+template <class Src>
+__global__ void __launch_bounds__(128)
+    k_epa_duo(Src src, OutArgs out, BucketPlan plan, int cls, unsigned* c, const EpaJob* jobs) {
+  __shared__ EpaShared<64> sh[2];
+  __shared__ EpaTable tb;
+  __shared__ DuoShared ex;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const unsigned njobs =
+      __builtin_amdgcn_readfirstlane(__atomic_load_n(job_counter(c, cls), __ATOMIC_RELAXED));
+  if (blockIdx.x >= njobs) return;
+  epa_table_begin(tb);
+  epa_shared_begin<64>(sh[wave], lane);
+  Simplex s = {};
+  Wit w = {};
+  double dist;
+  const int pair = __builtin_amdgcn_readfirstlane(
+      job_load(jobs + (plan.nb > 1 ? c[kClassStart + cls] : 0u) + blockIdx.x, s, w, dist));
+  using BT = typename Src::BodyT;
+  Duo<BT> A, B;
+  src.template load<64>(pair, lane, A, B, nullptr);  // validated by the GJK kernel
+  A.ex = B.ex = &ex;
+  D3 normal{0.0, 0.0, 0.0};
+  epa<64>(A, B, s, dist, w, normal, sh[wave], tb, lane);
+  if (threadIdx.x == 0) store(out, pair, s, w, dist, normal, true);
+}
+
 // The reference's launch shape (GJK/gpu/openGJK.cu:2968-3004): a GJK kernel
 // over every pair, then an EPA kernel over every pair, one group of LPP lanes
 // per pair in each, non-persistent (LPP = 1 is one thread per pair).  The
@@ -900,6 +972,10 @@ static int fill_lanes(int lanes, int n) {
   return lanes;
 }
 
+// Two waves to a pair up to here: two waves on every SIMD then, and past it
+// more waves than pairs would only repeat the work that both waves of a pair do.
+static bool use_duo(int lanes, int n) { return lanes == 64 && 64 * (int64_t)n <= kChipLanes; }
+
 // Resident grid for a persistent launch over at most n items.
 static unsigned persistent_blocks(int n, int gpb, unsigned cap = 4096u) {
   const unsigned want = (unsigned)((n + gpb - 1) / gpb);
@@ -940,6 +1016,14 @@ static hipError_t launch_epa_list(const Src& src, const OutArgs& o, int n, const
 template <bool EMIT, class Src>
 static hipError_t gjk_by_lanes(int lanes, const Src& src, const OutArgs& o, int n,
                                const BucketPlan& p, int b, int wpb, void* ws, hipStream_t st) {
+  if constexpr (Src::kDuo) {
+    if (use_duo(lanes, n)) {
+      hipLaunchKernelGGL((k_gjk_duo<EMIT, Src>), dim3((unsigned)n), dim3(128), 0, st, src, o, n, p,
+                         b, (unsigned*)ws, (const int*)((char*)ws + ws_list_off()),
+                         (EpaJob*)((char*)ws + ws_jobs_off(n)));
+      return hipGetLastError();
+    }
+  }
   switch (lanes) {
     case 8: return launch_gjk<8, EMIT>(src, o, n, p, b, wpb, ws, st);
     case 16: return launch_gjk<16, EMIT>(src, o, n, p, b, wpb, ws, st);
@@ -997,6 +1081,14 @@ static hipError_t launch_bucketed(int mode, const Src& src, const OutArgs& o, in
     done[cls] = true;
     // one launch per EPA class, shaped by the first bucket of the class
     const int w = cfg.epa_waves[b];
+    if constexpr (Src::kDuo) {
+      if (use_duo(cfg.epa_lanes[b], n)) {
+        hipLaunchKernelGGL((k_epa_duo<Src>), dim3((unsigned)n), dim3(128), 0, st, src, o, p, cls, c,
+                           (const EpaJob*)((char*)ws + ws_jobs_off(n)));
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        continue;
+      }
+    }
     switch (cfg.epa_lanes[b]) {
       case 16: e = launch_epa_list<16>(src, o, n, p, cls, w, ws, st); break;
       case 32: e = launch_epa_list<32>(src, o, n, p, cls, w, ws, st); break;
