@@ -114,8 +114,8 @@ ogjk_status ogjk_sync(void* stream);
  * a GJK kernel over every pair, then an EPA kernel over every pair, one group
  * per pair each, non-persistent (GJK/gpu/openGJK.cu:2968-3004), where GJK
  * lanes may also be 1 (one thread per pair); other calls run as fused 0.
- * A launch over so few pairs that SIMDs would stay idle doubles the lanes per
- * pair until it fills the chip or a pair has a whole wave (same results).
+ * A launch over few pairs (some thousands) doubles the lanes per pair until it
+ * fills the chip or a pair has a whole wave (same results).
  * Not synchronised with launches issued concurrently from other threads. */
 ogjk_status ogjk_set_config(int gjk_lanes, int epa_lanes, int fused);
 

@@ -11,18 +11,20 @@
 #ifndef OGJK_GJK_WAVES
 #define OGJK_GJK_WAVES 3
 #endif
-// Clustered and posed bodies carry more live state through GJK.
+// With the simplex in LDS the clustered 64-lane kernel needs 121 registers and
+// runs 4 waves/SIMD by itself; the posed one needs 133 and is held to 128 (12
+// B/lane of scratch; 50K posed pairs 432 us).
 #ifndef OGJK_GJK_WAVES_WIDE
 #define OGJK_GJK_WAVES_WIDE 3
 #endif
 #ifndef OGJK_GJK_WAVES_POSED
 #define OGJK_GJK_WAVES_POSED 4
 #endif
-// EPA: float scenes swept whole run faster at 3 waves/SIMD even though the
-// compiler then spills 80 B/lane (100K x 64: 1.22 -> 1.12 ms); the 64-lane
-// kernels of clustered scenes fit 3 waves without spilling (the group is the
-// wave, so the pair's descriptors are scalar); narrower clustered kernels
-// (200+ B/lane at 3), posed and the other sources stay at 2.
+// EPA: float scenes swept whole run at 3 waves/SIMD with 44 B/lane of scratch at
+// 32 lanes (179 registers wanted); the 64-lane kernels of clustered scenes fit 3
+// waves with 161 registers (at 4: 96 B/lane, 100K uneven pairs 1,550 -> 1,625 us);
+// posed ones stay at 2 (at 3: 112 B/lane, 375-390 -> 397 us over 50K pairs), and
+// so do narrower clustered ones and the other sources.
 #ifndef OGJK_EPA_WAVES
 #define OGJK_EPA_WAVES 2
 #endif
@@ -630,6 +632,10 @@ __global__ void __launch_bounds__(256) k_scatter(Src src, int n, BucketPlan plan
   }
 }
 
+// Bound by instruction issue and by the latency of one pair's chain: at 8 lanes
+// 7,750 vector instructions a wave keep the SIMDs 68% busy (100K pairs of 64
+// vertices 232 us, 258 with the sub-distance as a branching tree and the simplex
+// in registers), at 64 lanes 74% (100K uneven pairs 951 us, 1,297 before).
 // GJK over one bucket, one group per list entry and one wave per block: the
 // hardware dispatcher balances pairs of different sizes wave by wave, and no
 // wave waits for the slowest pair of a larger block.  Blocks past the bucket's
@@ -683,7 +689,11 @@ __global__ void __launch_bounds__(256, Src::kGjkWaves)
 }
 
 // EPA over one class's job list, persistent: the groups of a wave claim jobs
-// together from sliced cursors until the list is exhausted.
+// together from sliced cursors until the list is exhausted.  Bound by issue and
+// by dependent chains, not by memory: 60K penetrating pairs of 64 vertices at 32
+// lanes 620 us (834 with all faces in registers and every edge compared with
+// every other), 46K uneven ones at 64 lanes 1,550 us (1,851), vector units 64% and
+// 53% busy.
 template <int LPP, class Src>
 __global__ void __launch_bounds__(256, Src::template kEpaWaves<LPP>)
     k_epa_list(Src src, OutArgs out, BucketPlan plan, int cls, unsigned* c, const EpaJob* jobs) {
@@ -723,7 +733,8 @@ __global__ void __launch_bounds__(256, Src::template kEpaWaves<LPP>)
 // Clustered pairs, a block of two waves each (see Duo).  A whole-wave query of
 // a large body is a chain of some ten memory round trips and a lone wave on its
 // SIMD takes about ten cycles an instruction, so where the pairs are too few to
-// fill the chip a second wave takes half of the queries.
+// fill the chip a second wave takes half of the queries (1,000 pairs of 50,000
+// vertices: GJK 250 -> 155 us, EPA 950 -> 620 us).
 template <bool EMIT, class Src>
 __global__ void __launch_bounds__(128)
     k_gjk_duo(Src src, OutArgs out, int n, BucketPlan plan, int bucket, unsigned* c,
@@ -963,18 +974,31 @@ static hipError_t launch_pairs(const Src& src, const OutArgs& o, int n, hipStrea
 }
 
 // Lanes per pair of a launch over n pairs: the configured number, doubled while
-// the launch would still leave a SIMD idle (one wave for each, 1,024 on the
-// chip).  Nothing else runs there, so a wider group only shortens its pair's
-// chain: no waiting for the other pairs of the wave and fewer sweep steps.
+// the wider launch would have at most `waves` waves for each of the chip's 1,024
+// SIMDs.  A wider group shortens its pair's chain: no waiting for the other pairs
+// of its wave, fewer sweep steps.  It pays as long as the waves run side by side,
+// for EPA longer than for GJK, as only the penetrating pairs reach it.  Measured
+// on pairs of 64 vertices configured as 8 and 32 lanes, narrow -> wide:
+//   GJK 8, EPA 32:      64 pairs 110 ->  67 us with 64 and 64
+//   GJK 32, EPA 32:  1,500 pairs 181 -> 127 us with 64 and 64
+//   GJK 16, EPA 32:  3,000 pairs 188 -> 184 us with 32, 142 with 64 and 64
+//   GJK 8, EPA 32:   4,096 pairs 223 -> 182 us with 32 and 64
+//   GJK 8, EPA 32:   6,000 pairs 238 -> 227 us with 16 and 32
+//   GJK 8, EPA 32:   8,000 pairs 254 -> 263 us with 32 and 32
 constexpr int64_t kChipLanes = 1024 * 64;
-static int fill_lanes(int lanes, int n) {
-  while (lanes < 64 && 2 * (int64_t)lanes * n <= kChipLanes) lanes *= 2;
+constexpr int kFillGjk = 2, kFillEpa = 4;
+static int fill_lanes(int lanes, int n, int waves) {
+  while (lanes < 64 && 2 * (int64_t)lanes * n <= waves * kChipLanes) lanes *= 2;
   return lanes;
 }
 
-// Two waves to a pair up to here: two waves on every SIMD then, and past it
-// more waves than pairs would only repeat the work that both waves of a pair do.
-static bool use_duo(int lanes, int n) { return lanes == 64 && 64 * (int64_t)n <= kChipLanes; }
+// Two waves to a clustered pair up to here.  One and two waves measured (GJK and
+// EPA): pairs of 20,000 vertices 1,064 and 670 us for 2,000 pairs, 1,467 and 1,242
+// for 6,000; uneven pairs of 4-4,096 vertices 542 and 372 us for 2,000, 647 and 612
+// for 8,000, 851 and 873 for 16,000, where what both waves do alike costs more than
+// the shorter chain gains.
+constexpr int kDuoPairs = 8192;
+static bool use_duo(int lanes, int n) { return lanes == 64 && n <= kDuoPairs; }
 
 // Resident grid for a persistent launch over at most n items.
 static unsigned persistent_blocks(int n, int gpb, unsigned cap = 4096u) {
@@ -1034,7 +1058,7 @@ static hipError_t gjk_by_lanes(int lanes, const Src& src, const OutArgs& o, int 
 
 template <int MODE, class Src>
 static hipError_t pairs_by_lanes(const Src& src, const OutArgs& o, int n, hipStream_t st) {
-  switch (fill_lanes(g_cfg.epa_lanes[0], n)) {
+  switch (fill_lanes(g_cfg.epa_lanes[0], n, kFillEpa)) {
     case 16: return launch_pairs<16, MODE>(src, o, n, st);
     case 32: return launch_pairs<32, MODE>(src, o, n, st);
     default: return launch_pairs<64, MODE>(src, o, n, st);
@@ -1048,8 +1072,8 @@ static hipError_t launch_bucketed(int mode, const Src& src, const OutArgs& o, in
                                   hipStream_t st) {
   LaunchConfig cfg = g_cfg;
   for (int b = 0; b < cfg.nb; b++) {
-    cfg.gjk_lanes[b] = fill_lanes(cfg.gjk_lanes[b], n);
-    cfg.epa_lanes[b] = fill_lanes(cfg.epa_lanes[b], n);
+    cfg.gjk_lanes[b] = fill_lanes(cfg.gjk_lanes[b], n, kFillGjk);
+    cfg.epa_lanes[b] = fill_lanes(cfg.epa_lanes[b], n, kFillEpa);
   }
   const BucketPlan p = plan_of(cfg);
   unsigned* c = (unsigned*)ws;

@@ -37,12 +37,11 @@ def _join(batches):
 
 
 def _exact(torch, b, shape, cluster_min=None):
-    # launches that would leave SIMDs idle use wider groups than configured, or two
-    # waves to a clustered pair:
-    # as it is, and repeated until the configured ones run
+    # launches over few pairs use wider groups than configured, or two waves to a
+    # clustered pair: as it is, and repeated until the configured ones run
     ref = oracle_run(oracle.GJK_EPA, b)
     once = np.stack([b.pa, b.pb], 1).astype(np.int32)
-    for reps in (1, 1 + 65536 // (shape[0] * b.n_pairs)):
+    for reps in (1, 1 + 8192 // b.n_pairs):
         pairs = torch.from_numpy(np.ascontiguousarray(np.tile(once, (reps, 1)))).cuda()
         ogjk.set_config(*shape, 0)
         try:
