@@ -13,8 +13,8 @@
 //  * Completion thread: polls the events of running slots, copies each
 //    request's results to the caller's buffers, stamps its latency (submit to
 //    results on the host) and wakes its waiter.
-// Each pair is computed by the same kernels and lane layout whatever batch it
-// lands in, so a request's results do not depend on the mix.
+// Every launch shape gives a pair the same bits (few pairs take wider groups),
+// so a request's results do not depend on the batch it lands in.
 //
 // Shutdown (ogjk_server_destroy): new submissions are refused, requests not
 // yet launched are cancelled (their wait returns an error), launched batches
