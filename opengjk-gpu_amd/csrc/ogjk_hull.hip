@@ -463,10 +463,10 @@ struct BlockHull {
   static constexpr int kWaves = T / kWave;
   static constexpr bool kPlanes = NP <= 512;
   using Face = std::conditional_t<kPlanes, Tri, uint32_t>;
-  static constexpr int kSeg = kPlanes ? 128 : 256;  // visible faces a wave notes at an insertion
+  static constexpr int kSeg = kPlanes ? 128 : 256;  // visible faces a wave lists at an insertion
   static constexpr int kRoom = kPlanes ? 384 : 2048;  // slots an insertion finds free
   static constexpr int kRow = kWave / kWaves;  // of which the first wave takes these in one go
-  Face face[S];                     // ids: 3 x 10 bits, kDead
+  Face face[S];                     // ids: 3 x 10 bits, kDead, kLate
   float4 pt[NP];
   std::conditional_t<NP <= 512, EdgeBits<NP>, EdgeHash> edges;
   uint32_t seg[kWaves][kSeg];  // vertex ids of the visible faces each wave found
@@ -475,7 +475,9 @@ struct BlockHull {
   int full;                    // an edge found no place
   int id[4];
 };
-constexpr uint32_t kDead = 0x80000000u;
+// Flags beside a slot's 3 x 10 bits of ids: the face has left, and it left at the
+// insertion at hand and is on no wave's list.
+constexpr uint32_t kDead = 0x80000000u, kLate = 0x40000000u;
 
 __device__ __forceinline__ uint32_t& ids_of(Tri& f) { return f.ids; }
 __device__ __forceinline__ uint32_t& ids_of(uint32_t& f) { return f; }
@@ -591,8 +593,8 @@ __device__ int hull_block(const float* __restrict__ P, int n, int cap, BlockHull
           const int f = base + u * kWave + lane;
           const uint32_t ids = ids_of(F[u]);
           const uint32_t x = ids & 1023u, y = (ids >> 10) & 1023u, z = ids >> 20;
-          ids_of(s.face[f]) = ids | kDead;
           const int r = found + rank_below(bv, lane);
+          ids_of(s.face[f]) = ids | (r < B::kSeg ? kDead : kDead | kLate);
           if (r < B::kSeg) s.seg[wave][r] = ids;
           const bool i0 = s.edges.insert(x, y), i1 = s.edges.insert(y, z), i2 = s.edges.insert(z, x);
           if (!i0 || !i1 || !i2) s.full = 1;
@@ -608,7 +610,7 @@ __device__ int hull_block(const float* __restrict__ P, int n, int cap, BlockHull
     if (ballot(here != 0) == 0) continue;
     if (wave == 0) {
       int status = 4, nh = 0, nv = 0, at = tail;
-      if (ballot(here > B::kSeg) != 0 || s.full) {
+      if (s.full) {
         status = kToBig;
       } else {
         // Each lane takes a visible face (valid: ids), in slot order: its
@@ -652,6 +654,34 @@ __device__ int hull_block(const float* __restrict__ P, int n, int cap, BlockHull
           nv = __popcll(ballot(valid));
           fan(valid, ids);
           if (valid) unmark(ids);
+        } else if (ballot(here > B::kSeg) != 0) {
+          // A wave saw more than its list holds: new faces sit together at the
+          // tail, so a cloud whose face list grows fast has most of its visible
+          // ones in a few waves' runs.  Those past a list's end are found again
+          // by their flag, in the slots of the wave's run, behind the listed ones.
+          const auto each = [&](const auto& f) {
+            for (int w = 0; w < B::kWaves; w++) {
+              const int c = cnt[w], listed = min(c, B::kSeg);
+              for (int base = 0; base < listed; base += kWave)
+                f(base + lane < listed, base + lane < listed ? s.seg[w][base + lane] : 0u, -1);
+              if (c == listed) continue;
+              const int stop = min(tail, (w + 1) * run);
+              for (int base = w * run; base < stop; base += kWave) {
+                const int slot = base + lane;
+                const uint32_t ids = slot < stop ? ids_of(s.face[slot]) : 0u;
+                f((ids & kLate) != 0, ids & ~(kDead | kLate), slot);
+              }
+            }
+          };
+          nv = 0;
+          each([&](bool valid, uint32_t ids, int) {
+            nv += __popcll(ballot(valid));
+            fan(valid, ids);
+          });
+          each([&](bool valid, uint32_t ids, int slot) {
+            if (valid) unmark(ids);
+            if (valid && slot >= 0) ids_of(s.face[slot]) = ids | kDead;
+          });
         } else {
           int pre[B::kWaves + 1];  // visible faces of the waves before
           pre[0] = 0;
