@@ -7,9 +7,9 @@
 // faces with a 6x signed volume above 1e-7 (FP32) visible, visible faces
 // removed in place, one new face per horizon edge appended in the order the
 // visible faces and their edges are listed.  The reference runs that loop on
-// one CPU thread per cloud; here half a wave, a wave or a block owns a cloud
-// (by its size) and each step is data-parallel over it: visibility over faces,
-// the horizon test over the visible faces' edges, order-preserving
+// one CPU thread per cloud; here 16 lanes, a wave or a block own a cloud (by its
+// size and its face count) and each step is data-parallel over it: visibility
+// over faces, the horizon test over the visible faces' edges, order-preserving
 // compaction and appends by ballots and prefix counts.  Moments are summed in
 // face order, as the reference sums them (:433-481), so they are
 // bit-identical too.
@@ -27,17 +27,43 @@ ogjk_status ogjk_fail(ogjk_status code, const char* fmt, ...);
 
 namespace {
 
+using ogjk::wave_sync;
 using ogjk::xpair;
 
 constexpr int kWave = 64;
 
-// Results of d_nfaces that pass a cloud on to the next kernel of the call
-// (no result that a caller sees: the last kernel leaves none of them).
-constexpr int kToBlock = -100, kToBig = -101, kToGeneral = -102, kNowhere = -103;
+// Results of d_nfaces that pass a cloud on to the next kernel of the call, to be
+// started again or to go on from its saved state (no result that a caller sees:
+// the last kernel leaves none of them).
+constexpr int kToWave = -100, kSaved = -101;
+
+// The arguments of a build: cloud m's points, its part of the output buffer and
+// of the workspace (three words per face of its capacity in each).
+struct HullArgs {
+  const float* pts;
+  const int64_t* off;
+  const int32_t* cnt;
+  int nm;
+  const int64_t* face_off;
+  int64_t total_faces;
+  int32_t* faces;
+  int32_t* nfaces;
+  int32_t* scratch;
+  __device__ bool range_ok(int64_t m) const {
+    return face_off[m] >= 0 && face_off[m + 1] >= face_off[m] && face_off[m + 1] <= total_faces;
+  }
+  __device__ int64_t cap64(int64_t m) const { return face_off[m + 1] - face_off[m]; }
+  __device__ int cap(int64_t m) const {
+    return cap64(m) < 0x7fffffff ? (int)cap64(m) : 0x7fffffff;
+  }
+  __device__ const float* points(int64_t m) const { return pts + 3 * off[m]; }
+  __device__ int32_t* out(int64_t m) const { return faces + 3 * face_off[m]; }
+  __device__ int32_t* work(int64_t m) const { return scratch + 3 * face_off[m]; }
+};
 
 // A point of the working set and a face with its plane: the normal of
 // (v0, v1, v2) as vol6 forms it, and the packed vertex ids.
-struct Tri {
+struct alignas(16) Tri {
   float nx, ny, nz;
   uint32_t ids;
 };
@@ -64,12 +90,6 @@ __device__ __forceinline__ uint64_t ballot(bool v) { return __ballot(v); }
 
 __device__ __forceinline__ int rank_below(uint64_t mask, int lane) {
   return ogjk::lanes_below<kWave>(mask, lane);
-}
-
-// Orders the LDS accesses of the lanes of one wave.
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  __builtin_amdgcn_wave_barrier();
 }
 
 template <int L, int M = 1>
@@ -201,29 +221,27 @@ __device__ __forceinline__ int init_corner(const int (&id)[4], int f, int j) {
 
 // ------------------------------------------------- clouds of few points
 //
-// Clouds of NMIN..NMAX points, L lanes each, the whole working set in LDS.
+// Clouds of up to 32 points, 16 lanes each, the whole working set in LDS.
 // Bound by vector instructions (a step has ~20 faces and ~12 edges to look
-// at), hence: as many lanes as a small hull fills (16 for up to 32 points:
-// four clouds share a wave's instructions), the plane of each face kept from
-// its creation (an insertion reads it and one corner instead of three
-// gathered corners and a cross product), and the horizon test by one bit per
-// directed edge of the visible faces (row = start, bit = end) instead of a
-// search of their list.  100,000 clouds of 8-32 points: 0.29 ms at 16 lanes,
-// 0.33 at 32, 0.90 with one wave per cloud and no kept planes.
-template <int NMAX, int FMAX>
-struct GroupHull {
-  static constexpr int W = (NMAX + 31) / 32;  // words of a row of edge bits
-  float4 pt[NMAX];
-  Tri face[FMAX];
-  uint32_t vis[FMAX];
-  uint32_t adj[NMAX * W];
+// at), hence: as many lanes as a small hull fills (four clouds share a wave's
+// instructions), the plane of each face kept from its creation (an insertion
+// reads it and one corner instead of three gathered corners and a cross
+// product), and the horizon test by one bit per directed edge of the visible
+// faces (word = start, bit = end) instead of a search of their list.  100,000
+// clouds of 8-32 points: 0.29 ms at 16 lanes, 0.33 at 32, 0.90 with one wave
+// per cloud and no kept planes.
+constexpr int kFewLanes = 16, kFewPoints = 32, kFewFaces = 96;
+
+struct FewHull {
+  float4 pt[kFewPoints];
+  Tri face[kFewFaces];
+  uint32_t vis[kFewFaces];
+  uint32_t adj[kFewPoints];
 };
 
-template <int L, int NMAX, int FMAX>
-__device__ __forceinline__ int hull_group(const float* __restrict__ P, int n, int cap,
-                                          GroupHull<NMAX, FMAX>& s, int lane) {
-  constexpr int W = GroupHull<NMAX, FMAX>::W;
-  static_assert(NMAX <= 256, "vertex ids are packed in 8 bits");
+__device__ __forceinline__ int hull_few(const float* __restrict__ P, int n, int cap, FewHull& s,
+                                        int lane) {
+  constexpr int L = kFewLanes;
   const auto pt = [&](int i) { return s.pt[i]; };
   float lo[3], hi[3];
   int lo_i[3], hi_i[3];
@@ -245,7 +263,7 @@ __device__ __forceinline__ int hull_group(const float* __restrict__ P, int n, in
       if (hi_i[k] < 0 || p[k] > hi[k]) { hi[k] = p[k]; hi_i[k] = i; }
     }
   }
-  for (int i = lane; i < NMAX * W; i += L) s.adj[i] = 0u;
+  for (int i = lane; i < kFewPoints; i += L) s.adj[i] = 0u;
   if (ogjk::group_any<L>(bad)) return -2;
   wave_sync();
   int id[4];
@@ -280,9 +298,9 @@ __device__ __forceinline__ int hull_group(const float* __restrict__ P, int n, in
       if (v) {
         s.vis[nv + r] = F.ids;
         const uint32_t a = F.ids & 255u, b = (F.ids >> 8) & 255u, c = F.ids >> 16;
-        atomicOr(&s.adj[a * W + (b >> 5)], 1u << (b & 31u));
-        atomicOr(&s.adj[b * W + (c >> 5)], 1u << (c & 31u));
-        atomicOr(&s.adj[c * W + (a >> 5)], 1u << (a & 31u));
+        atomicOr(&s.adj[a], 1u << b);
+        atomicOr(&s.adj[b], 1u << c);
+        atomicOr(&s.adj[c], 1u << a);
       } else if (in) {
         s.face[w + lane - r] = F;  // lanes below that are not visible
       }
@@ -305,178 +323,554 @@ __device__ __forceinline__ int hull_group(const float* __restrict__ P, int n, in
         const uint32_t ids = s.vis[k];
         a = (ids >> (8 * e)) & 255u;
         b = (e == 2 ? ids : ids >> (8 * e + 8)) & 255u;
-        hz = !((s.adj[b * W + (a >> 5)] >> (a & 31u)) & 1u);
+        hz = !((s.adj[b] >> a) & 1u);
       }
       const auto bl = ogjk::lanes_where<L>(hz);
       const int r = w + nh + ogjk::lanes_below<L>(bl, lane);
-      if (hz && r < FMAX) s.face[r] = make_tri(s.pt[a], s.pt[b], Q, a | b << 8 | (uint32_t)q << 16);
+      if (hz && r < kFewFaces)
+        s.face[r] = make_tri(s.pt[a], s.pt[b], Q, a | b << 8 | (uint32_t)q << 16);
       nh += ogjk::count_lanes<L>(bl);
     }
     wave_sync();
-    if constexpr (NMAX * W <= 2 * L) {
-      for (int i = lane; i < NMAX * W; i += L) s.adj[i] = 0u;
-    } else {
-      for (int h = lane; h < ne; h += L) {
-        const int k = h / 3, e = h - 3 * k;
-        const uint32_t ids = s.vis[k];
-        const uint32_t a = (ids >> (8 * e)) & 255u;
-        const uint32_t b = (e == 2 ? ids : ids >> (8 * e + 8)) & 255u;
-        s.adj[a * W + (b >> 5)] = 0u;
-      }
-    }
+    for (int i = lane; i < kFewPoints; i += L) s.adj[i] = 0u;
     nf = w + nh;
     if (nf > cap) return -1;
-    if (nf > FMAX) return kToBlock;
+    if (nf > kFewFaces) return kToWave;
     wave_sync();
   }
   return nf;
 }
 
-// Clouds of NMIN..NMAX points, kWave / L to a one-wave block; gridDim.x *
-// kWave / L groups take the clouds in turn.
-template <int L, int NMIN, int NMAX, int FMAX>
-__global__ __launch_bounds__(kWave) void k_hull_group(const float* __restrict__ pts,
-                                                      const int64_t* __restrict__ off,
-                                                      const int32_t* __restrict__ cnt, int nm,
-                                                      const int64_t* __restrict__ face_off,
-                                                      int64_t total_faces,
-                                                      int32_t* __restrict__ faces,
-                                                      int32_t* __restrict__ nfaces) {
-  constexpr int G = kWave / L;
-  __shared__ GroupHull<NMAX, FMAX> lds[G];
-  GroupHull<NMAX, FMAX>& s = lds[threadIdx.x / L];
+// The clouds of up to kFewPoints points, 4 to a one-wave block; gridDim.x * 4
+// groups take the clouds in turn.
+__global__ __launch_bounds__(kWave) void k_hull_few(HullArgs h) {
+  constexpr int L = kFewLanes, G = kWave / L;
+  __shared__ FewHull lds[G];
+  FewHull& s = lds[threadIdx.x / L];
   const int lane = threadIdx.x & (L - 1);
   const int groups = gridDim.x * G;
   const int g = blockIdx.x * G + threadIdx.x / L;
   // L clouds of this group at a time, the ones of its class by ballot
-  for (int64_t first = g; first < nm; first += (int64_t)groups * L) {
+  for (int64_t first = g; first < h.nm; first += (int64_t)groups * L) {
     const int64_t mine = first + (int64_t)groups * lane;
     int n_mine = -1;
-    if (mine < nm) n_mine = cnt[mine] < 0 ? 0 : cnt[mine];
-    uint64_t todo = ogjk::group_ballot<L>(n_mine >= NMIN && n_mine <= NMAX);
+    if (mine < h.nm) n_mine = h.cnt[mine] < 0 ? 0 : h.cnt[mine];
+    uint64_t todo = ogjk::group_ballot<L>(n_mine >= 0 && n_mine <= kFewPoints);
     while (todo != 0) {
       const int src = (int)__builtin_ctzll(todo);
       todo &= todo - 1;
       const int64_t m = first + (int64_t)groups * src;
       const int n = __shfl(n_mine, src, L);
-      const int64_t f0 = face_off[m], cap64 = face_off[m + 1] - f0;
       int nf;
-      if (f0 < 0 || cap64 < 0 || face_off[m + 1] > total_faces) {
+      if (!h.range_ok(m)) {
         nf = -3;
       } else if (n < 4) {
         nf = 0;
       } else {
-        nf = hull_group<L>(pts + 3 * off[m], n, cap64 < 0x7fffffff ? (int)cap64 : 0x7fffffff, s,
-                           lane);
+        nf = hull_few(h.points(m), n, h.cap(m), s, lane);
       }
       wave_sync();
-      int32_t* out = faces + 3 * f0;
+      int32_t* out = h.out(m);
       for (int f = lane; f < nf; f += L) {
         const uint32_t ids = s.face[f].ids;
         out[3 * f] = (int32_t)(ids & 255u);
         out[3 * f + 1] = (int32_t)((ids >> 8) & 255u);
         out[3 * f + 2] = (int32_t)(ids >> 16);
       }
-      if (lane == 0) nfaces[m] = nf;
+      if (lane == 0) h.nfaces[m] = nf;
     }
   }
 }
 
-// ------------------------------------------------ clouds of more points
+// ------------------------------------------------------- a wave per cloud
 //
-// A block of T threads per cloud.  Insertions are serial and a cloud of 500
-// points has a thousand faces to test at each, so one wave per cloud leaves
-// the largest cloud of a call to run alone for milliseconds (4.4 ms for 2,000
-// ellipsoid clouds of 8-512 points, now 1.5 in all; an insertion into 512
-// points took 8 us, now 1.7).  The
-// whole block tests the faces (planes kept in LDS, as above) and notes the
-// visible ones; then the first wave alone does the short ordered part
-// (horizon, new faces): two block barriers per insertion, and what counts is
-// the chain of LDS round trips between them, so lists that would be written
-// and read again are avoided.  A face that leaves stays behind as a dead
-// slot, so nothing moves: slots are in creation order, which is the order the
-// reference's compaction keeps, and the first wave closes the gaps now and
-// then.  Each wave tests one contiguous run of slots, so the waves' lists of
-// visible faces joined together are in slot order.
+// The faces in LDS, the points where they are.  Most insertions into a large
+// cloud see no face, and then a step is one look at each face and nothing
+// else; many clouds at once want as many waves as there is room for, and a
+// barrier per insertion costs more than the other waves of a block bring: a
+// block per cloud took 8.1 ms for 3,000 clouds of 1,024 points, most of them
+// inside (0.64 ms with one wave each and the faces in global memory).  Hence:
+//   * a face is 32 bytes with its plane and its first corner, so that the
+//     visibility test is two LDS reads and no gather;
+//   * a lane holds one of 64 points at a time, an insertion's point comes from
+//     there by v_readlane;
+//   * the visible faces' directed edges are listed as keys (start | end << 16)
+//     and an edge is on the horizon if the list does not hold the reverse key:
+//     up to 16 edges (as nearly always) are compared with all others in one
+//     step, a quarter of the list per 16 lanes.
+// When the list outgrows FB faces the cloud's state is saved (see load_state) and
+// a kernel with more room goes on from there.
+constexpr int kWavePoints = 65536;  // ids are 16 bits
+
+template <int FB>
+struct WaveHull {
+  struct alignas(16) Corner {
+    float y, z;
+    uint32_t ab, c;  // ids: a | b << 16, c
+  };
+  float4 nx[FB];  // normal, x of corner a
+  Corner co[FB];  // y and z of corner a
+  alignas(16) uint32_t key[3 * FB + kWave];
+};
+
+// Where a cloud stands between two insertions: its faces in order in the
+// output buffer, and at the start of its workspace six words: the number of
+// faces, the next point, the first tetrahedron's points.  Only states of more
+// faces than a wave's room are saved, so the words have a place.
+__device__ __forceinline__ void load_state(const int32_t* save, int& nf, int& next, int (&id)[4]) {
+  // not from the scalar cache: a wave of the same block may have written them
+  const auto word = [&](int k) {
+    return __builtin_amdgcn_readfirstlane(
+        __hip_atomic_load(save + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+  };
+  nf = word(0);
+  next = word(1);
+#pragma unroll
+  for (int k = 0; k < 4; k++) id[k] = word(2 + k);
+}
+__device__ __forceinline__ void store_state(int32_t* save, int nf, int next, const int (&id)[4]) {
+  save[0] = nf;
+  save[1] = next;
+#pragma unroll
+  for (int k = 0; k < 4; k++) save[2 + k] = id[k];
+}
+
+// The first tetrahedron's points of P[0..n), or the status that ends the build.
+__device__ __forceinline__ int hull_begin(const float* __restrict__ P, int n, int cap, int lane, int (&id)[4]) {
+  const auto pt = [&](int i) {
+    return make_float4(P[3 * (int64_t)i], P[3 * (int64_t)i + 1], P[3 * (int64_t)i + 2], 0.0f);
+  };
+  float lo[3], hi[3];
+  int lo_i[3], hi_i[3];
+  bool bad = false;
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    lo[k] = INFINITY;
+    hi[k] = -INFINITY;
+    lo_i[k] = hi_i[k] = -1;
+  }
+  for (int i = lane; i < n; i += kWave) {
+    const float4 p4 = pt(i);
+    const float p[3] = {p4.x, p4.y, p4.z};
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      bad |= !isfinite(p[k]);
+      if (lo_i[k] < 0 || p[k] < lo[k]) { lo[k] = p[k]; lo_i[k] = i; }
+      if (hi_i[k] < 0 || p[k] > hi[k]) { hi[k] = p[k]; hi_i[k] = i; }
+    }
+  }
+  if (ballot(bad) != 0) return -2;
+  if (!first_tetrahedron<kWave>(pt, n, lane, lo, lo_i, hi, hi_i, id)) return 0;
+  return cap < 4 ? -1 : 4;
+}
+
+// Returns the face count (faces in s), a status of d_nfaces, or kSaved.
+template <int FB>
+__device__ __forceinline__ int hull_wave(const float* __restrict__ P, int n, int cap, WaveHull<FB>& s,
+                         int32_t* out, int32_t* save, bool resume, int lane) {
+  using Corner = typename WaveHull<FB>::Corner;
+  const auto pt = [&](uint32_t i) { return make_float4(P[3 * i], P[3 * i + 1], P[3 * i + 2], 0.0f); };
+  const auto put = [&](int f, uint32_t a, uint32_t b, uint32_t c, float4 A, float4 B, float4 C) {
+    const Tri t = make_tri(A, B, C, 0u);
+    s.nx[f] = make_float4(t.nx, t.ny, t.nz, A.x);
+    s.co[f] = Corner{A.y, A.z, a | b << 16, c};
+  };
+  int id[4] = {0, 0, 0, 0};
+  int nf = 4, q = 0;
+  wave_sync();
+  if (resume) {
+    load_state(save, nf, q, id);
+    if (nf > FB) return kSaved;
+    for (int f = lane; f < nf; f += kWave) {
+      const uint32_t a = out[3 * f], b = out[3 * f + 1], c = out[3 * f + 2];
+      put(f, a, b, c, pt(a), pt(b), pt(c));
+    }
+  } else {
+    const int st = hull_begin(P, n, cap, lane, id);
+    if (st != 4) return st;
+    if (lane < 4) {
+      const uint32_t a = init_corner(id, lane, 0), b = init_corner(id, lane, 1),
+                     c = init_corner(id, lane, 2);
+      put(lane, a, b, c, pt(a), pt(b), pt(c));
+    }
+  }
+  wave_sync();
+  for (int from = q & ~(kWave - 1); from < n; from += kWave) {
+    const float4 mine = pt(min(from + lane, n - 1));
+    const int end = min(n, from + kWave);
+    for (q = max(q, from); q < end; q++) {
+      if (q == id[0] || q == id[1] || q == id[2] || q == id[3]) continue;
+      const float4 Q = make_float4(ogjk::lane_value(mine.x, q - from),
+                                   ogjk::lane_value(mine.y, q - from),
+                                   ogjk::lane_value(mine.z, q - from), 0.0f);
+      // Visible faces leave the list (in place: a chunk is read before it is
+      // written, and only to lower positions) and list their edges.
+      constexpr int U = 2;  // chunks in flight
+      int nv = 0, w = 0;
+      for (int base = 0; base < nf; base += U * kWave) {
+        float4 N[U];
+        Corner A[U];
+        bool v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const int f = min(base + u * kWave + lane, nf - 1);
+          N[u] = s.nx[f];
+          A[u] = s.co[f];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const Tri t{N[u].x, N[u].y, N[u].z, 0u};
+          v[u] = base + u * kWave + lane < nf &&
+                 vol6(t, make_float4(N[u].w, A[u].y, A[u].z, 0.0f), Q) > 1e-7f;
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const uint64_t bv = ballot(v[u]);
+          const int left = max(min(nf - base - u * kWave, kWave), 0);
+          if (bv == 0 && nv == 0) {
+            w += left;
+            continue;
+          }
+          const int r = rank_below(bv, lane);
+          if (v[u]) {
+            uint32_t* k = s.key + 3 * (nv + r);
+            const uint32_t a = A[u].ab & 0xffffu, b = A[u].ab >> 16, c = A[u].c;
+            k[0] = A[u].ab;
+            k[1] = b | c << 16;
+            k[2] = c | a << 16;
+          } else if (lane < left) {
+            s.nx[w + lane - r] = N[u];  // lanes below that are not visible
+            s.co[w + lane - r] = A[u];
+          }
+          const int c = __popcll(bv);
+          nv += c;
+          w += left - c;
+        }
+      }
+      if (nv == 0) continue;
+      // the list filled up to a multiple of 64 with a key that is no reverse:
+      // an edge from a point to itself is on no face
+      const int ne = 3 * nv;
+      if (ne + lane < ((ne + kWave - 1) & ~(kWave - 1))) s.key[ne + lane] = 0u;
+      wave_sync();
+      // horizon: directed edges of visible faces whose reverse no visible face
+      // has, in (visible face, edge) order; each is the base of a new face
+      int nh = 0;
+      const auto four = [&](int at) {
+        uint4 k;
+        __builtin_memcpy(&k, __builtin_assume_aligned(s.key + at, 16), sizeof(k));
+        return k;
+      };
+      const auto any_of = [](uint4 k, uint32_t x) {
+        return k.x == x || k.y == x || k.z == x || k.w == x;
+      };
+      for (int base = 0; base < ne; base += kWave) {
+        uint32_t k;
+        bool hz;
+        if (ne <= 16) {
+          k = s.key[lane & 15];
+          const uint64_t b = ballot(any_of(four(lane >> 4 << 2), k << 16 | k >> 16));
+          hz = lane < ne && !(((b | b >> 16 | b >> 32 | b >> 48) >> lane) & 1u);
+        } else {
+          k = s.key[base + lane];
+          bool found = false;
+          for (int j = 0; j < ne; j += 4) found |= any_of(four(j), k << 16 | k >> 16);
+          hz = base + lane < ne && !found;
+        }
+        const uint64_t bl = ballot(hz);
+        const int r = w + nh + rank_below(bl, lane);
+        if (hz) {
+          const uint32_t a = k & 0xffffu, b = k >> 16;
+          if (r < FB) {
+            put(r, a, b, (uint32_t)q, pt(a), pt(b), Q);
+          } else if (r < cap) {  // straight to where the state is saved
+            out[3 * r] = (int32_t)a;
+            out[3 * r + 1] = (int32_t)b;
+            out[3 * r + 2] = q;
+          }
+        }
+        nh += __popcll(bl);
+      }
+      wave_sync();
+      nf = w + nh;
+      if (nf > cap) return -1;
+      if (nf > FB) {
+        for (int f = lane; f < FB; f += kWave) {
+          out[3 * f] = (int32_t)(s.co[f].ab & 0xffffu);
+          out[3 * f + 1] = (int32_t)(s.co[f].ab >> 16);
+          out[3 * f + 2] = (int32_t)s.co[f].c;
+        }
+        if (lane == 0) store_state(save, nf, q + 1, id);
+        return kSaved;
+      }
+    }
+  }
+  return nf;
+}
+
+template <int FB>
+__device__ __forceinline__ void write_faces(const WaveHull<FB>& s, int nf, int32_t* out, int lane) {
+  for (int f = lane; f < nf; f += kWave) {
+    out[3 * f] = (int32_t)(s.co[f].ab & 0xffffu);
+    out[3 * f + 1] = (int32_t)(s.co[f].ab >> 16);
+    out[3 * f + 2] = (int32_t)s.co[f].c;
+  }
+}
+
+// ------------------------------------------------------ over global memory
 //
-// The largest class keeps vertex ids alone (4 bytes a face, the normal formed
-// anew from the three corners), for the room: on dense, nearly coplanar
-// surfaces the face list grows tenfold within the last insertions, and such a
-// cloud of 8-512 points took 10 ms and more in the general kernel.
+// Any size, one wave over the output buffer and the workspace (F: 3 * cap
+// entries, vis: cap, hor: 2 * cap), from the start or from a saved state.
+
+__device__ __forceinline__ float vol6(const float* __restrict__ p, int a, int b, int c,
+                                      float qx, float qy, float qz) {
+  const float ax = p[3 * a], ay = p[3 * a + 1], az = p[3 * a + 2];
+  const float bx = p[3 * b] - ax, by = p[3 * b + 1] - ay, bz = p[3 * b + 2] - az;
+  const float cx = p[3 * c] - ax, cy = p[3 * c + 1] - ay, cz = p[3 * c + 2] - az;
+  const float dx = qx - ax, dy = qy - ay, dz = qz - az;
+  const float nx = by * cz - bz * cy, ny = bz * cx - bx * cz, nz = bx * cy - by * cx;
+  return nx * dx + ny * dy + nz * dz;
+}
+
+// Orders the global memory accesses of the lanes of one wave.
+__device__ __forceinline__ void memory_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+}
+
+__device__ __forceinline__ int hull_global(const float* __restrict__ P, int n, int cap, int32_t* F, int32_t* vis,
+                           int32_t* hor, bool resume, int lane) {
+  int id[4] = {0, 0, 0, 0};
+  int nf = 4, q = 0;
+  memory_sync();
+  if (resume) {
+    load_state(vis, nf, q, id);  // it lies where the visible faces are listed
+  } else {
+    const int st = hull_begin(P, n, cap, lane, id);
+    if (st != 4) return st;
+    if (lane < 4) {
+#pragma unroll
+      for (int j = 0; j < 3; j++) F[3 * lane + j] = init_corner(id, lane, j);
+    }
+  }
+  memory_sync();
+  for (; q < n; q++) {
+    if (q == id[0] || q == id[1] || q == id[2] || q == id[3]) continue;
+    const float qx = P[3 * q], qy = P[3 * q + 1], qz = P[3 * q + 2];
+    // visible faces, listed in ascending order
+    int nv = 0;
+    for (int base = 0; base < nf; base += kWave) {
+      const int f = base + lane;
+      bool v = false;
+      if (f < nf) v = vol6(P, F[3 * f], F[3 * f + 1], F[3 * f + 2], qx, qy, qz) > 1e-7f;
+      const uint64_t b = ballot(v);
+      if (v) vis[nv + rank_below(b, lane)] = f;
+      nv += __popcll(b);
+    }
+    if (nv == 0) continue;
+    memory_sync();
+    // horizon: directed edges of visible faces whose reverse no visible face
+    // has, in (visible face, edge) order
+    int nh = 0;
+    const int ne = 3 * nv;
+    for (int base = 0; base < ne; base += kWave) {
+      const int h = base + lane;
+      bool hz = false;
+      int a = 0, b = 0;
+      if (h < ne) {
+        const int k = h / 3, e = h - 3 * k;
+        const int g = vis[k];
+        a = F[3 * g + e];
+        b = F[3 * g + (e == 2 ? 0 : e + 1)];
+        bool found = false;
+        for (int k2 = 0; k2 < nv && !found; k2++) {
+          const int g2 = vis[k2];
+          const int x0 = F[3 * g2], x1 = F[3 * g2 + 1], x2 = F[3 * g2 + 2];
+          found = (x0 == b && x1 == a) || (x1 == b && x2 == a) || (x2 == b && x0 == a);
+        }
+        hz = !found;
+      }
+      const uint64_t bl = ballot(hz);
+      const int r = nh + rank_below(bl, lane);
+      if (hz && r < cap) {
+        hor[2 * r] = a;
+        hor[2 * r + 1] = b;
+      }
+      nh += __popcll(bl);
+    }
+    memory_sync();
+    // drop the visible faces, keeping the order of the others
+    int w = 0;
+    for (int base = 0; base < nf; base += kWave) {
+      const int f = base + lane;
+      bool alive = false;
+      int x0 = 0, x1 = 0, x2 = 0;
+      if (f < nf) {
+        x0 = F[3 * f];
+        x1 = F[3 * f + 1];
+        x2 = F[3 * f + 2];
+        alive = !(vol6(P, x0, x1, x2, qx, qy, qz) > 1e-7f);
+      }
+      const uint64_t b = ballot(alive);
+      if (alive) {
+        const int d = w + rank_below(b, lane);
+        F[3 * d] = x0;
+        F[3 * d + 1] = x1;
+        F[3 * d + 2] = x2;
+      }
+      w += __popcll(b);
+      memory_sync();
+    }
+    if (nh > cap || w + nh > cap) {
+      return -1;
+    }
+    for (int r = lane; r < nh; r += kWave) {
+      F[3 * (w + r)] = hor[2 * r];
+      F[3 * (w + r) + 1] = hor[2 * r + 1];
+      F[3 * (w + r) + 2] = q;
+    }
+    nf = w + nh;
+    memory_sync();
+  }
+  return nf;
+}
+
+// RESUME: the clouds whose state was saved, else those of more than kFewPoints
+// points and those of fewer that outgrew their lanes, from the start.  The waves
+// of the grid take the clouds in turn.  Two steps, for the room: with the larger
+// one at once a compute unit has 3 waves, with the smaller one 22.
+constexpr int kWaveFaces = 160, kWaveMoreFaces = 1200;
+
+template <int FB, bool RESUME>
+__global__ __launch_bounds__(kWave) void k_hull_wave(HullArgs h) {
+  __shared__ WaveHull<FB> s;
+  const int lane = threadIdx.x;
+  for (int64_t first = blockIdx.x; first < h.nm; first += (int64_t)gridDim.x * kWave) {
+    const int64_t mine = first + (int64_t)gridDim.x * lane;
+    int n_mine = 0;
+    bool take = false;
+    if (mine < h.nm) {
+      n_mine = h.cnt[mine];
+      take = RESUME ? h.nfaces[mine] == kSaved
+                    : n_mine > kFewPoints || h.nfaces[mine] == kToWave;
+    }
+    uint64_t todo = ballot(take);
+    while (todo != 0) {
+      const int src = (int)__builtin_ctzll(todo);
+      todo &= todo - 1;
+      const int64_t m = first + (int64_t)gridDim.x * src;
+      const int n = ogjk::lane_value(n_mine, src);
+      int nf = -3;
+      if (RESUME || (h.range_ok(m) && n <= kWavePoints)) {
+        nf = hull_wave(h.points(m), n, h.cap(m), s, h.out(m), h.work(m), RESUME, lane);
+        write_faces(s, nf, h.out(m), lane);
+      } else if (h.range_ok(m)) {
+        nf = hull_global(h.points(m), n, h.cap(m), h.out(m), h.work(m), h.work(m) + h.cap64(m),
+                         false, lane);
+      }
+      if (lane == 0) h.nfaces[m] = nf;
+    }
+  }
+}
+
+// ------------------------------------------------------ a block per cloud
 //
-// Directed edges of the visible faces: a bit per (start, end) for at most
-// 512 points, else a hash set.
-template <int NP>
+// For clouds of up to kBlockPoints points whose face list outgrows a wave's: the
+// whole block tests the faces and notes the visible ones, then the first wave
+// alone does the ordered part (horizon, new faces).  Two barriers per insertion,
+// but a lone wave takes some 70 instructions for every 64 faces.  A face that
+// leaves stays behind as a dead slot, so nothing moves: slots are in creation
+// order, which is the order the reference's compaction keeps, and the first
+// wave closes the gaps now and then.  Each wave tests one contiguous run of
+// slots, so the waves' lists of visible faces joined together are in slot order.
+// On dense, nearly coplanar surfaces the face list grows tenfold and more within
+// the last insertions (a cloud of 8-512 points took 10 ms and more over global
+// memory): when the faces with their planes outgrow the LDS, they are kept as
+// vertex ids alone (4 bytes a face, the normal formed anew from the corners).
+// A call over few clouds is one launch of this kernel: each block's first wave
+// starts its cloud, and the block goes on from kAloneFaces faces, where a wave's
+// insertion takes as long (512 points: 0.82 ms, 1.16 with the wave to the end,
+// 1.0 with the block from 64 faces).
+constexpr int kBlockThreads = 512, kBlockWaves = kBlockThreads / kWave, kBlockPoints = 1024;
+constexpr int kAloneFaces = 512;
+constexpr int kBlocksAtOnce = 256;  // compute units, one block each
+
+// Directed edges of the visible faces, in the same room: a bit per (start, end)
+// for at most kBitPoints points, else a hash set.  (One type that looks at the
+// point count cost the former 0.8 us an insertion.)
+constexpr int kBitPoints = 512, kEdgeWords = 8192;
+
 struct EdgeBits {
-  static constexpr int W = (NP + 31) / 32;
-  uint32_t bits[NP * W];
-  __device__ __forceinline__ void clear_all(int t, int threads) {
-    for (int i = t; i < NP * W; i += threads) bits[i] = 0u;
+  static constexpr uint32_t kClear = 0u;
+  uint32_t word[kEdgeWords];
+  __device__ __forceinline__ static uint32_t place(uint32_t a, uint32_t b) {
+    return a * (kBitPoints / 32) + (b >> 5);
   }
   __device__ __forceinline__ bool insert(uint32_t a, uint32_t b) {
-    atomicOr(&bits[a * W + (b >> 5)], 1u << (b & 31u));
+    atomicOr(&word[place(a, b)], 1u << (b & 31u));
     return true;
   }
   __device__ __forceinline__ bool found(uint32_t a, uint32_t b) const {
-    return (bits[a * W + (b >> 5)] >> (b & 31u)) & 1u;
+    return (word[place(a, b)] >> (b & 31u)) & 1u;
   }
-  __device__ __forceinline__ void erase(uint32_t a, uint32_t b) { bits[a * W + (b >> 5)] = 0u; }
-  __device__ __forceinline__ void end_step(int) {}
+  // after the last look-up of a step
+  __device__ __forceinline__ void erase(uint32_t a, uint32_t b) { word[place(a, b)] = kClear; }
 };
 
 struct EdgeHash {
-  static constexpr uint32_t kSize = 8192, kNone = 0xffffffffu;
+  static constexpr uint32_t kClear = 0xffffffffu;
   static constexpr int kProbes = 32;  // an edge lies within this many places of its own, or nowhere
-  alignas(16) uint32_t key[kSize];
-  __device__ __forceinline__ static uint32_t place(uint32_t k) {
-    return (k * 0x9e3779b1u) >> 19;
-  }
-  __device__ __forceinline__ void clear_all(int t, int threads) {
-    for (int i = t; i < (int)kSize; i += threads) key[i] = kNone;
+  uint32_t word[kEdgeWords];
+  __device__ __forceinline__ static uint32_t place(uint32_t k, int p) {
+    return ((k * 0x9e3779b1u >> 19) + p) & (kEdgeWords - 1);
   }
   __device__ __forceinline__ bool insert(uint32_t a, uint32_t b) {
-    const uint32_t k = a << 10 | b, h = place(k);
+    const uint32_t k = a << 10 | b;
     for (int p = 0; p < kProbes; p++) {
-      const uint32_t was = atomicCAS(&key[(h + p) & (kSize - 1u)], kNone, k);
-      if (was == kNone || was == k) return true;
+      const uint32_t was = atomicCAS(&word[place(k, p)], kClear, k);
+      if (was == kClear || was == k) return true;
     }
     return false;
   }
   __device__ __forceinline__ bool found(uint32_t a, uint32_t b) const {
-    const uint32_t k = a << 10 | b, h = place(k);
+    const uint32_t k = a << 10 | b;
     for (int p = 0; p < kProbes; p++) {
-      const uint32_t x = key[(h + p) & (kSize - 1u)];
+      const uint32_t x = word[place(k, p)];
       if (x == k) return true;
-      if (x == kNone) return false;
+      if (x == kClear) return false;
     }
     return false;
   }
-  __device__ __forceinline__ void erase(uint32_t, uint32_t) {}
-  __device__ __forceinline__ void end_step(int lane) {
-    for (int i = lane; i < (int)kSize / 4; i += kWave)
-      ((uint4*)key)[i] = uint4{kNone, kNone, kNone, kNone};
+  // Places of other edges may be clear already, so a clear one does not end
+  // the search.
+  __device__ __forceinline__ void erase(uint32_t a, uint32_t b) {
+    const uint32_t k = a << 10 | b;
+    for (int p = 0; p < kProbes; p++) {
+      if (word[place(k, p)] == k) {
+        word[place(k, p)] = kClear;
+        return;
+      }
+    }
   }
 };
 
-template <int T, int S, int NP>
+template <bool PLANES, class Edges>
 struct BlockHull {
-  static constexpr int kWaves = T / kWave;
-  static constexpr bool kPlanes = NP <= 512;
-  using Face = std::conditional_t<kPlanes, Tri, uint32_t>;
-  static constexpr int kSeg = kPlanes ? 128 : 256;  // visible faces a wave lists at an insertion
-  static constexpr int kRoom = kPlanes ? 384 : 2048;  // slots an insertion finds free
-  static constexpr int kRow = kWave / kWaves;  // of which the first wave takes these in one go
-  Face face[S];                     // ids: 3 x 10 bits, kDead, kLate
-  float4 pt[NP];
-  std::conditional_t<NP <= 512, EdgeBits<NP>, EdgeHash> edges;
-  uint32_t seg[kWaves][kSeg];  // vertex ids of the visible faces each wave found
-  int cnt[2][kWaves];          // how many, by the parity of the step
-  int tail, status;            // read by every thread after an insertion
-  int full;                    // an edge found no place
-  int id[4];
+  using Face = std::conditional_t<PLANES, Tri, uint32_t>;
+  static constexpr int kFaces = 65536 / sizeof(Face);
+  static constexpr int kRoom = kFaces / 8;  // slots an insertion finds free
+  static constexpr int kSeg = 256;          // visible faces a wave lists at an insertion
+  static constexpr int kRow = kWave / kBlockWaves;  // of which the first wave takes these in one go
+  Face face[kFaces];  // ids: 3 x 10 bits, kDead, kLate
+  float4 pt[kBlockPoints];
+  Edges edges;
+  uint32_t seg[kBlockWaves][kSeg];  // vertex ids of the visible faces each wave found
+  int cnt[2][kBlockWaves];          // how many, by the parity of the step
+  int tail, status;                 // read by every thread after an insertion
+  int full;                         // an edge found no place
 };
-// Flags beside a slot's 3 x 10 bits of ids: the face has left, and it left at the
-// insertion at hand and is on no wave's list.
+// Flags beside a slot's ids: the face has left, and it left at the insertion at
+// hand and is on no wave's list.
 constexpr uint32_t kDead = 0x80000000u, kLate = 0x40000000u;
 
 __device__ __forceinline__ uint32_t& ids_of(Tri& f) { return f.ids; }
@@ -485,84 +879,66 @@ __device__ __forceinline__ uint32_t& ids_of(uint32_t& f) { return f; }
 // Live slots of [0, tail) moved down in order, by one wave.  Returns their count.
 template <class Face>
 __device__ __forceinline__ int close_gaps(Face* face, int tail, int lane) {
+  // as plain words: copies of the struct end in the stack frame
+  using Words = std::conditional_t<sizeof(Face) == sizeof(uint4), uint4, uint32_t>;
   int w = 0;
   for (int base = 0; base < tail; base += kWave) {
     const int f = base + lane;
-    Face F{};
-    if (f < tail) F = face[f];
-    const bool live = f < tail && !(ids_of(F) & kDead);
+    Words F;
+    __builtin_memcpy(&F, &face[min(f, tail - 1)], sizeof(F));
+    const bool live = f < tail && !(ids_of(face[min(f, tail - 1)]) & kDead);
     const uint64_t b = ballot(live);
     wave_sync();
-    if (live) face[w + rank_below(b, lane)] = F;
+    if (live) __builtin_memcpy(&face[w + rank_below(b, lane)], &F, sizeof(F));
     wave_sync();
     w += __popcll(b);
   }
   return w;
 }
 
-// Whole block.  Returns the face count (faces in s.face[0..)), a status of
-// d_nfaces, or kToBig when the working set is too small.
-template <int T, int S, int NP>
-__device__ int hull_block(const float* __restrict__ P, int n, int cap, BlockHull<T, S, NP>& s) {
-  using B = BlockHull<T, S, NP>;
-  static_assert(NP <= 1024, "vertex ids are packed in 10 bits");
+__device__ __forceinline__ void write_ids(int32_t* out, uint32_t ids) {
+  out[0] = (int32_t)(ids & 1023u);
+  out[1] = (int32_t)((ids >> 10) & 1023u);
+  out[2] = (int32_t)(ids >> 20);
+}
+
+// Whole block, from a saved state.  Returns the face count (faces in
+// s.face[0..)), a status of d_nfaces, or kSaved when the slots or the edge set
+// are too few: the state is then the one of the last insertion that left room
+// for another, or the one it started from.
+template <bool PLANES, class Edges>
+__device__ __forceinline__ int hull_block(const float* __restrict__ P, int n, int cap, BlockHull<PLANES, Edges>& s,
+                          int32_t* out, int32_t* save) {
+  using B = BlockHull<PLANES, Edges>;
+  constexpr int T = kBlockThreads, S = B::kFaces;
+  static_assert(kBlockPoints <= 1024, "vertex ids are packed in 10 bits");
   const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
-  const auto pt = [&](int i) { return s.pt[i]; };
   const auto put = [&](int f, float4 a, float4 b, float4 c, uint32_t ids) {
-    if constexpr (B::kPlanes) s.face[f] = make_tri(a, b, c, ids);
+    if constexpr (PLANES) s.face[f] = make_tri(a, b, c, ids);
     else s.face[f] = ids;
   };
-  __syncthreads();  // the block's previous cloud has been written out
-  s.edges.clear_all(t, T);
+  __syncthreads();  // the block's LDS is free
+  int tail, q0, id[4];
+  load_state(save, tail, q0, id);
+  if (tail > S - B::kRoom) return kSaved;
+  int alive = tail;  // the first wave's
+  for (int i = t; i < kEdgeWords; i += T) s.edges.word[i] = Edges::kClear;
   for (int i = t; i < n; i += T) s.pt[i] = make_float4(P[3 * i], P[3 * i + 1], P[3 * i + 2], 0.0f);
-  __syncthreads();
-  if (wave == 0) {
-    float lo[3], hi[3];
-    int lo_i[3], hi_i[3];
-    bool bad = false;
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-      lo[k] = INFINITY;
-      hi[k] = -INFINITY;
-      lo_i[k] = hi_i[k] = -1;
-    }
-    for (int i = lane; i < n; i += kWave) {
-      const float4 p4 = s.pt[i];
-      const float p[3] = {p4.x, p4.y, p4.z};
-#pragma unroll
-      for (int k = 0; k < 3; k++) {
-        bad |= !isfinite(p[k]);
-        if (lo_i[k] < 0 || p[k] < lo[k]) { lo[k] = p[k]; lo_i[k] = i; }
-        if (hi_i[k] < 0 || p[k] > hi[k]) { hi[k] = p[k]; hi_i[k] = i; }
-      }
-    }
-    int id[4] = {0, 0, 0, 0};
-    int st = 4;
-    if (ballot(bad)) st = -2;
-    else if (!first_tetrahedron<kWave>(pt, n, lane, lo, lo_i, hi, hi_i, id)) st = 0;
-    else if (cap < 4) st = -1;
-    if (st == 4 && lane < 4) {
-      const int a = init_corner(id, lane, 0), b = init_corner(id, lane, 1),
-                c = init_corner(id, lane, 2);
-      put(lane, s.pt[a], s.pt[b], s.pt[c], (uint32_t)(a | b << 10 | c << 20));
-    }
-    if (lane == 0) {
-#pragma unroll
-      for (int k = 0; k < 4; k++) s.id[k] = id[k];
-      s.tail = 4;
-      s.full = 0;
-      s.status = st;
-    }
+  if (t == 0) {
+    s.full = 0;
+    s.status = 4;
   }
   __syncthreads();
-  if (s.status != 4) return s.status;
-  const int f0 = s.id[0], f1 = s.id[1], f2 = s.id[2], f3 = s.id[3];
-  int tail = 4, alive = 4;  // alive: the first wave's
-  float4 next = s.pt[0];
-  for (int q = 0, step = 0; q < n; q++) {
+  for (int f = t; f < tail; f += T) {
+    const uint32_t a = out[3 * f], b = out[3 * f + 1], c = out[3 * f + 2];
+    put(f, s.pt[a], s.pt[b], s.pt[c], a | b << 10 | c << 20);
+  }
+  __syncthreads();
+  float4 next = s.pt[min(q0, n - 1)];
+  for (int q = q0, step = 0; q < n; q++) {
     const float4 Q = next;
     next = s.pt[q + 1 < n ? q + 1 : q];
-    if (q == f0 || q == f1 || q == f2 || q == f3) continue;
+    if (q == id[0] || q == id[1] || q == id[2] || q == id[3]) continue;
     const int run = (tail + T - 1) / T * kWave;
     const int end = min(tail, (wave + 1) * run);
     int found = 0;
@@ -572,17 +948,15 @@ __device__ int hull_block(const float* __restrict__ P, int n, int cap, BlockHull
       bool v[U];
 #pragma unroll
       for (int u = 0; u < U; u++) {
-        const int f = base + u * kWave + lane;
-        F[u] = typename B::Face{};
-        ids_of(F[u]) = kDead;
-        if (f < end) F[u] = s.face[f];
+        F[u] = s.face[min(base + u * kWave + lane, end - 1)];
+        if (base + u * kWave + lane >= end) ids_of(F[u]) = kDead;
       }
 #pragma unroll
       for (int u = 0; u < U; u++) {
         const uint32_t ids = ids_of(F[u]);
         const float4 a = s.pt[ids & 1023u];
         float d;
-        if constexpr (B::kPlanes) d = vol6(F[u], a, Q);
+        if constexpr (PLANES) d = vol6(F[u], a, Q);
         else d = vol6(a, s.pt[(ids >> 10) & 1023u], s.pt[(ids >> 20) & 1023u], Q);
         v[u] = !(ids & kDead) && d > 1e-7f;
       }
@@ -596,7 +970,8 @@ __device__ int hull_block(const float* __restrict__ P, int n, int cap, BlockHull
           const int r = found + rank_below(bv, lane);
           ids_of(s.face[f]) = ids | (r < B::kSeg ? kDead : kDead | kLate);
           if (r < B::kSeg) s.seg[wave][r] = ids;
-          const bool i0 = s.edges.insert(x, y), i1 = s.edges.insert(y, z), i2 = s.edges.insert(z, x);
+          const bool i0 = s.edges.insert(x, y), i1 = s.edges.insert(y, z),
+                     i2 = s.edges.insert(z, x);
           if (!i0 || !i1 || !i2) s.full = 1;
         }
         found += __popcll(bv);
@@ -611,7 +986,7 @@ __device__ int hull_block(const float* __restrict__ P, int n, int cap, BlockHull
     if (wave == 0) {
       int status = 4, nh = 0, nv = 0, at = tail;
       if (s.full) {
-        status = kToBig;
+        status = kSaved;
       } else {
         // Each lane takes a visible face (valid: ids), in slot order: its
         // edges whose reverse no visible face has are bases of new faces, in
@@ -660,7 +1035,7 @@ __device__ int hull_block(const float* __restrict__ P, int n, int cap, BlockHull
           // ones in a few waves' runs.  Those past a list's end are found again
           // by their flag, in the slots of the wave's run, behind the listed ones.
           const auto each = [&](const auto& f) {
-            for (int w = 0; w < B::kWaves; w++) {
+            for (int w = 0; w < kBlockWaves; w++) {
               const int c = cnt[w], listed = min(c, B::kSeg);
               for (int base = 0; base < listed; base += kWave)
                 f(base + lane < listed, base + lane < listed ? s.seg[w][base + lane] : 0u, -1);
@@ -683,15 +1058,15 @@ __device__ int hull_block(const float* __restrict__ P, int n, int cap, BlockHull
             if (valid && slot >= 0) ids_of(s.face[slot]) = ids | kDead;
           });
         } else {
-          int pre[B::kWaves + 1];  // visible faces of the waves before
+          int pre[kBlockWaves + 1];  // visible faces of the waves before
           pre[0] = 0;
 #pragma unroll
-          for (int w = 0; w < B::kWaves; w++) pre[w + 1] = pre[w] + cnt[w];
-          nv = pre[B::kWaves];
+          for (int w = 0; w < kBlockWaves; w++) pre[w + 1] = pre[w] + cnt[w];
+          nv = pre[kBlockWaves];
           const auto visible = [&](int j) {
             int w = 0, st = 0;
 #pragma unroll
-            for (int k = 1; k < B::kWaves; k++) {
+            for (int k = 1; k < kBlockWaves; k++) {
               w = j >= pre[k] ? k : w;
               st = j >= pre[k] ? pre[k] : st;
             }
@@ -703,16 +1078,20 @@ __device__ int hull_block(const float* __restrict__ P, int n, int cap, BlockHull
           }
           for (int j = lane; j < nv; j += kWave) unmark(visible(j));
         }
-        s.edges.end_step(lane);
         alive += nh - nv;
         at += nh;
         if (alive > cap) {
           status = -1;
         } else if (at > S) {
-          status = kToBig;
-        } else if (at > S - B::kRoom || at > 2 * alive + T) {
+          status = kSaved;
+        } else if (at > S - B::kRoom || at > alive + alive / 8 + 256) {
           wave_sync();
           at = close_gaps(s.face, at, lane);
+          if (at > S - B::kRoom) {
+            for (int f = lane; f < at; f += kWave) write_ids(out + 3 * f, ids_of(s.face[f]));
+            if (lane == 0) store_state(save, at, q + 1, id);
+            status = kSaved;
+          }
         }
       }
       if (lane == 0) {
@@ -721,8 +1100,9 @@ __device__ int hull_block(const float* __restrict__ P, int n, int cap, BlockHull
       }
     }
     __syncthreads();
-    if (s.status != 4) return s.status;
-    tail = s.tail;
+    const int status = __builtin_amdgcn_readfirstlane(s.status);
+    if (status != 4) return status;
+    tail = __builtin_amdgcn_readfirstlane(s.tail);
   }
   __syncthreads();
   if (wave == 0) {
@@ -730,302 +1110,83 @@ __device__ int hull_block(const float* __restrict__ P, int n, int cap, BlockHull
     if (lane == 0) s.tail = nf;
   }
   __syncthreads();
-  return s.tail;
+  return __builtin_amdgcn_readfirstlane(s.tail);
 }
 
-// Clouds of NMIN..NP points and those an earlier kernel passed on as FROM; the
-// blocks of the grid take the clouds in turn.  PASS: how this kernel passes on.
-template <int T, int S, int NMIN, int NP, int FROM, int PASS>
-__global__ __launch_bounds__(T) void k_hull_block(const float* __restrict__ pts,
-                                                  const int64_t* __restrict__ off,
-                                                  const int32_t* __restrict__ cnt, int nm,
-                                                  const int64_t* __restrict__ face_off,
-                                                  int64_t total_faces,
-                                                  int32_t* __restrict__ faces,
-                                                  int32_t* __restrict__ nfaces) {
-  __shared__ BlockHull<T, S, NP> s;
+// One cloud from its saved state; the block writes the faces out.
+template <bool PLANES, class Edges>
+__device__ __forceinline__ int hull_block_out(const HullArgs& h, int64_t m, int n,
+                                              BlockHull<PLANES, Edges>& s) {
+  const int nf = hull_block(h.points(m), n, h.cap(m), s, h.out(m), h.work(m));
+  int32_t* out = h.out(m);
+  for (int f = threadIdx.x; f < nf; f += kBlockThreads) write_ids(out + 3 * f, ids_of(s.face[f]));
+  return nf;
+}
+
+// ALL: every cloud of the call, from the start, else those whose state was
+// saved.  The blocks of the grid take the clouds in turn; a block's clouds that
+// it has no room for are spread over its waves at the end, over global memory.
+template <bool ALL>
+__global__ __launch_bounds__(kBlockThreads) void k_hull_block(HullArgs h) {
+  __shared__ union Lds {
+    WaveHull<kAloneFaces> w;
+    BlockHull<true, EdgeBits> p;
+    BlockHull<false, EdgeBits> b;
+    BlockHull<true, EdgeHash> ph;
+    BlockHull<false, EdgeHash> bh;
+  } s;
+  __shared__ int result;
   const int lane = threadIdx.x & (kWave - 1);
-  for (int64_t first = blockIdx.x; first < nm; first += (int64_t)gridDim.x * kWave) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  for (int64_t first = blockIdx.x; first < h.nm; first += (int64_t)gridDim.x * kWave) {
     const int64_t mine = first + (int64_t)gridDim.x * lane;
-    int n_mine = -1;
-    bool take = false;
-    if (mine < nm) {
-      n_mine = cnt[mine];
-      take = n_mine >= NMIN ? n_mine <= NP : nfaces[mine] == FROM;
-    }
-    uint64_t todo = ballot(take);  // the same in every wave of the block
+    const int n_mine = mine < h.nm ? h.cnt[mine] : 0;
+    uint64_t todo = ballot(mine < h.nm && (ALL || h.nfaces[mine] == kSaved));
+    uint64_t large = 0;  // the same in every wave, as todo is
+    __syncthreads();     // every wave has read the counts that this block writes
     while (todo != 0) {
       const int src = (int)__builtin_ctzll(todo);
       todo &= todo - 1;
       const int64_t m = first + (int64_t)gridDim.x * src;
-      const int n = __shfl(n_mine, src, kWave);
-      const int64_t f0 = face_off[m], cap64 = face_off[m + 1] - f0;
-      int nf;
-      if (f0 < 0 || cap64 < 0 || face_off[m + 1] > total_faces) {
-        nf = -3;
-      } else {
-        nf = hull_block(pts + 3 * off[m], n, cap64 < 0x7fffffff ? (int)cap64 : 0x7fffffff, s);
-        if (nf == kToBig) nf = PASS;
-      }
-      int32_t* out = faces + 3 * f0;
-      for (int f = threadIdx.x; f < nf; f += T) {
-        const uint32_t ids = ids_of(s.face[f]);
-        out[3 * f] = (int32_t)(ids & 1023u);
-        out[3 * f + 1] = (int32_t)((ids >> 10) & 1023u);
-        out[3 * f + 2] = (int32_t)(ids >> 20);
-      }
-      // every wave has read its clouds' nfaces before this write only for the
-      // chunk at hand; a result is never FROM, so a later read cannot take it
-      if (threadIdx.x == 0) nfaces[m] = nf;
-    }
-  }
-}
-
-// ------------------------------------------------------ any other cloud
-//
-// More than 1,024 points, or a working set past the block's LDS: one wave per
-// cloud over the output buffer and the workspace.
-
-__device__ __forceinline__ float vol6(const float* __restrict__ p, int a, int b, int c,
-                                      float qx, float qy, float qz) {
-  const float ax = p[3 * a], ay = p[3 * a + 1], az = p[3 * a + 2];
-  const float bx = p[3 * b] - ax, by = p[3 * b + 1] - ay, bz = p[3 * b + 2] - az;
-  const float cx = p[3 * c] - ax, cy = p[3 * c + 1] - ay, cz = p[3 * c + 2] - az;
-  const float dx = qx - ax, dy = qy - ay, dz = qz - az;
-  const float nx = by * cz - bz * cy, ny = bz * cx - bx * cz, nz = bx * cy - by * cx;
-  return nx * dx + ny * dy + nz * dz;
-}
-
-// Wave argmax over (value, index): larger value, then lower index.  Lanes
-// with index < 0 hold nothing.
-__device__ __forceinline__ void wave_argmax(float& v, int& i) {
-#pragma unroll
-  for (int m = 1; m < kWave; m <<= 1) {
-    const float ov = __shfl_xor(v, m);
-    const int oi = __shfl_xor(i, m);
-    const bool take = oi >= 0 && (i < 0 || ov > v || (ov == v && oi < i));
-    v = take ? ov : v;
-    i = take ? oi : i;
-  }
-}
-
-__device__ __forceinline__ void wave_argmin(float& v, int& i) {
-#pragma unroll
-  for (int m = 1; m < kWave; m <<= 1) {
-    const float ov = __shfl_xor(v, m);
-    const int oi = __shfl_xor(i, m);
-    const bool take = oi >= 0 && (i < 0 || ov < v || (ov == v && oi < i));
-    v = take ? ov : v;
-    i = take ? oi : i;
-  }
-}
-
-// F: 3 * cap entries, vis: cap, hor: 2 * cap.
-__device__ int hull_global(const float* __restrict__ P, int n, int cap, int32_t* F, int32_t* vis,
-                           int32_t* hor, int lane) {
-  // axis extremes (first index on ties), rejecting non-finite input
-  float mnv[3], mxv[3];
-  int mni[3], mxi[3];
-  bool bad = false;
-#pragma unroll
-  for (int k = 0; k < 3; k++) {
-    mnv[k] = INFINITY;
-    mxv[k] = -INFINITY;
-    mni[k] = mxi[k] = -1;
-  }
-  for (int i = lane; i < n; i += kWave) {
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-      const float v = P[3 * i + k];
-      bad |= !isfinite(v);
-      if (mni[k] < 0 || v < mnv[k]) { mnv[k] = v; mni[k] = i; }
-      if (mxi[k] < 0 || v > mxv[k]) { mxv[k] = v; mxi[k] = i; }
-    }
-  }
-  if (ballot(bad)) {
-    return -2;
-  }
-#pragma unroll
-  for (int k = 0; k < 3; k++) {
-    wave_argmin(mnv[k], mni[k]);
-    wave_argmax(mxv[k], mxi[k]);
-  }
-  // most separated pair among the six
-  int i0 = 0, i1 = 1;
-  {
-    const int c[6] = {mni[0], mxi[0], mni[1], mxi[1], mni[2], mxi[2]};
-    float bd = 0;
-    for (int a = 0; a < 6; a++)
-      for (int b = a + 1; b < 6; b++) {
-        const float dx = P[3 * c[b]] - P[3 * c[a]], dy = P[3 * c[b] + 1] - P[3 * c[a] + 1],
-                    dz = P[3 * c[b] + 2] - P[3 * c[a] + 2];
-        const float d = dx * dx + dy * dy + dz * dz;
-        if (d > bd) {
-          bd = d;
-          i0 = c[a];
-          i1 = c[b];
+      const int n = ogjk::lane_value(n_mine, src);
+      int nf = kSaved;
+      if (ALL) {
+        __syncthreads();  // the block's LDS is free
+        if (wave == 0) {
+          int r = kSaved;
+          if (!h.range_ok(m)) {
+            r = -3;
+          } else if (n < 4) {
+            r = 0;
+          } else if (n <= kWavePoints) {
+            r = hull_wave(h.points(m), n, h.cap(m), s.w, h.out(m), h.work(m), false, lane);
+            write_faces(s.w, r, h.out(m), lane);
+          }
+          if (lane == 0) result = r;
         }
+        __syncthreads();
+        nf = __builtin_amdgcn_readfirstlane(result);
       }
-  }
-  // farthest from the line i0-i1
-  int i2;
-  {
-    const float e0 = P[3 * i1] - P[3 * i0], e1 = P[3 * i1 + 1] - P[3 * i0 + 1],
-                e2 = P[3 * i1 + 2] - P[3 * i0 + 2];
-    float bv = 0;
-    int bi = -1;
-    for (int i = lane; i < n; i += kWave) {
-      if (i == i0 || i == i1) continue;
-      const float vx = P[3 * i] - P[3 * i0], vy = P[3 * i + 1] - P[3 * i0 + 1],
-                  vz = P[3 * i + 2] - P[3 * i0 + 2];
-      const float cx = vy * e2 - vz * e1, cy = vz * e0 - vx * e2, cz = vx * e1 - vy * e0;
-      const float d = cx * cx + cy * cy + cz * cz;
-      if (d > bv) { bv = d; bi = i; }
-    }
-    wave_argmax(bv, bi);
-    i2 = bi;
-  }
-  if (i2 < 0) {
-    return 0;
-  }
-  // farthest from the plane i0-i1-i2
-  int i3;
-  {
-    float bv = 0;
-    int bi = -1;
-    for (int i = lane; i < n; i += kWave) {
-      if (i == i0 || i == i1 || i == i2) continue;
-      float d = vol6(P, i0, i1, i2, P[3 * i], P[3 * i + 1], P[3 * i + 2]);
-      if (d < 0) d = -d;
-      if (d > bv) { bv = d; bi = i; }
-    }
-    wave_argmax(bv, bi);
-    i3 = bi;
-  }
-  if (i3 < 0) {
-    return 0;
-  }
-  if (vol6(P, i0, i1, i2, P[3 * i3], P[3 * i3 + 1], P[3 * i3 + 2]) > 0) {
-    const int t = i1;
-    i1 = i2;
-    i2 = t;
-  }
-  if (cap < 4) {
-    return -1;
-  }
-  if (lane < 12) {
-    const int init[12] = {i0, i1, i2, i0, i2, i3, i0, i3, i1, i1, i3, i2};
-    F[lane] = init[lane];
-  }
-  __syncthreads();
-  int nf = 4;
-  for (int q = 0; q < n; q++) {
-    if (q == i0 || q == i1 || q == i2 || q == i3) continue;
-    const float qx = P[3 * q], qy = P[3 * q + 1], qz = P[3 * q + 2];
-    // visible faces, listed in ascending order
-    int nv = 0;
-    for (int base = 0; base < nf; base += kWave) {
-      const int f = base + lane;
-      bool v = false;
-      if (f < nf) v = vol6(P, F[3 * f], F[3 * f + 1], F[3 * f + 2], qx, qy, qz) > 1e-7f;
-      const uint64_t b = ballot(v);
-      if (v) vis[nv + rank_below(b, lane)] = f;
-      nv += __popcll(b);
-    }
-    if (nv == 0) continue;
-    __syncthreads();
-    // horizon: directed edges of visible faces whose reverse no visible face
-    // has, in (visible face, edge) order
-    int nh = 0;
-    const int ne = 3 * nv;
-    for (int base = 0; base < ne; base += kWave) {
-      const int h = base + lane;
-      bool hz = false;
-      int a = 0, b = 0;
-      if (h < ne) {
-        const int k = h / 3, e = h - 3 * k;
-        const int g = vis[k];
-        a = F[3 * g + e];
-        b = F[3 * g + (e == 2 ? 0 : e + 1)];
-        bool found = false;
-        for (int k2 = 0; k2 < nv && !found; k2++) {
-          const int g2 = vis[k2];
-          const int x0 = F[3 * g2], x1 = F[3 * g2 + 1], x2 = F[3 * g2 + 2];
-          found = (x0 == b && x1 == a) || (x1 == b && x2 == a) || (x2 == b && x0 == a);
-        }
-        hz = !found;
+      if (nf == kSaved && n <= kBitPoints) {
+        nf = hull_block_out(h, m, n, s.p);
+        if (nf == kSaved) nf = hull_block_out(h, m, n, s.b);
+      } else if (nf == kSaved && n <= kBlockPoints) {
+        nf = hull_block_out(h, m, n, s.ph);
+        if (nf == kSaved) nf = hull_block_out(h, m, n, s.bh);
       }
-      const uint64_t bl = ballot(hz);
-      const int r = nh + rank_below(bl, lane);
-      if (hz && r < cap) {
-        hor[2 * r] = a;
-        hor[2 * r + 1] = b;
-      }
-      nh += __popcll(bl);
+      if (nf == kSaved) large |= 1ull << src;
+      else if (threadIdx.x == 0) h.nfaces[m] = nf;
     }
     __syncthreads();
-    // drop the visible faces, keeping the order of the others
-    int w = 0;
-    for (int base = 0; base < nf; base += kWave) {
-      const int f = base + lane;
-      bool alive = false;
-      int x0 = 0, x1 = 0, x2 = 0;
-      if (f < nf) {
-        x0 = F[3 * f];
-        x1 = F[3 * f + 1];
-        x2 = F[3 * f + 2];
-        alive = !(vol6(P, x0, x1, x2, qx, qy, qz) > 1e-7f);
-      }
-      const uint64_t b = ballot(alive);
-      if (alive) {
-        const int d = w + rank_below(b, lane);
-        F[3 * d] = x0;
-        F[3 * d + 1] = x1;
-        F[3 * d + 2] = x2;
-      }
-      w += __popcll(b);
-      __syncthreads();
-    }
-    if (nh > cap || w + nh > cap) {
-      return -1;
-    }
-    for (int r = lane; r < nh; r += kWave) {
-      F[3 * (w + r)] = hor[2 * r];
-      F[3 * (w + r) + 1] = hor[2 * r + 1];
-      F[3 * (w + r) + 2] = q;
-    }
-    nf = w + nh;
-    __syncthreads();
-  }
-  return nf;
-}
-
-// Clouds of more than NMAX points and those passed on as kToGeneral, one
-// wave each; the waves take the clouds in turn.
-template <int NMAX>
-__global__ __launch_bounds__(kWave) void k_hull_global(const float* __restrict__ pts,
-                                                       const int64_t* __restrict__ off,
-                                                       const int32_t* __restrict__ cnt, int nm,
-                                                       const int64_t* __restrict__ face_off,
-                                                       int64_t total_faces,
-                                                       int32_t* __restrict__ faces,
-                                                       int32_t* __restrict__ nfaces,
-                                                       int32_t* __restrict__ scratch) {
-  const int lane = threadIdx.x;
-  for (int64_t first = blockIdx.x; first < nm; first += (int64_t)gridDim.x * kWave) {
-    const int64_t mine = first + (int64_t)gridDim.x * lane;
-    bool take = false;
-    if (mine < nm) take = cnt[mine] > NMAX || nfaces[mine] == kToGeneral;
-    uint64_t todo = ballot(take);
-    while (todo != 0) {
-      const int64_t m = first + (int64_t)gridDim.x * (int)__builtin_ctzll(todo);
-      todo &= todo - 1;
-      const int64_t f0 = face_off[m], cap64 = face_off[m + 1] - f0;
-      int nf = -3;
-      if (!(f0 < 0 || cap64 < 0 || face_off[m + 1] > total_faces))
-        nf = hull_global(pts + 3 * off[m], cnt[m], cap64 < 0x7fffffff ? (int)cap64 : 0x7fffffff,
-                         faces + 3 * f0, scratch + 3 * f0, scratch + 3 * f0 + cap64, lane);
-      if (lane == 0) nfaces[m] = nf;
+    for (int k = 0; large != 0; k++) {
+      const int src = (int)__builtin_ctzll(large);
+      large &= large - 1;
+      if (wave != k % kBlockWaves) continue;
+      const int64_t m = first + (int64_t)gridDim.x * src;
+      const int n = ogjk::lane_value(n_mine, src);
+      const int nf = hull_global(h.points(m), n, h.cap(m), h.out(m), h.work(m),
+                                 h.work(m) + h.cap64(m), !ALL || n <= kWavePoints, lane);
+      if (lane == 0) h.nfaces[m] = nf;
     }
   }
 }
@@ -1173,38 +1334,27 @@ ogjk_status ogjk_build_hulls(const float* d_points, const int64_t* d_point_off,
   if (!d_workspace || workspace_bytes < need)
     return ogjk_fail(OGJK_ERR_INVALID, "workspace of %zu bytes needed", need);
   const hipStream_t st = (hipStream_t)stream;
-  // Sizes are on the device, so every class's kernel goes over the counts (an
-  // idle one takes about 4 us) and takes its own clouds; one whose working set
-  // outgrows its LDS leaves a mark in d_nfaces and a later kernel starts it
-  // again.  Classes, measured alone on equal clouds: up to 32 points 16 lanes
-  // a cloud, then a wave (1.2 us an insertion at 128 points, 1.7 as a block),
-  // then a block as large as 2 n faces fill (at 512 points 1.7 us an
-  // insertion, one wave over global memory 8), and past 1,024 points, where
-  // ids and planes no longer fit, one wave over global memory as before.
-  // Blocks are launched per cloud up to 2,048, so that the dispatcher balances
+  const HullArgs h{d_points, d_point_off, d_point_cnt, n_clouds, d_face_off, total_faces,
+                   d_faces, d_nfaces, (int32_t*)d_workspace};
+  // Sizes are on the device, so each kernel goes over the counts and takes its
+  // own clouds.  A block has room for any of them and a compute unit for one
+  // such block, so up to as many clouds are one launch; past that the launches
+  // by size, of which an idle one takes about 3 us.  Blocks are launched per
+  // cloud as far as an idle launch stays cheap, so that the dispatcher balances
   // them; larger batches take the clouds in turn.
   const auto grid = [&](int clouds_per_block, int64_t most) {
     const int64_t b = ((int64_t)n_clouds + clouds_per_block - 1) / clouds_per_block;
     return dim3((unsigned)(b < most ? b : most));
   };
-  hipLaunchKernelGGL((k_hull_group<16, 0, 32, 96>), grid(4, 1 << 20), dim3(kWave), 0, st, d_points,
-                     d_point_off, d_point_cnt, n_clouds, d_face_off, total_faces, d_faces,
-                     d_nfaces);
-  hipLaunchKernelGGL((k_hull_group<64, 33, 128, 528>), grid(1, 2560), dim3(kWave), 0, st, d_points,
-                     d_point_off, d_point_cnt, n_clouds, d_face_off, total_faces, d_faces,
-                     d_nfaces);
-  hipLaunchKernelGGL((k_hull_block<256, 1024, 129, 256, kNowhere, kToBlock>), grid(1, 2048),
-                     dim3(256), 0, st, d_points, d_point_off, d_point_cnt, n_clouds, d_face_off,
-                     total_faces, d_faces, d_nfaces);
-  hipLaunchKernelGGL((k_hull_block<512, 2048, 257, 512, kToBlock, kToBig>), grid(1, 2048),
-                     dim3(512), 0, st, d_points, d_point_off, d_point_cnt, n_clouds, d_face_off,
-                     total_faces, d_faces, d_nfaces);
-  hipLaunchKernelGGL((k_hull_block<1024, 16384, 513, 1024, kToBig, kToGeneral>), grid(1, 512),
-                     dim3(1024), 0, st, d_points, d_point_off, d_point_cnt, n_clouds, d_face_off,
-                     total_faces, d_faces, d_nfaces);
-  hipLaunchKernelGGL((k_hull_global<1024>), grid(1, 4096), dim3(kWave), 0, st, d_points,
-                     d_point_off, d_point_cnt, n_clouds, d_face_off, total_faces, d_faces,
-                     d_nfaces, (int32_t*)d_workspace);
+  if (n_clouds <= kBlocksAtOnce) {
+    hipLaunchKernelGGL((k_hull_block<true>), dim3((unsigned)n_clouds), dim3(kBlockThreads), 0, st, h);
+  } else {
+    hipLaunchKernelGGL(k_hull_few, grid(kWave / kFewLanes, 1 << 20), dim3(kWave), 0, st, h);
+    hipLaunchKernelGGL((k_hull_wave<kWaveFaces, false>), grid(1, 4096), dim3(kWave), 0, st, h);
+    hipLaunchKernelGGL((k_hull_wave<kWaveMoreFaces, true>), grid(1, 4096), dim3(kWave), 0, st, h);
+    hipLaunchKernelGGL((k_hull_block<false>), grid(1, 2 * kBlocksAtOnce), dim3(kBlockThreads), 0, st,
+                       h);
+  }
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? OGJK_OK : hip_err(e, "hull launch");
 }

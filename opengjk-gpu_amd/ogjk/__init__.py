@@ -695,7 +695,7 @@ def build_hulls(points, off, cnt, face_cap=None, stream=None):
     cap = (4 * cnt.long() + 16) if face_cap is None else face_cap.long()
     face_off = torch.zeros(n + 1, dtype=torch.int64, device=dev)
     if n:
-        face_off[1:] = torch.cumsum(cap, 0)
+        torch.cumsum(cap, 0, out=face_off[1:])
     total = int(face_off[-1].item()) if n else 0
     faces = torch.empty((max(total, 1), 3), dtype=torch.int32, device=dev)
     nfaces = torch.empty(max(n, 1), dtype=torch.int32, device=dev)
