@@ -212,24 +212,43 @@ __device__ __forceinline__ void bp_walk(const BpRec* __restrict__ rec,
     }
     int2 cur = my[0];  // never empty: the object's own row holds it
     int at = 0;
-    for (int m = 0; m < total; m += 4) {
-      // four candidates in flight; indices past the last repeat it and are
-      // skipped.  An index is loaded only for an overlapping sphere.
-      int t[4];
-      float4 q[4];
+    int m = 0;
+    while (m < total) {
+      if (__all(m + 8 <= cur.x)) {
+        // Within a row on every lane, as nearly always in crowded scenes (a
+        // wave's objects share their cells): eight candidates in flight, nothing
+        // to clamp, and most spheres overlap, so the indices come with them.
+        const BpRec* p = rec + m + cur.y;
+        float4 q[8];
+        int j[8];
 #pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const int mu = m + u < total ? m + u : total - 1;
-        if (mu >= cur.x) cur = my[++at * kBlock];
-        t[u] = mu + cur.y;
-        q[u] = rec[t[u]].s;
-      }
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        if (m + u < total && t[u] != s && overlap(me.s, q[u])) {
-          const int j = rec[t[u]].id;
-          if (j > o) f(j);
+        for (int u = 0; u < 8; u++) {
+          q[u] = p[u].s;
+          j[u] = p[u].id;
         }
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+          if (j[u] > o && overlap(me.s, q[u])) f(j[u]);
+        m += 8;
+      } else {
+        // Four in flight; indices past the last repeat it and are skipped.  An
+        // index is loaded only for an overlapping sphere.
+        float4 q[4];
+        int t[4], j[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const int mu = m + u < total ? m + u : total - 1;
+          if (mu >= cur.x) cur = my[++at * kBlock];
+          t[u] = mu + cur.y;
+          q[u] = rec[t[u]].s;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+          j[u] = m + u < total && t[u] != s && overlap(me.s, q[u]) ? rec[t[u]].id : -1;
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+          if (j[u] > o) f(j[u]);
+        m += 4;
       }
     }
     return;
