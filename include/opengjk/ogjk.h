@@ -114,8 +114,9 @@ ogjk_status ogjk_sync(void* stream);
  * a GJK kernel over every pair, then an EPA kernel over every pair, one group
  * per pair each, non-persistent (GJK/gpu/openGJK.cu:2968-3004), where GJK
  * lanes may also be 1 (one thread per pair); other calls run as fused 0.
- * A launch over few pairs (some thousands) doubles the lanes per pair until it
- * fills the chip or a pair has a whole wave (same results).
+ * A launch over few pairs doubles the lanes per pair while the wider launch has
+ * at most two waves (GJK) or four (EPA, and GJK+EPA as one kernel) for each of
+ * the chip's SIMDs; results are the same.  ogjk_set_exact_lanes refuses that.
  * Not synchronised with launches issued concurrently from other threads. */
 ogjk_status ogjk_set_config(int gjk_lanes, int epa_lanes, int fused);
 
@@ -124,6 +125,7 @@ ogjk_status ogjk_set_config(int gjk_lanes, int epa_lanes, int fused);
  * (its max_verts entry is ignored).  Each bucket runs GJK on gjk_lanes[b]
  * (8, 16, 32, 64) and EPA on epa_lanes[b] (16, 32, 64) lanes per pair, all
  * scheduled on the device (classify, scatter, persistent per-bucket kernels).
+ * A launch over few pairs widens each bucket's lanes as under ogjk_set_config.
  * Same process-wide scope as ogjk_set_config, which it replaces. */
 ogjk_status ogjk_set_buckets(int n_buckets, const int* max_verts, const int* gjk_lanes,
                              const int* epa_lanes);
@@ -133,8 +135,16 @@ ogjk_status ogjk_set_buckets(int n_buckets, const int* max_verts, const int* gjk
  * waves per block of the GJK kernel and of the persistent EPA kernel (1, 2
  * or 4) for each of the n_buckets buckets; pairs per block = 64 * waves /
  * lanes per pair.  EPA runs one launch per lane class, shaped by the first
- * bucket of the class.  Same process-wide scope as ogjk_set_config. */
+ * bucket of the class.  Launches over up to 8,192 pairs of a clustered scene
+ * give a pair on 64 lanes a block of two waves, one per body, whatever is set
+ * here (see ogjk_set_exact_lanes).  Same process-wide scope as ogjk_set_config. */
 ogjk_status ogjk_set_block_waves(int n_buckets, const int* gjk_waves, const int* epa_waves);
+
+/* exact != 0: launches over few pairs keep the lanes per pair and the waves per
+ * block set by the calls above, as launches over many do (to time a shape, or
+ * where a caller knows better).  ogjk_set_config and ogjk_set_buckets reset it
+ * to 0.  Same process-wide scope as ogjk_set_config. */
+ogjk_status ogjk_set_exact_lanes(int exact);
 
 /* Device workspace bytes a GJK or GJK+EPA call over n_pairs needs. */
 size_t ogjk_workspace_bytes(int32_t n_pairs);

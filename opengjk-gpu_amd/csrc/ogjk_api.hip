@@ -338,6 +338,13 @@ ogjk_status ogjk_set_block_waves(int n_buckets, const int* gjk_waves, const int*
   return OGJK_OK;
 }
 
+ogjk_status ogjk_set_exact_lanes(int exact) {
+  ogjk::LaunchConfig c = ogjk::get_config();
+  c.exact = exact != 0;
+  ogjk::set_config(c);  // the configuration was valid
+  return OGJK_OK;
+}
+
 size_t ogjk_workspace_bytes(int32_t n_pairs) { return ogjk::workspace_bytes(n_pairs); }
 
 ogjk_status ogjk_sync(void* stream) {

@@ -71,6 +71,7 @@ struct LaunchConfig {
   int gjk_waves[kMaxBuckets] = {1, 1, 1, 1};
   int epa_waves[kMaxBuckets] = {4, 4, 4, 4};
   int fused = 0;
+  bool exact = false;  // these lanes also for few pairs (see fill_lanes, use_duo)
 };
 
 // Per-launch copy of the bucket table passed to the kernels.

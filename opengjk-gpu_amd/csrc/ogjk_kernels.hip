@@ -977,18 +977,24 @@ static hipError_t launch_pairs(const Src& src, const OutArgs& o, int n, hipStrea
 // the wider launch would have at most `waves` waves for each of the chip's 1,024
 // SIMDs.  A wider group shortens its pair's chain: no waiting for the other pairs
 // of its wave, fewer sweep steps.  It pays as long as the waves run side by side,
-// for EPA longer than for GJK, as only the penetrating pairs reach it.  Measured
-// on pairs of 64 vertices configured as 8 and 32 lanes, narrow -> wide:
-//   GJK 8, EPA 32:      64 pairs 110 ->  67 us with 64 and 64
-//   GJK 32, EPA 32:  1,500 pairs 181 -> 127 us with 64 and 64
-//   GJK 16, EPA 32:  3,000 pairs 188 -> 184 us with 32, 142 with 64 and 64
-//   GJK 8, EPA 32:   4,096 pairs 223 -> 182 us with 32 and 64
-//   GJK 8, EPA 32:   6,000 pairs 238 -> 227 us with 16 and 32
-//   GJK 8, EPA 32:   8,000 pairs 254 -> 263 us with 32 and 32
+// for EPA longer than for GJK, as only the penetrating pairs reach it.  Not done
+// where the caller asked for exact lanes.  Pairs of spheres of 64 vertices
+// configured as 8 and 32 lanes, us, * what the rule picks (GJK, EPA lanes):
+//             8,32  16,32  32,32  16,64  32,64  64,64
+//     64       107     98     94     87     84    80*
+//  1,000       166    157    154    124    119   116*
+//  2,000       197    187    183    149    143   142*
+//  3,000       186    177    175    142   141*    144
+//  4,096       206    193    189    159   155*    172
+//  6,000       197   190*    193    165    168    183
+//  8,000       251   245*    269    198    228    246
+// 12,000      268*    265    287    244    262    291
+// EPA's line could lie higher for these, but for spheres of 8 vertices 8,000 pairs
+// take 70 us at 16,32, 77 at 16,64 and 92 at 32,64; of 256 vertices 430, 356, 342.
 constexpr int64_t kChipLanes = 1024 * 64;
 constexpr int kFillGjk = 2, kFillEpa = 4;
 static int fill_lanes(int lanes, int n, int waves) {
-  while (lanes < 64 && 2 * (int64_t)lanes * n <= waves * kChipLanes) lanes *= 2;
+  while (!g_cfg.exact && lanes < 64 && 2 * (int64_t)lanes * n <= waves * kChipLanes) lanes *= 2;
   return lanes;
 }
 
@@ -998,7 +1004,7 @@ static int fill_lanes(int lanes, int n, int waves) {
 // for 8,000, 851 and 873 for 16,000, where what both waves do alike costs more than
 // the shorter chain gains.
 constexpr int kDuoPairs = 8192;
-static bool use_duo(int lanes, int n) { return lanes == 64 && n <= kDuoPairs; }
+static bool use_duo(int lanes, int n) { return !g_cfg.exact && lanes == 64 && n <= kDuoPairs; }
 
 // Resident grid for a persistent launch over at most n items.
 static unsigned persistent_blocks(int n, int gpb, unsigned cap = 4096u) {

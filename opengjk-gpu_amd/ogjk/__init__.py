@@ -47,7 +47,7 @@ C_ABI_SYMBOLS = [
     "ogjk_expand_pairs_workspace", "ogjk_expand_pairs", "ogjk_collide_scene_contacts",
     "ogjk_collide_posed_bodies_contacts", "ogjk_build_hulls", "ogjk_hull_moments",
     "ogjk_center_points", "ogjk_collide_scene_noalloc", "ogjk_pack_scene_f64_aos",
-    "ogjk_set_block_waves",
+    "ogjk_set_block_waves", "ogjk_set_exact_lanes",
 ]
 
 
@@ -102,6 +102,7 @@ def lib():
             "ogjk_set_config": (C.c_int, [C.c_int, C.c_int, C.c_int]),
             "ogjk_set_buckets": (C.c_int, [C.c_int, vp, vp, vp]),
             "ogjk_set_block_waves": (C.c_int, [C.c_int, vp, vp]),
+            "ogjk_set_exact_lanes": (C.c_int, [C.c_int]),
             "ogjk_workspace_bytes": (C.c_size_t, [i32]),
             "ogjk_collide_scene_ws": (C.c_int, [C.c_int, C.POINTER(_Scene), vp, i32, vp, vp, vp, vp,
                                                 vp, C.c_size_t, vp]),
@@ -194,6 +195,12 @@ def set_block_waves(gjk_waves, epa_waves) -> None:
     gw = np.array(gjk_waves, dtype=np.int32)
     ew = np.array(epa_waves, dtype=np.int32)
     _check(lib().ogjk_set_block_waves(len(gw), _ptr(gw), _ptr(ew)))
+
+
+def set_exact_lanes(exact: bool = True) -> None:
+    """Launches over few pairs keep the configured shape too (see
+    ogjk_set_exact_lanes in include/opengjk/ogjk.h)."""
+    _check(lib().ogjk_set_exact_lanes(int(exact)))
 
 
 def device_count() -> int:

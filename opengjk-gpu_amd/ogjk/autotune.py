@@ -14,6 +14,8 @@ Search (coordinate descent, about seventy launches):
   4. the cluster threshold again, on the best table;
   5. pairs per workgroup: for each bucket, the GJK kernel's and then the EPA
      kernel's waves per block in WAVES (pairs per block = 64 * waves / lanes).
+Candidates run exactly as named; `apply()` leaves launches over few pairs to
+widen (ogjk_set_config in include/opengjk/ogjk.h).
 """
 from __future__ import annotations
 
@@ -84,6 +86,7 @@ def tune(scene, n_pairs: int, log=print) -> dict:
 
     def run(table, cmin):
         _apply_table(table)
+        ogjk.set_exact_lanes()  # each candidate as it is named, also over few pairs
         _set_clusters(scene, cmin)
         ms = _time(scene, n_pairs)
         tried.append(dict(table, cluster_min=cmin, ms=ms))
