@@ -789,9 +789,12 @@ __global__ __launch_bounds__(kWave) void k_hull_wave(HullArgs h) {
 // vertex ids alone (4 bytes a face, the normal formed anew from the corners).
 // A call over few clouds is one launch of this kernel: each block's first wave
 // starts its cloud, and the block goes on from kAloneFaces faces, where a wave's
-// insertion takes as long (512 points: 0.82 ms, 1.16 with the wave to the end,
-// 1.0 with the block from 64 faces).
-constexpr int kBlockThreads = 512, kBlockWaves = kBlockThreads / kWave, kBlockPoints = 1024;
+// insertion takes as long (512 points: 0.83 ms, 1.16 with the wave to the end,
+// 1.2 with the block from 64 faces).  16 waves a block, one block to a compute
+// unit: 8 are 2% faster there, but clouds that end over global memory want all
+// the waves (300 clouds of 1,500 points on a sphere 58 ms with 512 blocks of 8
+// waves, 37 with 256 of 16).
+constexpr int kBlockThreads = 1024, kBlockWaves = kBlockThreads / kWave, kBlockPoints = 1024;
 constexpr int kAloneFaces = 512;
 constexpr int kBlocksAtOnce = 256;  // compute units, one block each
 
@@ -1338,10 +1341,11 @@ ogjk_status ogjk_build_hulls(const float* d_points, const int64_t* d_point_off,
                    d_faces, d_nfaces, (int32_t*)d_workspace};
   // Sizes are on the device, so each kernel goes over the counts and takes its
   // own clouds.  A block has room for any of them and a compute unit for one
-  // such block, so up to as many clouds are one launch; past that the launches
-  // by size, of which an idle one takes about 3 us.  Blocks are launched per
-  // cloud as far as an idle launch stays cheap, so that the dispatcher balances
-  // them; larger batches take the clouds in turn.
+  // such block, so up to as many clouds are one launch (10 clouds of 8 points 41
+  // us, 53 as four launches); past that the launches by size, of which an idle
+  // one takes about 3 us.  Waves are launched per cloud as far as an idle launch
+  // stays cheap, so that the dispatcher balances them; larger batches take the
+  // clouds in turn.
   const auto grid = [&](int clouds_per_block, int64_t most) {
     const int64_t b = ((int64_t)n_clouds + clouds_per_block - 1) / clouds_per_block;
     return dim3((unsigned)(b < most ? b : most));
@@ -1352,7 +1356,7 @@ ogjk_status ogjk_build_hulls(const float* d_points, const int64_t* d_point_off,
     hipLaunchKernelGGL(k_hull_few, grid(kWave / kFewLanes, 1 << 20), dim3(kWave), 0, st, h);
     hipLaunchKernelGGL((k_hull_wave<kWaveFaces, false>), grid(1, 4096), dim3(kWave), 0, st, h);
     hipLaunchKernelGGL((k_hull_wave<kWaveMoreFaces, true>), grid(1, 4096), dim3(kWave), 0, st, h);
-    hipLaunchKernelGGL((k_hull_block<false>), grid(1, 2 * kBlocksAtOnce), dim3(kBlockThreads), 0, st,
+    hipLaunchKernelGGL((k_hull_block<false>), grid(1, kBlocksAtOnce), dim3(kBlockThreads), 0, st,
                        h);
   }
   const hipError_t e = hipGetLastError();

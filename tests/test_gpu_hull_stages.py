@@ -145,27 +145,39 @@ def test_few_clouds_are_one_launch(torch_cuda, n):  # noqa: F811
     assert nodes.value == 1
 
 
+def _seconds(torch, clouds, cap):
+    args, nf, keep = _device_args(torch, clouds, [cap] * len(clouds))
+    best = 1e9
+    for _ in range(6):
+        torch.cuda.synchronize()
+        t = time.perf_counter()
+        for _ in range(5):
+            assert ogjk.lib().ogjk_build_hulls(*args, None) == 0
+        torch.cuda.synchronize()
+        best = min(best, time.perf_counter() - t)
+    return best, nf
+
+
 @pytest.mark.parametrize("points", [400, 1024])
 def test_many_inner_point_clouds_run_side_by_side(torch_cuda, points):  # noqa: F811
     """3,000 clouds with most points inside take little longer than one: a
     wave each (1.3 times here; 12 times with a block of 16 waves per cloud)."""
     torch = torch_cuda
     shapes = [inside(points, k) for k in range(100)]
-
-    def seconds(clouds):
-        args, nf, keep = _device_args(torch, clouds, [4 * points + 16] * len(clouds))
-        best = 1e9
-        for _ in range(6):
-            torch.cuda.synchronize()
-            t = time.perf_counter()
-            for _ in range(5):
-                assert ogjk.lib().ogjk_build_hulls(*args, None) == 0
-            torch.cuda.synchronize()
-            best = min(best, time.perf_counter() - t)
-        assert (nf > 0).all()
-        return best
-
-    one, many = seconds(shapes[:1]), seconds(shapes * 30)
+    one, nf1 = _seconds(torch, shapes[:1], 4 * points + 16)
+    many, nf = _seconds(torch, shapes * 30, 4 * points + 16)
     print(f"\n[{points} points] one cloud {one / 5 * 1e6:.0f} us, 3,000 {many / 5 * 1e6:.0f} us",
           flush=True)
+    assert (nf1 > 0).all() and (nf > 0).all()
     assert many < 4 * one
+
+
+def test_large_clouds_run_side_by_side(torch_cuda):  # noqa: F811
+    """300 clouds past the LDS working sets take no longer than 100: a wave
+    each, all in flight (1.4 times with the waves of one block to a cloud)."""
+    torch = torch_cuda
+    shapes = [sphere(1100, k) for k in range(100)]
+    few, _ = _seconds(torch, shapes, 4 * 1100 + 16)
+    more, _ = _seconds(torch, shapes * 3, 4 * 1100 + 16)
+    print(f"\n100 clouds {few / 5 * 1e3:.1f} ms, 300 {more / 5 * 1e3:.1f} ms", flush=True)
+    assert more < 1.2 * few
