@@ -95,20 +95,8 @@ OGJK_DEV int lanes_below(lane_mask<LPP> m, int l) {
 }
 
 template <int LPP>
-OGJK_DEV int lane_in() {
-  return lane_id() & (LPP - 1);
-}
-
-template <int LPP>
 OGJK_DEV bool group_any(bool p) {
   return group_ballot<LPP>(p) != 0;
-}
-
-// Number of set predicates in lower lanes of the group.
-template <int LPP>
-OGJK_DEV int group_prefix(uint64_t gb) {
-  const int l = lane_id() & (LPP - 1);
-  return __popcll(gb & ((1ull << l) - 1ull));
 }
 
 // Exchange step m (1, 2, 4, ...) of an all-reduce over LPP lanes.  Steps
