@@ -737,9 +737,11 @@ __device__ __forceinline__ int hull_global(const float* __restrict__ P, int n, i
 
 // RESUME: the clouds whose state was saved, else those of more than kFewPoints
 // points and those of fewer that outgrew their lanes, from the start.  The waves
-// of the grid take the clouds in turn.  Two steps, for the room: with the larger
-// one at once a compute unit has 3 waves, with the smaller one 22.
-constexpr int kWaveFaces = 160, kWaveMoreFaces = 1200;
+// of the grid take the clouds in turn.  Two steps, for the room: a compute unit
+// has 22 waves of the first and 4, one to a SIMD, of the second (3 with 1,200 faces:
+// 1,000 clouds of 256 points on a sphere 750 us, 460 with 880; 5 and 6 with 700 and
+// 560: 2,000 clouds of 8-512 points 1.22 ms with 880, 1.38 with 1,200, 1.41, 1.64).
+constexpr int kWaveFaces = 160, kWaveMoreFaces = 880;
 
 template <int FB, bool RESUME>
 __global__ __launch_bounds__(kWave) void k_hull_wave(HullArgs h) {

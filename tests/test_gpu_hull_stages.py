@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
 
 # Faces that the working sets hold: 16 lanes, a wave, the wave of a call over few
 # clouds, a wave with more room, a block with planes, a block with vertex ids.
-ROOM = [96, 160, 512, 1200, 3584, 14336]
+ROOM = [96, 160, 512, 880, 3584, 14336]
 FEW_CLOUDS, FEW_POINTS, BLOCK_POINTS = 256, 32, 1024
 
 
@@ -38,7 +38,7 @@ GROUPS = {
     # small clouds past their 16 lanes' faces, and within
     "few points": [ellipsoid(32, 46, 0.03), ellipsoid(32, 0, 1.0), sphere(32, 1), sphere(33, 2)],
     # 2 n - 4 faces around a wave's, an alone wave's and the larger wave's room
-    "edges": [sphere(n, 3) for n in (80, 81, 82, 83, 255, 256, 257, 258, 259, 601, 602, 603, 604)],
+    "edges": [sphere(n, 3) for n in (80, 81, 82, 83, 255, 256, 257, 258, 259, 441, 442, 443, 444)],
     "sizes": [sphere(n, 4) for n in (511, 512, 513, 1023, 1024, 1025, 1200)],
     # face lists that blow up: bits and hash set, planes and ids, past both
     "dense": [ellipsoid(*c) for c in ((256, 0, 0.12), (512, 39, 0.2), (436, 6, 0.2), (800, 1, 0.35),
