@@ -805,7 +805,7 @@ def hulls(args) -> dict:
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS,
                      "traffic": profile_value("hulls", "traffic_bytes_per_step"),
-                     "kernel": "k_hull (one hull build of every cloud)",
+                     "kernel": "k_hull_few (one hull build of every cloud)",
                      "kernel_ms_mean": float(np.mean(hms)), "algorithmic_bytes_per_launch": alg,
                      "algorithmic_bytes": "12 B per point read, 12 B per face written, 16 B "
                                           "per cloud of offsets and counts"},

@@ -11,7 +11,7 @@
 #ifndef OGJK_GJK_WAVES
 #define OGJK_GJK_WAVES 3
 #endif
-// With the simplex in LDS the clustered 64-lane kernel needs 121 registers and
+// With the simplex in LDS the clustered 64-lane kernel needs 123 registers and
 // runs 4 waves/SIMD by itself; the posed one needs 133 and is held to 128 (12
 // B/lane of scratch; 50K posed pairs 432 us).
 #ifndef OGJK_GJK_WAVES_WIDE
@@ -22,7 +22,7 @@
 #endif
 // EPA: float scenes swept whole run at 3 waves/SIMD with 44 B/lane of scratch at
 // 32 lanes (179 registers wanted); the 64-lane kernels of clustered scenes fit 3
-// waves with 161 registers (at 4: 96 B/lane, 100K uneven pairs 1,550 -> 1,625 us);
+// waves with 167 registers (at 4: 96 B/lane, 100K uneven pairs 1,550 -> 1,625 us);
 // posed ones stay at 2 (at 3: 112 B/lane, 375-390 -> 397 us over 50K pairs), and
 // so do narrower clustered ones and the other sources.
 #ifndef OGJK_EPA_WAVES
